@@ -865,6 +865,11 @@ long cert_slots(const CertShape& c) {
 
 }  // namespace
 
+// row steps a block's time holds beyond its rows' (launch, tables, first row:
+// a two-row part of one 32x32 patch, three row steps, measured 5.7 us above an
+// empty launch, a row step 2.1)
+constexpr double kCertStart = 2.0;
+
 long real_cert_round(int cin, int cout, int W) {
   const CertShape c = cert_shape(cin, cout, W);
   const long slots = cert_slots(c);
@@ -882,14 +887,29 @@ hipError_t launch_real_cert(const RealArgs& a, hipStream_t s) {
   if (hipError_t e = cert_attr(c.var); e != hipSuccess) return e;
   const long npatch_items = (long)a.N * c.per_patch;
   // Row parts: a block's time is its row steps (the kernel is latency-bound,
-  // a block alone on its CU takes about as long as two), so a launch that
-  // leaves slots of the round empty splits each patch's rows over S = 2 or 4
-  // blocks while S times the blocks still fit in one round, each part at
-  // least 8 rows (a part re-reads the input row above it: 17 row steps
-  // for half of 32 rows against 33 for all of them)
+  // a block alone on its CU takes about as long as two), so each patch's rows
+  // are split over S blocks where that fills the device better.  A part of
+  // rh rows takes rh + 1 row steps (it re-reads the input row above it) and
+  // about kCertStart of them before its first row; the S taken has the least
+  // rounds x steps, the fewest blocks among equals.  Against halves and
+  // quarters within one round only, conv time by events: one 32x32 patch
+  // 19.0 -> 10.3 us (16 parts for 4), 64 patches 29.4 -> 21.4 (8 for 4), one
+  // 512x512 image 285 -> 68 us (32 parts for 4, 64 blocks of 512 possible).
   const long slots = cert_slots(c);
   int S = 1;
-  while (S < 4 && slots > 0 && npatch_items * S * 2 <= slots && a.H / (S * 2) >= 8) S *= 2;
+  if (slots > 0) {
+    double best = 0.0;
+    for (int rh = a.H; rh >= 2; --rh) {
+      const int parts = (a.H + rh - 1) / rh;
+      if ((a.H + parts - 1) / parts != rh) continue;  // a smaller rh has as many parts
+      const long items = npatch_items * parts;
+      const double t = (double)((items + slots - 1) / slots) * (rh + 1 + kCertStart);
+      if (rh == a.H || t < 0.98 * best) {
+        best = t;
+        S = parts;
+      }
+    }
+  }
   const long nitems = npatch_items * S;
   if (nitems >= 0x7FFFFFF0) return hipErrorInvalidValue;
   RealArgs b = a;

@@ -172,6 +172,23 @@ def test_cert_row_parts(tmp_path, orc, N, H, W, base):
     exact.close()
 
 
+@pytest.mark.parametrize("N,H,W,base", [(1, 32, 32, 16), (1, 16, 16, 8), (1, 129, 256, 16), (2, 65, 160, 32),
+                                         (170, 33, 32, 16)])
+def test_cert_many_row_parts(tmp_path, orc, N, H, W, base):
+    """Few blocks to a launch: parts of two rows (one patch of 32 or 16 rows),
+    a last part of one row (129 and 65 rows), and 170 patches, whose rows
+    split in three or more parts over one round of blocks or several."""
+    b = synth.make_blob(seed=80 + H, base=base)
+    x = synth.make_input(81 + W, N, 120, H, W)
+    x[0, 40, H // 2, :] = np.inf  # an undecided row in a middle part
+    fast = _engine(tmp_path, b, "a.blob", cert=True)
+    exact = _engine(tmp_path, b, "b.blob", cert=False)
+    assert _bits_equal(fast.forward_batch(x), exact.forward_batch(x))
+    _check(fast, orc.parse(B.to_bytes(b)), x[[0]])
+    fast.close()
+    exact.close()
+
+
 @pytest.mark.parametrize("base,H,W", [(16, 32, 32), (32, 32, 32), (8, 16, 16), (16, 20, 28), (24, 32, 16),
                                        (16, 16, 72), (8, 20, 100), (32, 16, 256), (16, 36, 36)])
 def test_cert_shapes(tmp_path, orc, base, H, W):
