@@ -45,12 +45,12 @@ before each other configuration.  Prints ONE JSON line on stdout:
                 VALU-popcount roofline and the HBM rate of its bytes
   fused_pool    the isolated fused bconv+fold+maxpool kernel at 128->128,
                 32x32, batch 1024 (the benchmark's fused-kernel config):
-                the kernel the default rule takes (the int8 matrix cores)
-                against the int8 peak, and the bit-packed popcount kernel
+                the kernel the default rule takes (the matrix cores, FP4)
+                against the FP4 peak, and the bit-packed popcount kernel
                 (BNN_BCONV_MFMA=0) against the VALU-popcount peak
   cfg4          benchmark config 4: 256x256x120 patches, batch 64, base 32;
-                per-kernel times, the int8 matrix-core convs against the
-                dense int8 peak
+                per-kernel times, the wide matrix-core convs against the
+                dense FP4 peak
   scene         benchmark config 3: a 956x684x120 scene by 32x32 patches,
                 device-resident and from host memory (PCIe included)
   v2_stem       the v2 spectral-stem model (16-channel 1x1 stem, then the
@@ -81,7 +81,7 @@ sys.path.insert(0, ROOT)
 # MI355X published peaks
 PEAK_FP32_FLOPS = 157.3e12          # dense FP32 matrix (MFMA); also the packed-vector figure
 PEAK_HBM = 8.0e12
-PEAK_INT8_MACS = 2.5e15             # dense int8 matrix: 5.0 POP/s = 2.5e15 MAC/s
+PEAK_FP4_MACS = 5.03e15             # dense FP4 matrix: 10.07 PFLOP/s = 5.03e15 MAC/s
 
 
 def valu_binop_peak() -> float:
@@ -389,8 +389,7 @@ def bench_cfg4(sp, stream, td, reps4=5):
     from bnns_to_c_amd import blob, engine, synth
 
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-    # the int8 matrix-core conv takes the fold convs of 32-wide rows with at
-    # least 4 chunks of 64 input channels, the popcount kernel the rest
+    # every binary layer of this shape runs on the matrix cores
     b4 = synth.make_blob(seed=0, base=32)
     p4 = os.path.join(td, "bench_cfg4.blob")
     blob.write(b4, p4)
@@ -426,12 +425,12 @@ def bench_cfg4(sp, stream, td, reps4=5):
         us = tot / cnt * 1e3
         k4 = {"label": lab, "op": op, "us": round(us, 2)}
         if op.endswith("_mfma"):
-            k4["mac_s"] = round(work / (us / 1e6), 1)  # bit-MACs = int8 MACs
-            k4["frac_int8_peak"] = round(work / (us / 1e6) / PEAK_INT8_MACS, 4)
+            k4["mac_s"] = round(work / (us / 1e6), 1)  # bit-MACs = FP4 MACs
+            k4["frac_fp4_peak"] = round(work / (us / 1e6) / PEAK_FP4_MACS, 4)
         cfg4_kern.append(k4)
     log(f"cfg4 256x256x120 b{N4} base 32: {cfg4_ms:.3f} ms/step, {N4 / cfg4_ms * 1e3:,.0f} patches/s")
     for k4 in cfg4_kern:
-        extra = f"  {k4['frac_int8_peak']:.3f} of int8 peak" if "mac_s" in k4 else ""
+        extra = f"  {k4['frac_fp4_peak']:.3f} of FP4 peak" if "mac_s" in k4 else ""
         log(f"  {k4['label']:10s} {k4['op']:16s} {k4['us']:9.1f} us{extra}")
     eng4.close()
     del x4, y4
@@ -549,12 +548,12 @@ def main() -> int:
         pool_ms = e0.elapsed_time(e1) / reps
         pool_bitmacs = N * C * H * W * C * 9
         pool_rate = 2 * pool_bitmacs / (pool_ms / 1e3)
-        # this shape (cout 128, 32-wide rows) is inside the int8 matrix-core
+        # this shape (cout 128, 32-wide rows) is inside the matrix-core
         # rule unless BNN_BCONV_MFMA=0 keeps the popcount kernel; the
         # fraction is of the path's own peak
         pool_mfma = os.environ.get("BNN_BCONV_MFMA") != "0"
-        pool_frac = pool_bitmacs / (pool_ms / 1e3) / PEAK_INT8_MACS if pool_mfma else pool_rate / valu_binop_peak()
-        pool_peak = "int8 matrix peak" if pool_mfma else "VALU popcount peak"
+        pool_frac = pool_bitmacs / (pool_ms / 1e3) / PEAK_FP4_MACS if pool_mfma else pool_rate / valu_binop_peak()
+        pool_peak = "FP4 matrix peak" if pool_mfma else "VALU popcount peak"
         log(f"fused bconv+fold+pool 128->128 32x32 b{N}: {pool_ms * 1e3:.1f} us, frac {pool_frac:.3f} of {pool_peak}")
         L.close()
         pool_pc = None
@@ -960,14 +959,14 @@ def main() -> int:
                      "hbm_frac": round(c1_bytes / (c1_ms / 1e3) / PEAK_HBM, 4)},
             "fused_pool": {"config": "bconv 128->128 + fold + 2x2 maxpool + fold, 32x32, batch 1024",
                            "us": round(pool_ms * 1e3, 2), "binary_op_s": round(pool_rate, 1),
-                           "kernel": "k_bconv_mfma (int8 matrix cores)" if pool_mfma else "k_bconv (VALU popcount)",
+                           "kernel": "k_bconv_mfma (FP4 matrix cores)" if pool_mfma else "k_bconv (VALU popcount)",
                            "frac": round(pool_frac, 4), "frac_of": pool_peak,
                            **({"popcount": pool_pc} if pool_pc else {})},
             "cfg4": {"config": "large tiles: 256x256x120, batch 64, base 32 (512 channels at the bottleneck)",
                      "ms_per_step": round(cfg4_ms, 4), "patches_s": round(N4 / cfg4_ms * 1e3, 1),
                      "kernels": cfg4_kern,
-                     "int8_mfma_rule": "fold and pool convs with cout % 64 == 0, rows at least 16 wide and "
-                                       "64+ input channels (enc2.c2 .. dec2.c2 here)"},
+                     "mfma_rule": "every binary layer; \"_mfma\" marks fold and pool convs with cout % 64 == 0, "
+                                  "rows at least 16 wide and 64+ input channels (enc2.c2 .. dec2.c2 here)"},
             "scene": {"config": f"{SH}x{SW}x{b.n_bands} cube, {PS}x{PS} patches ({npatch}, edge patches zero "
                                 "past the scene), benchmark config 3",
                       "device_ms": round(scene_dev_ms, 4), "device_patches_s": round(npatch / scene_dev_ms * 1e3, 1),

@@ -1,11 +1,11 @@
-// bnn_bconv_mfma.hip - the v1 binary 3x3 conv on the int8 matrix cores of
-// gfx950, with the rule (fold) and the fused 2x2 max-pool epilogues; layers
-// with cout % 64 == 0.  Same P, bits and dumps as the popcount kernel
-// (csrc/bnn_conv.c:23-36, csrc/bnn_maxpool.c:28-48).
+// bnn_bconv_mfma.hip - the binary 3x3 conv on the matrix cores of gfx950, as
+// an FP4 product with FP32 sums, with the rule (fold), the fused 2x2
+// max-pool, the 1x1 head or the integer P as its epilogue.  Same P, bits,
+// logits and dumps as the popcount kernel (csrc/bnn_conv.c:23-36,
+// csrc/bnn_maxpool.c:28-48, csrc/bnn_head.c:21-34).
 //
 // Built with the matrix instructions' accumulators in ordinary VGPRs
-// (-mllvm -amdgpu-mfma-vgpr-form): with AGPR accumulators the compiler
-// copies the 64 accumulator registers through VGPRs on every K step.
+// (-mllvm -amdgpu-mfma-vgpr-form): the epilogue reads all of them.
 #include <algorithm>
 #include <atomic>
 
@@ -15,476 +15,816 @@
 namespace bnn {
 namespace {
 
-// ------------------------------------------------------------------------
-// binary conv on the int8 matrix cores (cout % 64 == 0, fold / pool epilogues)
-// ------------------------------------------------------------------------
-// A block of four waves computes D for 64 output channels (4 groups of 16,
-// the A operand: int8 +-1 weights) x one tile of 256 output pixels (each
-// wave 4 groups of 16, the B operand: activation bits as 0/1 bytes) with
-// v_mfma_i32_16x16x64_i8; P = 2*D - S[border class][co] (bnn_kernels.h).
-// A tile is TR rows of TW columns of one patch (a patch of TR rows or more)
-// or TI whole patches (smaller patches), TR * TW = 256: TW = W for rows up
-// to 64 wide (whole rows), 32 for wider ones (W a power of two).
+// The product.  v_mfma_f32_16x16x128_f8f6f4 with both operands in FP4 (E2M1:
+// 0, 0.5, 1, 2, 4 and their negatives are exact) runs 128 terms at twice the
+// rate of the int8 instruction's 64, and an operand element takes half a
+// byte.  An activation bit needs no conversion beyond a mask: bit 4k + j of
+// a packed word is nibble k of `word & (0x11111111 << j)`, which FP4 reads as
+// 0 or 0.5, 1, 2 for j = 0, 1, 2 (j = 3 is shifted down to 0.5: bit 3 is the
+// sign).  The weights' magnitudes make up for it (4, 2, 1, 4), so every
+// product is 2*w*alpha, alpha in {0, 1}.  The accumulator starts at
+// -S - c (S: the weight sum over the taps inside the image, one of 16 border
+// classes, c: the centre of the channel's rule) and ends at P - c, since
+// P = 2*sum(w*alpha) - S.  Every term and sum is an integer or a half below
+// 2^24, so the FP32 sums are exact in any order.
 //
-// B comes from LDS: for each chunk of two activation words the block stages
-// the tile's rows with a one-pixel halo, (TR + 2) x (W + 2) pixels per patch,
-// zeros outside the patch (and where a concat's upsample does not reach), so
-// every tap of every pixel is a fixed offset from the pixel and no tap needs
-// a mask.  A pixel's 64 bytes sit in an 80-byte slot and a row's slots are
-// padded to 128 bytes mod 256, so the 16 lanes of a group (16 pixels of one
-// row) read distinct banks.  Two buffers: chunk c + 1 is expanded and stored
-// while chunk c is consumed, and its words are loaded from HBM one chunk
-// earlier.  A (the same for the block's four waves) goes through LDS too:
-// each K step's 64 channels x 64 bytes are loaded once per block (16 bytes
-// a thread, four steps ahead of their use and two ahead of their store;
-// one step ahead of the store measured 1-3% slower) into a ring of three slots, one
-// barrier per K step, and each wave reads the next step's A from its slot
-// while the current step's matrix ops run.  (Read straight from the weight
-// table by every wave, A was the layer's bottleneck: the four waves'
-// identical 4 KB per K step through the vector L1 held the matrix cores
-// near a fifth of their rate.)
+// Work split.  A wave makes MT*16 channels x G*16 pixels, a block of four
+// waves the same channels of 64*G pixels: a tile of TR rows x TW columns of a
+// patch, or of TI whole patches.  The tile's words with a one-pixel zero halo
+// sit in LDS, staged once for all its channels' taps, [plane of 4 words]
+// [pixel][word], so one 4-byte read per lane is a whole B operand: lane
+// 16q + j takes pixel j of the group and K slot 4*step + q.  A K slot is one
+// (word, tap), or, for a first segment of at most 16 channels, one (row, pair
+// of taps): that word holds the pixel's 16 bits and its right neighbour's.
+// The weights come as ready FP4 operands ([channel group][step][m][lane][16
+// bytes]); they stay in LDS for the block's life when they fit (kResident),
+// else they pass through it in phases of kPhase steps, two buffers, the next
+// phase's loads in flight while this one is used.
 //
-// One K step (64) is one tap of one chunk: lane group q = lane / 16 takes
-// word q / 2 of the chunk, channels 16 * (q % 2) .. +15 of it, in A and B
-// alike.  D register r of lane l holds channel 4 * (l / 16) + r, pixel l % 16
-// of its group.  Fold tiles number pixels row by row.  Pool tiles give a
-// group pair (0, 1 or 2, 3) the two rows of 8 consecutive 2x2 blocks, group
-// 2p the top row, so a block's four pixels are lanes j, j ^ 1 of both groups.
-// The epilogues rebuild each pixel's words: every lane folds its four
-// channels and two lane swaps (v_permlane16_swap, v_permlane32_swap) gather
-// the 16-bit group; the block max is a max across the pair and one DPP step.
+// Blocks are persistent and XCD-aware: block b runs on XCD b % 8, whose
+// blocks walk the tiles x, x + 8, ... with a tile's channel groups side by
+// side, so the words of a pixel merge in one L2.
 typedef int i32x4v __attribute__((ext_vector_type(4)));
+typedef int i32x8v __attribute__((ext_vector_type(8)));
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+typedef int i32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// 16 activation bits -> 16 bytes of 0/1, bit k to byte k: n * 0x00204081 is
-// the OR of four shifted copies of the nibble n (they do not overlap), and
-// bits 0, 8, 16, 24 of it are n's bits 0..3
-__device__ __forceinline__ i32x4v bits_to_bytes(uint32_t b16) {
-  i32x4v r;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) r[k] = (int)((((b16 >> (4 * k)) & 0xFu) * 0x00204081u) & 0x01010101u);
-  return r;
+constexpr int kPhase = 4;                   // K steps a streamed phase
+constexpr size_t kResident = 40u * 1024;    // weight bytes of a channel group kept in LDS
+constexpr uint32_t kFar = 0x80000000u;
+
+__device__ __forceinline__ f32x4v mfma_f4(const i32x4v& a, const i32x4v& b, const f32x4v& c) {
+  const i32x8v A = {a[0], a[1], a[2], a[3], 0, 0, 0, 0}, B = {b[0], b[1], b[2], b[3], 0, 0, 0, 0};
+  // cbsz = blgp = 4: FP4 operands (four registers each); both scales 1
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B, c, 4, 4, 0, 0, 0, 0);
 }
-// OR of v over the four lane groups of 16 (lanes l, l ^ 16, l ^ 32, l ^ 48)
-__device__ __forceinline__ uint32_t or_groups(uint32_t v) {
-  const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  v = a[0] | a[1];
-  const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  return b[0] | b[1];
+__device__ __forceinline__ i32x4v bits_f4(uint32_t w) {
+  return i32x4v{(int)(w & 0x11111111u), (int)(w & 0x22222222u), (int)(w & 0x44444444u), (int)((w >> 3) & 0x11111111u)};
 }
-// max of x over lanes l, l ^ 1
-__device__ __forceinline__ int32_t max_pair(int32_t x) {
-  return max(x, __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xF, 0xF, false));  // quad_perm [1, 0, 3, 2]
+// rows of 16 lanes: from a and b, rows 0, 1 hold a's row pairs (0 | 2, 1 | 3)
+// and rows 2, 3 b's
+__device__ __forceinline__ uint32_t or_halves(uint32_t a, uint32_t b) {
+  const auto s = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  return s[0] | s[1];
+}
+// rows {a0 | a1, b0 | b1, a2 | a3, b2 | b3}
+__device__ __forceinline__ uint32_t or_rows(uint32_t a, uint32_t b) {
+  const auto s = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  return s[0] | s[1];
+}
+// shift the sign bit of d into v
+__device__ __forceinline__ uint32_t push_sign(uint32_t v, float d) {
+  return __builtin_amdgcn_alignbit(v, __builtin_bit_cast(uint32_t, d), 31);
+}
+// (one instruction; fmaxf would first quiet each operand)
+__device__ __forceinline__ float max2(float x, float y) { return __builtin_elementwise_maximum(x, y); }
+// x of lane l ^ 1
+__device__ __forceinline__ float swap_pair(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, true));  // [1, 0, 3, 2]
 }
 
-constexpr int kSlot = 80;     // LDS bytes per staged pixel
-constexpr int kStageMax = 2;  // staged pixels per thread and chunk
-// A ring: 3 slots of 64 channels x 80 bytes (64 of weights, 16 of padding,
-// so a read's 16 lanes of one 16-byte column hit distinct banks)
-constexpr int kArow = 80;
-constexpr uint32_t kAslot = 64 * kArow;
-constexpr uint32_t kAring = 3 * kAslot;
+// n / d for 0 <= n < 2^31 as mulhi(2n, mul) >> sh, for any d >= 1 without a
+// branch: sh = ceil(log2 d), mul = ceil(2^(31 + sh) / d)
+struct KDiv {
+  uint32_t d, mul, sh;
+};
+inline KDiv make_kdiv(uint32_t d) {
+  KDiv f{d, 0u, 0u};
+  while ((1ull << f.sh) < d) ++f.sh;
+  f.mul = (uint32_t)(((1ull << (31 + f.sh)) + d - 1) / d);
+  return f;
+}
 
+// The tile geometry of one launch, and where its LDS regions lie.
 struct MfmaTile {
-  int lw, ltr, lti;     // log2 of TW, of rows per patch in a tile (min(TR, H)), of patches per tile
-  int lcw;              // log2 of tiles across a row (W / TW)
-  int hpt;              // tiles per patch (H / TR * W / TW), 1 for multi-patch tiles
-  int rs, ps;           // LDS bytes per staged row, per staged patch
-  FastDiv dps, drow;    // staged pixels per patch, per row
-  int ns;               // staged pixels per chunk buffer
+  int TW, TR, TI;         // columns, rows, patches of a tile (TI > 1: whole patches)
+  KDiv dpat, dcol;        // pixels (pool: 2x2 blocks) per patch of a tile, per row
+  KDiv dsp, dsr;          // staged pixels per patch, per row
+  KDiv dhp, dtc;          // tiles per patch, per row of tiles
+  int npat;               // dpat.d * TI: pixels (blocks) of a tile
+  int sub;                // tiles staged together: the next one's is subn patches or suby rows on,
+  int subn, suby;         // subl bytes of a staged plane on
+  uint32_t subl;
+  int ns;                 // staged pixels
+  int ps, planes;         // words per staged pixel and plane, planes
+  uint32_t plane_b;       // bytes of a plane
+  uint32_t off_tab, off_s, off_a;  // LDS bytes: slot offsets, -S - c, weights
   uint32_t ntiles;
-  uint32_t wbytes;      // weight table bytes
-  int npair, nc0, nch;  // pairs; chunks of the first segment, in total
+  int ncg;                // channel groups
+  int steps, slots;
+  int resident;
 };
 
-template <int EPI, bool DUMP>
-__global__ __launch_bounds__(256) void k_bconv_mfma(const BconvArgs a, const int8_t* __restrict__ wi8,
-                                                   const int32_t* __restrict__ stab, const MfmaTile T,
-                                                   uint32_t bytes0, uint32_t bytes1) {
+// The kernel's arguments, read where they are used straight from the kernarg
+// segment: held across the tile loop they took twice the scalar registers
+// there are.  fresh() makes a new pointer the compiler cannot trace, so loads
+// through it stay in their section.
+struct MfmaParams {
+  BconvArgs a;
+  MfmaConv mc;
+  MfmaTile T;
+  uint32_t bytes0, bytes1;
+};
+typedef const __attribute__((address_space(4))) MfmaParams* MfmaKarg;
+typedef const __attribute__((address_space(4))) KDiv* DivKarg;
+__device__ __forceinline__ MfmaKarg fresh(MfmaKarg k) {
+  asm volatile("" : "+s"(k));
+  return k;
+}
+__device__ __forceinline__ uint32_t kdiv(uint32_t n, DivKarg f) { return __umulhi(2u * n, f->mul) >> f->sh; }
+
+// waves a SIMD (blocks a CU) the registers are held to
+constexpr int mfma_waves(int mt, int epi) { return (mt < 4 ? 4 : 3) - (mt > 1 && epi == EPI_P ? 1 : 0); }
+
+template <int MT, int G, int EPI, bool RES>
+__global__ __launch_bounds__(256, mfma_waves(MT, EPI)) void k_bconv_mfma(const MfmaParams) {
+  const MfmaKarg kp = (MfmaKarg)__builtin_amdgcn_kernarg_segment_ptr();
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  constexpr uint32_t kFar = 0x80000000u;
   const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, j = lane & 15, wave = tid >> 6;
-  const int ncot = a.cout >> 6;  // 64-channel groups
-  const uint32_t nitems = T.ntiles * (uint32_t)ncot;
-  const int coutp = a.cout;
-  const int h = q & 1;
-  const int W = a.W, H = a.H;
-  // this lane's pixel in each of its four groups, within a tile: patch,
-  // row, column (the same for every tile)
-  int pi[4], py[4], px[4];
+  const int H = kp->a.H, W = kp->a.W;
+  const uint32_t ntiles = kp->T.ntiles, ncg = (uint32_t)kp->T.ncg;
+  // block -> XCD, channel group, first tile; tiles advance by nslot * 8
+  const uint32_t xcd = blockIdx.x & 7u, bi = blockIdx.x >> 3, tstep = (gridDim.x >> 3) / ncg * 8u;
+  const int cg = (int)(bi % ncg);
+  uint32_t tile = (bi / ncg) * 8u + xcd;
+  if (tile >= ntiles) return;
+  const int co0 = cg * MT * 16;
+
+  // this lane's pixel of each group, within a tile (the same for every
+  // tile): patch, row, column.  Pixels are numbered along the tile's rows,
+  // group g = 16 consecutive ones; EPI_P takes 4j + g instead, so a lane's
+  // four pixels are neighbours and its P leaves in 16-byte stores; a pooled
+  // tile numbers its 2x2 blocks, groups 2p and 2p + 1 hold the upper and
+  // lower rows of eight of them.
+  uint32_t lb[G];
+  int pc[G];  // patch << 20 | row << 10 | column, -1 past the tile
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    int l;  // tile-local row-major pixel index
+  for (int g = 0; g < G; ++g) {
+    int ip, r, c;
+    bool in;
     if (EPI == EPI_POOL) {
-      // block 8 * (group pair) + j / 2 of the wave's 16, row g % 2 of it
-      const int blk = 16 * wave + 8 * (g >> 1) + (j >> 1);
-      const int bx = blk & ((1 << (T.lw - 1)) - 1), br = blk >> (T.lw - 1);  // block row within the tile
-      l = ((2 * br + (g & 1)) << T.lw) + 2 * bx + (j & 1);
+      const int blk = wave * (G * 4) + 8 * (g >> 1) + (j >> 1);
+      in = blk < kp->T.npat;
+      const uint32_t b = in ? (uint32_t)blk : 0u;
+      ip = (int)kdiv(b, &kp->T.dpat);
+      const uint32_t rem = b - (uint32_t)ip * kp->T.dpat.d;
+      const uint32_t br = kdiv(rem, &kp->T.dcol);
+      r = 2 * (int)br + (g & 1);
+      c = 2 * (int)(rem - br * kp->T.dcol.d) + (j & 1);
+      in = in && r < kp->T.TR && c < kp->T.TW;
     } else {
-      l = 64 * wave + 16 * g + j;
+      const int l = wave * (G * 16) + (EPI == EPI_P ? G * j + g : 16 * g + j);
+      in = l < kp->T.npat;
+      const uint32_t b = in ? (uint32_t)l : 0u;
+      ip = (int)kdiv(b, &kp->T.dpat);
+      const uint32_t rem = b - (uint32_t)ip * kp->T.dpat.d;
+      r = (int)kdiv(rem, &kp->T.dcol);
+      c = (int)(rem - (uint32_t)r * kp->T.dcol.d);
     }
-    px[g] = l & ((1 << T.lw) - 1);
-    const int r = l >> T.lw;
-    py[g] = r & ((1 << T.ltr) - 1);
-    pi[g] = r >> T.ltr;
+    if (!in) { ip = 0; r = 0; c = 0; }
+    lb[g] = ((uint32_t)ip * kp->T.dsp.d + (uint32_t)r * kp->T.dsr.d + (uint32_t)c) * (uint32_t)(kp->T.ps * 4);
+    pc[g] = in ? (ip << 20 | r << 10 | c) : -1;
   }
-  const int lq = (q >> 1) * 32 + h * 16;  // this lane's 16 bytes in a slot
-  uint32_t lb[4];
+  // the pixel whose word this lane stores (the epilogue's lane rows)
+  int po = pc[0];
 #pragma unroll
-  for (int g = 0; g < 4; ++g)
-    lb[g] = (uint32_t)(pi[g] * T.ps + (py[g] + 1) * T.rs + (px[g] + 1) * kSlot + lq);
-  const uint32_t bufb = (uint32_t)(T.ps << T.lti);  // bytes per buffer
+  for (int g = 1; g < G; ++g)
+    if ((G == 4 ? q : q >> 1) == g) po = pc[g];
 
-  const __amdgpu_buffer_rsrc_t rw = make_rsrc(wi8, T.wbytes);
-  const __amdgpu_buffer_rsrc_t r0 = make_rsrc(a.in0, bytes0);
-  const __amdgpu_buffer_rsrc_t r1 = make_rsrc(a.in1 ? a.in1 : a.in0, bytes1);
-  const uint32_t cw0b = (uint32_t)a.cw0 * 4u, cw1b = (uint32_t)a.cw1 * 4u;
-  // item it: tile it / ncot (patches n0 .. n0 + 2^lti - 1, rows y0 ..
-  // y0 + 2^ltr - 1
-  // (columns x0 .. x0 + TW - 1), output channels 64 * (it % ncot) ..
-  auto tile_n0 = [&](uint32_t it) { return (int)((it / (uint32_t)ncot) / (uint32_t)T.hpt) << T.lti; };
-  auto tile_y0 = [&](uint32_t it) { return (int)(((it / (uint32_t)ncot) % (uint32_t)T.hpt) >> T.lcw) << T.ltr; };
-  auto tile_x0 = [&](uint32_t it) {
-    return (int)(((it / (uint32_t)ncot) % (uint32_t)T.hpt) & ((1u << T.lcw) - 1u)) << T.lw;
+  // ---- staging: piece e = words 4p .. of staged pixel i (e = p * ns + i)
+  auto coords = [&](uint32_t t, int* n0, int* y0, int* x0) {
+    const MfmaKarg k = fresh(kp);
+    const uint32_t tp = kdiv(t, &k->T.dhp), tr = t - tp * k->T.dhp.d;  // patch (group), tile within the patch
+    const uint32_t ty = kdiv(tr, &k->T.dtc);
+    *n0 = (int)tp * (k->T.TI > 1 ? k->T.TI * k->T.sub : 1);
+    *y0 = (int)ty * (k->T.TR * (k->T.TI > 1 ? 1 : k->T.sub));
+    *x0 = (int)(tr - ty * k->T.dtc.d) * k->T.TW;
   };
-
-  // ---- staging: the two words of chunk c of item it for this thread's staged pixels
-  uint32_t sw[kStageMax][2];
-  auto stage_load = [&](uint32_t it, int c) {
-    const int n0 = tile_n0(it), y0 = tile_y0(it), x0 = tile_x0(it);
-    const bool s1 = c >= T.nc0;
-    const int wd = 2 * (s1 ? c - T.nc0 : c);
-    const bool two = wd + 1 < (s1 ? a.cw1 : a.cw0);
-#pragma unroll
-    for (int k = 0; k < kStageMax; ++k) {
-      const uint32_t i = (uint32_t)(tid + 256 * k);
-      const uint32_t ip = fdiv(i, T.dps), ir = i - ip * T.dps.d, rr = fdiv(ir, T.drow), cc = ir - rr * T.drow.d;
-      const int n = n0 + (int)ip, y = y0 + (int)rr - 1, x = x0 + (int)cc - 1;
-      bool ok = i < (uint32_t)T.ns && n < a.N && (unsigned)y < (unsigned)H && (unsigned)x < (unsigned)W;
-      uint32_t off;
-      if (!s1) {
-        off = (((uint32_t)n * (uint32_t)H + (uint32_t)y) * (uint32_t)W + (uint32_t)x) * cw0b + (uint32_t)wd * 4u;
-      } else {
-        // nearest 2x upsample placed at (oh, ow); positions it does not
-        // cover read 0 bits
-        const int uy = y - a.oh, ux = x - a.ow;
-        ok = ok && (unsigned)uy < (unsigned)a.uh && (unsigned)ux < (unsigned)a.uw;
-        off = (((uint32_t)n * (uint32_t)a.h1 + (uint32_t)(uy >> 1)) * (uint32_t)a.w1 + (uint32_t)(ux >> 1)) * cw1b +
-              (uint32_t)wd * 4u;
+  // the byte offsets of staged pixel i in the two inputs, and of its right
+  // neighbour in the first (kFar: outside the image, reads 0)
+  auto stage_offs = [&](MfmaKarg k, uint32_t i, int n0, int y0, int x0, uint32_t& off0, uint32_t& off1, uint32_t& offn) {
+    // (recomputed for every tile: kept, it took a dozen registers a pixel)
+    asm volatile("" : "+v"(i));
+    const uint32_t ip = kdiv(i, &k->T.dsp), ir = i - ip * k->T.dsp.d;
+    const uint32_t rr = kdiv(ir, &k->T.dsr), cc = ir - rr * k->T.dsr.d;
+    const int n = n0 + (int)ip, y = y0 + (int)rr - 1, x = x0 + (int)cc - 1;
+    const bool okr = n < k->a.N && (unsigned)y < (unsigned)H, ok = okr && (unsigned)x < (unsigned)W;
+    const uint32_t pix = ((uint32_t)n * (uint32_t)H + (uint32_t)y) * (uint32_t)W + (uint32_t)x;
+    off0 = ok ? pix * ((uint32_t)k->a.cw0 * 4u) : kFar;
+    // (in the column left of the image too: column 0's bits)
+    offn = okr && (unsigned)(x + 1) < (unsigned)W ? (pix + 1u) * 4u : kFar;
+    off1 = kFar;
+    if (k->a.cw1) {
+      // nearest 2x upsample placed at (oh, ow); what it does not cover reads at padoff
+      const int uy = y - k->a.oh, ux = x - k->a.ow;
+      off1 = (unsigned)uy < (unsigned)k->a.uh && (unsigned)ux < (unsigned)k->a.uw
+                 ? (((uint32_t)n * (uint32_t)k->a.h1 + (uint32_t)(uy >> 1)) * (uint32_t)k->a.w1 +
+                    (uint32_t)(ux >> 1)) * ((uint32_t)k->a.cw1 * 4u)
+                 : k->a.padoff;
+      off1 = ok ? off1 : kFar;
+    }
+  };
+  const uint32_t ns = (uint32_t)kp->T.ns;
+  // one plane (at most four words a pixel): pixel i's words
+  auto load_px = [&](MfmaKarg k, uint32_t i, int n0, int y0, int x0) -> i32x4v {
+    uint32_t off0, off1, offn;
+    stage_offs(k, i, n0, y0, x0, off0, off1, offn);
+    const int cw0 = k->a.cw0, cw1 = k->a.cw1;
+    const __amdgpu_buffer_rsrc_t r0 = make_rsrc(k->a.in0, k->bytes0);
+    i32x4v v = {0, 0, 0, 0};
+    if (cw0 == 4) {
+      v = __builtin_bit_cast(i32x4v, __builtin_amdgcn_raw_buffer_load_b128(r0, (int)off0, 0, 0));
+    } else {
+      v[0] = (int)ld_u32(r0, off0, 0);
+      if (cw0 > 1) v[1] = (int)ld_u32(r0, off0 + 4u, 0);
+      if (cw0 > 2) v[2] = (int)ld_u32(r0, off0 + 8u, 0);
+      if (k->a.pair) v[0] |= (int)(ld_u32(r0, offn, 0) << 16);
+      if (cw1) {
+        const __amdgpu_buffer_rsrc_t r1 = make_rsrc(k->a.in1, k->bytes1);
+        const int u0 = (int)ld_u32(r1, off1, 0), u1 = cw1 > 1 ? (int)ld_u32(r1, off1 + 4u, 0) : 0,
+                  u2 = cw1 > 2 ? (int)ld_u32(r1, off1 + 8u, 0) : 0;
+        if (cw0 == 1) { v[1] = u0; v[2] = u1; v[3] = u2; }
+        else if (cw0 == 2) { v[2] = u0; v[3] = u1; }
+        else v[3] = u0;
       }
-      off = ok ? off : kFar;
-      sw[k][0] = ld_u32(s1 ? r1 : r0, off, 0);
-      sw[k][1] = two ? ld_u32(s1 ? r1 : r0, off + 4u, 0) : 0u;
+    }
+    return v;
+  };
+  auto store_px = [&](MfmaKarg k, uint32_t i, const i32x4v& v) {
+    asm volatile("" : "+v"(i));
+    const int ps = k->T.ps;
+    if (ps == 4) {
+      *reinterpret_cast<i32x4v*>(smem + i * 16u) = v;
+    } else {
+      int* d = reinterpret_cast<int*>(smem) + i * (uint32_t)ps;
+      d[0] = v[0];
+      if (ps > 1) d[1] = v[1];
+      if (ps > 2) d[2] = v[2];
     }
   };
-  auto stage_store = [&](int buf) {
+  // several planes: pixel i, four planes' loads in flight
+  auto copy_px = [&](MfmaKarg k, uint32_t i, int n0, int y0, int x0) {
+    uint32_t off0, off1, offn;
+    stage_offs(k, i, n0, y0, x0, off0, off1, offn);
+    const int cw0 = k->a.cw0, cw = cw0 + k->a.cw1, planes = k->T.planes;
+    const uint32_t pb = k->T.plane_b;
+    const __amdgpu_buffer_rsrc_t r0 = make_rsrc(k->a.in0, k->bytes0);
+    const __amdgpu_buffer_rsrc_t r1 = make_rsrc(k->a.in1, k->bytes1);  // (read for words past cw0 only)
+#pragma unroll 1
+    for (int p0 = 0; p0 < planes; p0 += 4) {
+      i32x4v v[4];
 #pragma unroll
-    for (int k = 0; k < kStageMax; ++k) {
-      const uint32_t i = (uint32_t)(tid + 256 * k);
-      if (i < (uint32_t)T.ns) {
-        const uint32_t ip = fdiv(i, T.dps), ir = i - ip * T.dps.d, rr = fdiv(ir, T.drow), cc = ir - rr * T.drow.d;
-        uint8_t* d = smem + (uint32_t)buf * bufb + ip * (uint32_t)T.ps + rr * (uint32_t)T.rs + cc * kSlot;
+      for (int j = 0; j < 4; ++j) {
+        const int w0 = 4 * (p0 + j);
+        v[j] = i32x4v{0, 0, 0, 0};
+        if (w0 + 4 <= cw0) {
+          v[j] = __builtin_bit_cast(
+              i32x4v, __builtin_amdgcn_raw_buffer_load_b128(r0, (int)(off0 + (uint32_t)w0 * 4u), 0, 0));
+        } else if (w0 >= cw0 && w0 + 4 <= cw) {
+          v[j] = __builtin_bit_cast(
+              i32x4v, __builtin_amdgcn_raw_buffer_load_b128(r1, (int)(off1 + (uint32_t)(w0 - cw0) * 4u), 0, 0));
+        } else if (w0 < cw) {
 #pragma unroll
-        for (int w2 = 0; w2 < 2; ++w2)
-#pragma unroll
-          for (int hh = 0; hh < 2; ++hh)
-            *reinterpret_cast<i32x4v*>(d + 32 * w2 + 16 * hh) = bits_to_bytes((sw[k][w2] >> (16 * hh)) & 0xFFFFu);
+          for (int t = 0; t < 4; ++t) {
+            if (w0 + t < cw0) v[j][t] = (int)ld_u32(r0, off0 + (uint32_t)(w0 + t) * 4u, 0);
+            else if (w0 + t < cw) v[j][t] = (int)ld_u32(r1, off1 + (uint32_t)(w0 + t - cw0) * 4u, 0);
+          }
+        }
       }
+      if (k->a.pair && p0 == 0) v[0][0] |= (int)(ld_u32(r0, offn, 0) << 16);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (p0 + j < planes) *reinterpret_cast<i32x4v*>(smem + (uint32_t)(p0 + j) * pb + i * 16u) = v[j];
     }
   };
-
-  // ---- A: each thread stages 16 bytes of a K step's 64 x 64 weight
-  // bytes: channel ac = tid / 4 of the item's group, bytes 16 * (tid % 4);
-  // the table row of channel co, K step st is 64 bytes at (co * npair + 2 st) * 32
-  const int ac = tid >> 2, ap = tid & 3;
-  auto a_piece = [&](uint32_t itm, int st) {
-    return (uint32_t)((((int)(itm % (uint32_t)ncot) * 64 + ac) * T.npair + 2 * st) * 32 + 16 * ap);
-  };
-  auto a_load = [&](uint32_t itm, int st) {
-    return __builtin_bit_cast(i32x4v, __builtin_amdgcn_raw_buffer_load_b128(rw, (int)a_piece(itm, st), 0, 0));
-  };
-  const uint32_t aring = 2 * bufb;  // the ring after the two staging buffers
-  auto a_store = [&](uint32_t slot, const i32x4v& v) {
-    *reinterpret_cast<i32x4v*>(smem + aring + slot * kAslot + (uint32_t)(ac * kArow + 16 * ap)) = v;
-  };
-  // the wave's operand A[m] (channel 16 m + j, K bytes 16 q ..) from a slot
-  auto a_read = [&](uint32_t slot, i32x4v (&A)[4]) {
+  const bool one = RES && kp->T.planes == 1;  // (a streamed group has more than one)
+  // one plane: a thread's first kAhead pixels are loaded while the tile
+  // before is multiplied
+  constexpr int kAhead = 2;
+  i32x4v st[kAhead];
+  int n0, y0, x0;
+  coords(tile, &n0, &y0, &x0);
+  if (one) {
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
-      A[m] = *reinterpret_cast<const i32x4v*>(smem + aring + slot * kAslot + (uint32_t)((16 * m + j) * kArow + 16 * q));
-  };
-
-  i32x4v acc[4][4];
-#pragma unroll
-  for (int m = 0; m < 4; ++m)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) acc[m][g] = i32x4v{0, 0, 0, 0};
-
-  // This block's items, XCD-aware: blocks go to the XCDs in turn (block b
-  // to XCD b % 8, the grid a multiple of 8), XCD x takes the tiles
-  // x, x + 8, x + 16, ... and its blocks walk that list's items (tile, then
-  // channel group fastest) in turn, so a tile's channel groups, which read
-  // the same staged rows and write different words of the same pixels, run
-  // side by side on one XCD and their stores merge in its L2.  Local item
-  // li of XCD x is tile (li / ncot) * 8 + x, group li % ncot; the chunks of
-  // all of a block's items form one pipeline.
-  const uint32_t xcd = blockIdx.x & 7u, nslot = gridDim.x >> 3;
-  auto item_of = [&](uint32_t li) -> uint32_t {
-    const uint32_t tile = (li / (uint32_t)ncot) * 8u + xcd;
-    return tile < T.ntiles ? tile * (uint32_t)ncot + li % (uint32_t)ncot : 0xFFFFFFFFu;
-  };
-  uint32_t li = blockIdx.x >> 3;
-  uint32_t it = item_of(li);
-  if (it >= nitems) return;
-  stage_load(it, 0);
-  stage_store(0);
-  // the chunk after (it, c) is (it, c + 1), or (the block's next item, 0)
-  uint32_t lli = li, lit = it;  // item and chunk of the staged-ahead words in sw
-  int lc = 0;
-  bool lok = true;
-  auto advance = [&]() {
-    if (++lc == T.nch) {
-      lc = 0;
-      lli += nslot;
-      lit = item_of(lli);
-      lok = lit < nitems;
+    for (int k = 0; k < kAhead; ++k) {
+      st[k] = i32x4v{0, 0, 0, 0};
+      if (tid + 256u * k < ns) st[k] = load_px(kp, (uint32_t)tid + 256u * k, n0, y0, x0);
     }
+  }
+
+  // weights: step st of this channel group is MT KB at wg + st * MT KB
+  const int steps = kp->T.steps;
+  const i32x4v* wg = reinterpret_cast<const i32x4v*>(kp->mc.w) + (size_t)cg * steps * MT * 64;
+  i32x4v* abuf = reinterpret_cast<i32x4v*>(smem + kp->T.off_a);
+  const int nph = RES ? 1 : (steps + kPhase - 1) / kPhase, na = steps * MT * 64;
+  constexpr int kAL = kPhase * MT / 4;  // 16-byte pieces a thread moves per phase
+  i32x4v ap[kAL];
+  auto a_fetch = [&](int ph) {
+#pragma unroll
+    for (int k = 0; k < kAL; ++k) ap[k] = wg[min(ph * (kPhase * MT * 64) + k * 256 + tid, na - 1)];
   };
-  advance();
-  if (lok) stage_load(lit, lc);
-  // the K steps of the block's items run as one sequence: step S (item
-  // steps st = c * 9 + t) takes A from slot S % 3; at its start (a barrier)
-  // A of step S + 1 is visible and slot (S + 2) % 3 is free
-  const int nst = T.nch * 9;  // K steps per item
-  auto a_load_ahead = [&](int st) {  // A of in-item step st, or of the next item past its end
-    return st < nst ? a_load(it, st) : a_load(item_of(li + nslot), st - nst);
+  auto a_put = [&](int buf) {
+#pragma unroll
+    for (int k = 0; k < kAL; ++k) abuf[buf * (kPhase * MT * 64) + k * 256 + tid] = ap[k];
   };
-  a_store(0, a_load(it, 0));
-  a_store(1, a_load_ahead(1));
-  i32x4v ag = a_load_ahead(2);   // A of step S + 2, stored during step S
-  i32x4v ag2 = a_load_ahead(3);  // A of step S + 3
-  __syncthreads();
-  i32x4v Ar[4];
-  a_read(0, Ar);
-  uint32_t S = 0;
-  int buf = 0;
+  // slot offsets and border sums, then the weights, each batch's loads
+  // issued together
+  uint32_t* tab = reinterpret_cast<uint32_t*>(smem + kp->T.off_tab);
+  float* stab = reinterpret_cast<float*>(smem + kp->T.off_s);
+  {
+    // [16 border classes][channel] -S - c1, then per channel r1, c1 - c2, r2
+    constexpr int kC4 = MT * 4, kS4 = 16 * kC4, kT4 = kS4 + 3 * kC4;  // float4s
+    constexpr int kTB = (kT4 + 255) / 256;
+    f32x4v sv[kTB];
+#pragma unroll
+    for (int k = 0; k < kTB; ++k) {
+      const int i = tid + 256 * k, row = i / kC4;
+      const float* src = row < 16 ? kp->mc.s + (size_t)row * kp->mc.coutp : row == 16 ? kp->mc.r1 : row == 17 ? kp->mc.c12 : kp->mc.r2;
+      sv[k] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
+      if (i < kT4 && src) sv[k] = *reinterpret_cast<const f32x4v*>(src + co0 + i % kC4 * 4);
+    }
+    if constexpr (RES) {
+      constexpr int kB = 5;
+      for (int i = tid; i < na; i += 256 * kB) {
+        i32x4v r[kB];
+#pragma unroll
+        for (int k = 0; k < kB; ++k) r[k] = wg[min(i + 256 * k, na - 1)];
+#pragma unroll
+        for (int k = 0; k < kB; ++k)
+          if (i + 256 * k < na) abuf[i + 256 * k] = r[k];
+      }
+    } else {
+      a_fetch(0);
+      a_put(0);
+      a_fetch(1);  // a streamed group has at least two phases
+    }
+    for (int s = tid; s < steps * 4; s += 256) {
+      const uint32_t sl = s < kp->T.slots ? kp->mc.slot[s] : 0u;  // tap | word << 8 (past the last: any, the weights are 0)
+      const uint32_t t = sl & 255u, wd = sl >> 8;
+      tab[s] = (t / 3 * kp->T.dsr.d + t % 3) * (uint32_t)(kp->T.ps * 4) + (wd >> 2) * kp->T.plane_b + (wd & 3) * 4u;
+    }
+#pragma unroll
+    for (int k = 0; k < kTB; ++k)
+      if (tid + 256 * k < kT4) *reinterpret_cast<f32x4v*>(stab + (tid + 256 * k) * 4) = sv[k];
+  }
+  int abf = 0;
+
 #pragma unroll 1
   for (;;) {
+    const MfmaKarg ks = fresh(kp);
+    if (one) {
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k)
+        if (tid + 256u * k < ns) store_px(ks, (uint32_t)tid + 256u * k, st[k]);
 #pragma unroll 1
-    for (int c = 0; c < T.nch; ++c) {
-      const uint32_t bo = (uint32_t)buf * bufb;
-#pragma unroll
-      for (int t = 0; t < 9; ++t) {
-        const int ky = t / 3, kx = t % 3;
-        __syncthreads();
-        const uint32_t s0 = S % 3u, s1 = s0 == 2u ? 0u : s0 + 1u, s2 = s1 == 2u ? 0u : s1 + 1u;
-        i32x4v An[4];
-        a_read(s1, An);
-        const uint32_t dt = bo + (uint32_t)((ky - 1) * T.rs + (kx - 1) * kSlot);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const i32x4v B = *reinterpret_cast<const i32x4v*>(smem + lb[g] + dt);
-#pragma unroll
-          for (int m = 0; m < 4; ++m) acc[m][g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(Ar[m], B, acc[m][g], 0, 0, 0);
-        }
-        // A of step S + 2 into its slot, the load of step S + 4
-        a_store(s2, ag);
-        ag = ag2;
-        ag2 = a_load_ahead(c * 9 + t + 4);
-#pragma unroll
-        for (int m = 0; m < 4; ++m) Ar[m] = An[m];
-        ++S;
+      for (uint32_t i = (uint32_t)tid + 256u * kAhead; i < ns; i += 512u) {
+        const i32x4v v0 = load_px(ks, i, n0, y0, x0);
+        i32x4v v1 = {0, 0, 0, 0};
+        if (i + 256u < ns) v1 = load_px(ks, i + 256u, n0, y0, x0);
+        store_px(ks, i, v0);
+        if (i + 256u < ns) store_px(ks, i + 256u, v1);
       }
-      // the next chunk into the other buffer (visible after the next step's
-      // barrier), the one after it from HBM
-      if (lok) {
-        stage_store(buf ^ 1);
-        advance();
-        if (lok) stage_load(lit, lc);
-      }
-      buf ^= 1;
+    } else {
+#pragma unroll 1
+      for (uint32_t i = (uint32_t)tid; i < ns; i += 256u) copy_px(ks, i, n0, y0, x0);
     }
-    // ---------------------------------------------------------- epilogue --
-    // one group of 16 channels at a time: P, the rule, and the gather into
-    // 16-bit halves of the output words; then the word stores
+    __syncthreads();
+    const uint32_t next = tile + tstep;
+    int n1, y1, x1;
+    coords(next, &n1, &y1, &x1);
+    if (one && next < ntiles) {
+      const MfmaKarg kl = fresh(kp);
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k)
+        if (tid + 256u * k < ns) st[k] = load_px(kl, (uint32_t)tid + 256u * k, n1, y1, x1);
+    }
+
+    const int nsub = kp->T.sub;
+    uint32_t sl = 0;  // LDS bytes of the sub-tile
+#pragma unroll 1
+    for (int sb = 0; sb < nsub; ++sb) {
+    // ---- sums
+    f32x4v acc[MT][G];
     {
-      const int n0 = tile_n0(it), y0 = tile_y0(it), x0 = tile_x0(it);
-      const int co0 = (int)(it % (uint32_t)ncot) * 64;
-      const int HW = H * W;
-      const int Hh = H >> 1, Wh = W >> 1;
-      int cls[4];
-      bool pv[4];
-      size_t pix[4];  // global pixel index
+      int cls[G];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int y = y0 + py[g], x = x0 + px[g];
-        pv[g] = n0 + pi[g] < a.N;
-        cls[g] = ((y == 0 ? 1 : 0) | (y == H - 1 ? 2 : 0)) * 4 + ((x == 0 ? 1 : 0) | (x == W - 1 ? 2 : 0));
-        pix[g] = ((size_t)(n0 + pi[g]) * H + y) * W + x;
+      for (int g = 0; g < G; ++g) cls[g] = 0;
+      if (x0 == 0 || x0 + kp->T.TW >= W) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const int x = x0 + (pc[g] & 1023);
+          cls[g] = (x == 0 ? MT * 16 : 0) + (x == W - 1 ? 2 * MT * 16 : 0);
+        }
       }
-      uint32_t half[4][4], half2[4][2];
+      if (y0 == 0 || y0 + kp->T.TR >= H) {
 #pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const int cb = co0 + 16 * m + 4 * q;  // this lane's four channels cb .. cb+3
-        const i32x4v lo1 = *reinterpret_cast<const i32x4v*>(a.f1.lo + cb);
-        const i32x4v wd1 = *reinterpret_cast<const i32x4v*>(a.f1.wid + cb);
-        int32_t P[4][4];
+        for (int g = 0; g < G; ++g) {
+          const int y = y0 + ((pc[g] >> 10) & 1023);
+          cls[g] += (y == 0 ? 4 * MT * 16 : 0) + (y == H - 1 ? 8 * MT * 16 : 0);
+        }
+      }
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const i32x4v sv = *reinterpret_cast<const i32x4v*>(stab + (size_t)cls[g] * coutp + cb);
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[m][g] = *reinterpret_cast<const f32x4v*>(stab + cls[g] + m * 16 + q * 4);
+    }
+    {
+      uint32_t w0[G], w1[G];
+      i32x4v A0[MT], A1[MT];
+      auto rd_w = [&](uint32_t off, uint32_t (&w)[G]) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) w[g] = *reinterpret_cast<const uint32_t*>(smem + lb[g] + (sl + off));
+      };
+      auto mul = [&](const i32x4v (&A)[MT], const uint32_t (&w)[G]) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const i32x4v B = bits_f4(w[g]);
+#pragma unroll
+          for (int m = 0; m < MT; ++m) acc[m][g] = mfma_f4(A[m], B, acc[m][g]);
+        }
+      };
+      const uint32_t* tq = tab + q;
+      const int last = steps - 1;
+      rd_w(tq[0], w0);
+      uint32_t on = tq[4 * min(1, last)];
+      int s = 0;
+#pragma unroll 1
+      for (int ph = 0; ph < nph; ++ph) {
+        const i32x4v* ab = abuf + abf * (kPhase * MT * 64) + lane;
+        const int n = RES ? steps : min(kPhase, steps - ph * kPhase);
+        auto rd_a = [&](int k, i32x4v (&A)[MT]) {
+#pragma unroll
+          for (int m = 0; m < MT; ++m) A[m] = ab[(k * MT + m) * 64];
+        };
+        rd_a(0, A0);
+        int k = 0;
+#pragma unroll 1
+        for (; k + 2 <= n; k += 2, s += 2) {
+          rd_a(k + 1, A1);
+          rd_w(on, w1);
+          on = tq[4 * min(s + 2, last)];
+          mul(A0, w0);
+          rd_a(min(k + 2, n - 1), A0);
+          rd_w(on, w0);
+          on = tq[4 * min(s + 3, last)];
+          mul(A1, w1);
+        }
+        if (k < n) {
+          mul(A0, w0);
+          rd_w(on, w0);
+          on = tq[4 * min(s + 2, last)];
+          ++s;
+        }
+        if constexpr (!RES) {
+          // the next phase (of the next tile after the last) into the other
+          // buffer, which every wave left before the previous barrier
+          abf ^= 1;
+          a_put(abf);
+          a_fetch((ph + 2) % nph);
+          __syncthreads();
+        }
+      }
+    }
+
+    // ---- epilogue: acc = P - c1
+    const MfmaKarg ke = fresh(kp);
+    const int HW = H * W;
+    const int cb = co0 + 4 * q;  // this lane's channels: cb + 16 m + r
+    // a pixel code's patch, row and column, and whether it is in the image
+    auto at = [&](int code, int* n, int* y, int* x) {
+      *n = n0 + (code >> 20);
+      *y = y0 + ((code >> 10) & 1023);
+      *x = x0 + (code & 1023);
+      return code >= 0 && *n < ke->a.N && *y < H && *x < W;
+    };
+    if constexpr (EPI == EPI_P) {
+      bool pv[G], run = G == 4;
+      size_t pp[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        int n, y, x;
+        pv[g] = at(pc[g], &n, &y, &x);
+        pp[g] = (size_t)n * ke->a.cout * HW + (size_t)y * W + x;
+        run = run && pv[g] && pp[g] == pp[0] + (size_t)g;
+      }
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const f32x4v c1 = *reinterpret_cast<const f32x4v*>(ke->mc.c1 + cb + 16 * m);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (cb + 16 * m + r >= ke->a.cout) continue;
+          int32_t* const plane = ke->a.P + (size_t)(cb + 16 * m + r) * HW;
+          if (run) {
+            i32x4u v;
+#pragma unroll
+            for (int g = 0; g < G; ++g) v[g] = (int)(acc[m][g][r] + c1[r]);
+            *reinterpret_cast<i32x4u*>(plane + pp[0]) = v;
+          } else {
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+              if (pv[g]) plane[pp[g]] = (int)(acc[m][g][r] + c1[r]);
+          }
+        }
+      }
+    }
+    if constexpr (EPI != EPI_P) {
+      constexpr int NW = (MT + 1) / 2;  // output words of the group
+      const uint32_t* iv1 = ke->mc.inv1 + (co0 >> 5);
+      // rule 1 per channel: |P - c1| < r1 (inverted channels flipped on the
+      // packed word).  A lane has 4 channels of each 16 as a nibble at 4q
+      // (m odd: 16 + 4q) of the word; the four lane rows are OR-ed together
+      // by two lane swaps, which also leave lane row q with group q's pixel.
+      uint32_t v[NW][G];
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int h = 0; h < NW; ++h) v[h][g] = 0u;
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const f32x4v r1v = *reinterpret_cast<const f32x4v*>(stab + 16 * MT * 16 + m * 16 + q * 4);
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
           uint32_t nib = 0;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            P[g][r] = 2 * acc[m][g][r] - sv[r];
-            nib |= ((uint32_t)P[g][r] - (uint32_t)lo1[r] < (uint32_t)wd1[r] ? 1u : 0u) << r;
-            if (DUMP && pv[g]) a.P[((size_t)(n0 + pi[g]) * a.cout + cb + r) * HW + (size_t)(y0 + py[g]) * W + x0 + px[g]] = P[g][r];
-          }
-          half[m][g] = or_groups(nib << (4 * q));
-        }
-        if constexpr (EPI == EPI_POOL) {
-          const i32x4v lo2 = *reinterpret_cast<const i32x4v*>(a.f2.lo + cb);
-          const i32x4v wd2 = *reinterpret_cast<const i32x4v*>(a.f2.wid + cb);
-#pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            uint32_t nib2 = 0;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int32_t pm = max_pair(max(P[2 * p][r], P[2 * p + 1][r]));
-              nib2 |= ((uint32_t)pm - (uint32_t)lo2[r] < (uint32_t)wd2[r] ? 1u : 0u) << r;
-              if (DUMP && pv[2 * p] && (j & 1) == 0)
-                a.P2[((size_t)(n0 + pi[2 * p]) * a.cout + cb + r) * Hh * Wh + (size_t)((y0 + py[2 * p]) >> 1) * Wh +
-                     ((x0 + px[2 * p]) >> 1)] = pm;
-            }
-            half2[m][p] = or_groups(nib2 << (4 * q));
-          }
-        }
-      }
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        if (a.out != nullptr && pv[g] && q < 2) {  // a pooled layer may skip its full-size bits
-          const uint32_t word = q == 0 ? (half[0][g] | half[1][g] << 16) : (half[2][g] | half[3][g] << 16);
-          a.out[pix[g] * a.cwo + (co0 >> 5) + q] = word;
+          for (int r = 3; r >= 0; --r) nib = push_sign(nib, __builtin_fabsf(acc[m][g][r]) - r1v[r]);
+          v[m >> 1][g] |= nib << (4 * q + 16 * (m & 1));
         }
       }
       if constexpr (EPI == EPI_POOL) {
+        const uint32_t* iv2 = ke->mc.inv2 + (co0 >> 5);
+        const int Hh = H >> 1, Wh = W >> 1;
+        // the max of a block's P: the rows (groups 2p, 2p + 1), then the two
+        // columns (lanes j, j ^ 1).  G = 4: the even lanes take the blocks of
+        // pair 0, the odd ones those of pair 1.
+        uint32_t u[NW];
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          if (pv[2 * p] && (j & 1) == 0 && q < 2) {
-            const uint32_t word = q == 0 ? (half2[0][p] | half2[1][p] << 16) : (half2[2][p] | half2[3][p] << 16);
-            const size_t dp = ((size_t)(n0 + pi[2 * p]) * Hh + ((y0 + py[2 * p]) >> 1)) * Wh + ((x0 + px[2 * p]) >> 1);
-            a.out2[dp * a.cwo + (co0 >> 5) + q] = word;
+        for (int h = 0; h < NW; ++h) u[h] = 0u;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          const f32x4v dc = *reinterpret_cast<const f32x4v*>(stab + 17 * MT * 16 + m * 16 + q * 4);
+          const f32x4v r2v = *reinterpret_cast<const f32x4v*>(stab + 18 * MT * 16 + m * 16 + q * 4);
+          uint32_t nib = 0;
+#pragma unroll
+          for (int r = 3; r >= 0; --r) {
+            const float v0 = max2(acc[m][0][r], acc[m][1][r]);
+            float pm;
+            if constexpr (G == 4) {
+              const float v1 = max2(acc[m][2][r], acc[m][3][r]);
+              pm = max2(j & 1 ? v1 : v0, swap_pair(j & 1 ? v0 : v1));
+            } else {
+              pm = max2(v0, swap_pair(v0));
+            }
+            nib = push_sign(nib, __builtin_fabsf(pm + dc[r]) - r2v[r]);
+          }
+          u[m >> 1] |= nib << (4 * q + 16 * (m & 1));
+        }
+        // lane row q -> word q / 2
+        const uint32_t t = or_halves(u[0], u[NW - 1]), d = or_rows(t, t);
+        const int wd = q >> 1;
+        int n, y, x;
+        const bool ok = at(G == 4 && (j & 1) ? pc[G - 2] : pc[0], &n, &y, &x) && y + 1 < H && x < 2 * Wh && wd < NW &&
+                        (G == 4 || (j & 1) == 0) && (q & 1) == 0 && (co0 >> 5) + wd < ke->a.cwo;
+        if (ok) ke->a.out2[(((size_t)n * Hh + (y >> 1)) * Wh + (x >> 1)) * ke->a.cwo + (co0 >> 5) + wd] = d ^ iv2[wd];
+      }
+      // lane row -> (group, word): G = 4: group q, all words; G = 2: group
+      // q / 2, word q % 2
+      uint32_t o[NW];
+      if constexpr (G == 4) {
+#pragma unroll
+        for (int h = 0; h < NW; ++h) o[h] = or_rows(or_halves(v[h][0], v[h][2]), or_halves(v[h][1], v[h][3])) ^ iv1[h];
+      } else {
+        const uint32_t t0 = or_halves(v[0][0], v[0][1]), t1 = or_halves(v[NW - 1][0], v[NW - 1][1]);
+        o[0] = or_rows(t0, t1);
+      }
+      int on_, oy, ox;
+      const bool ov = at(po, &on_, &oy, &ox);
+      if (ke->a.out != nullptr && ov) {
+        uint32_t* dst = ke->a.out + (((size_t)on_ * H + oy) * W + ox) * ke->a.cwo + (co0 >> 5);
+        if constexpr (G == 4) {
+#pragma unroll
+          for (int h = 0; h < NW; ++h)
+            if ((co0 >> 5) + h < ke->a.cwo) dst[h] = o[h];
+        } else {
+          const int h = q & 1;
+          if (h < NW && (co0 >> 5) + h < ke->a.cwo) dst[h] = o[0] ^ iv1[h];
+        }
+      }
+      if constexpr (EPI == EPI_HEAD) {
+        // one pixel per lane: bias, then the channels in order, one fused
+        // step each (csrc/bnn_head.c:21-34)
+        bool keep = ov;
+        size_t lbase = (size_t)on_ * ke->a.ncls * HW + (size_t)oy * W + ox, lstride = HW;
+        if (ke->a.pcols > 0) {
+          const int prw = ke->a.prow0 + on_ / ke->a.pcols, pcl = on_ % ke->a.pcols;
+          const int sy = prw * H + oy, sx = pcl * W + ox;
+          keep = keep && sy < ke->a.sH && sx < ke->a.sW;
+          lbase = (size_t)sy * ke->a.sW + sx;
+          lstride = (size_t)ke->a.sH * ke->a.sW;
+        }
+        typedef const __attribute__((address_space(4))) float* const_hf;
+        const const_hf hw = (const_hf)ke->a.hw, hb = (const_hf)ke->a.hb;
+        float sg[MT * 16];
+#pragma unroll
+        for (int c = 0; c < MT * 16; ++c) sg[c] = (o[0] >> c) & 1u ? 1.0f : -1.0f;
+        if (keep) {
+          if (ke->a.cout == MT * 16) {
+#pragma unroll 1
+            for (int k = 0; k < ke->a.ncls; ++k) {
+              float wv[MT * 16];
+#pragma unroll
+              for (int c = 0; c < MT * 16; ++c) wv[c] = hw[k * (MT * 16) + c];
+              float s = hb[k];
+#pragma unroll
+              for (int c = 0; c < MT * 16; ++c) s = __fmaf_rn(wv[c], sg[c], s);
+              ke->a.logits[lbase + (size_t)k * lstride] = s;
+            }
+          } else {
+#pragma unroll 1
+            for (int k = 0; k < ke->a.ncls; ++k) {
+              float s = hb[k];
+#pragma unroll
+              for (int c = 0; c < MT * 16; ++c)
+                if (c < ke->a.cout) s = __fmaf_rn(hw[k * ke->a.cout + c], sg[c], s);
+              ke->a.logits[lbase + (size_t)k * lstride] = s;
+            }
           }
         }
       }
     }
-    li += nslot;
-    it = item_of(li);
-    if (it >= nitems) break;
-#pragma unroll
-    for (int m = 0; m < 4; ++m)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) acc[m][g] = i32x4v{0, 0, 0, 0};
+    sl += kp->T.subl;
+    n0 += kp->T.subn;
+    y0 += kp->T.suby;
+    if (y0 >= H || n0 >= kp->a.N) break;
+    }
+    if (next >= ntiles) break;
+    tile = next;
+    n0 = n1;
+    y0 = y1;
+    x0 = x1;
+    if (RES) __syncthreads();  // (a streamed group's last phase ended with one)
   }
 }
 
 }  // namespace
 
-// The tile of a (H, W) layer: TR = 256 / TW rows of TW columns of a patch
-// (TW = W up to 64 wide, else 32), or 256 / (H W) whole patches; false when
-// the shape has no such tile or its two staging buffers exceed 64 KB of LDS
-// (with the A ring, under 80 KB: two blocks a CU).
-static bool mfma_tile(int H, int W, int epi, MfmaTile* T) {
-  if (W < 8 || (W & (W - 1)) || W > (1 << 20) || H <= 0) return false;
-  if (epi == EPI_POOL && (H & 1)) return false;
-  const int TW = W > 64 ? 32 : W;
-  const int TR = 256 / TW;
-  int ltr = 0, lti = 0, hpt = 1, lcw = 0;
-  while ((TW << lcw) < W) ++lcw;
-  if (H >= TR) {
-    if (H % TR) return false;
-    hpt = (H / TR) << lcw;
-    while ((1 << ltr) < TR) ++ltr;
+// The tile of a layer for blocks of `pb` pixels: whole patches, whole rows
+// of a patch (rows up to 64 wide), or about 32 columns of wider rows; a
+// pooled tile has an even number of rows and counts 2x2 blocks.  `sub` such
+// tiles are staged together.
+static void mfma_tile(int N, int H, int W, int cw, bool pool, int pb, int sub, MfmaTile* T) {
+  const int We = pool ? (W + 1) & ~1 : W, He = pool ? (H + 1) & ~1 : H;
+  int tr, tw = W, ti = 1, ntr = 1, ntc = 1;
+  if ((long)We * He <= pb) {
+    tr = He;
+    // (at most 56 KB of staged words: two blocks a CU)
+    const long per = (long)(tr + 2) * (tw + 2) * (cw < 4 ? cw : (cw + 3) / 4 * 4) * 4;
+    ti = (int)std::max(1l, std::min({(long)N, (long)pb / (We * He), 56 * 1024 / per}));
   } else {
-    if (TW != W || TR % H || (H & (H - 1))) return false;
-    while ((1 << ltr) < H) ++ltr;
-    while ((1 << lti) < TR / H) ++lti;
+    if (We > 64) {
+      ntc = (We + 31) / 32;
+      tw = ((We + ntc - 1) / ntc + 3) & ~3;
+      ntc = (We + tw - 1) / tw;
+    }
+    const int wp = pool ? (tw + 1) & ~1 : tw;
+    int most = pb / wp;
+    if (pool) most &= ~1;
+    ntr = (He + most - 1) / most;
+    tr = (He + ntr - 1) / ntr;
+    if (pool) tr = (tr + 1) & ~1;
+    ntr = (He + tr - 1) / tr;
   }
-  int lw = 0;
-  while ((1 << lw) < TW) ++lw;
-  const int rows = (1 << ltr) + 2, cols = TW + 2;
-  int rs = cols * kSlot;
-  rs += (128 - rs % 256 + 256) % 256;  // rows 128 bytes apart mod 256
-  int ps = rows * rs;
-  if (2 * (ps << lti) > 65536) {  // no room for the padding
-    rs = cols * kSlot;
-    ps = rows * rs;
-  }
-  if (2 * (ps << lti) > 65536) return false;
-  const int ns = (rows * cols) << lti;
-  if (ns > 256 * kStageMax) return false;
-  if (T) {
-    T->lw = lw; T->ltr = ltr; T->lti = lti; T->lcw = lcw; T->hpt = hpt;
-    T->rs = rs; T->ps = ps;
-    T->dps = make_fastdiv((uint32_t)(rows * cols));
-    T->drow = make_fastdiv((uint32_t)cols);
-    T->ns = ns;
-  }
-  return true;
+  if (ti == 1) sub = std::min(sub, ntr);
+  const int px = pool ? (tr / 2) * ((tw + 1) / 2) : tr * tw;
+  const int srows = ti > 1 ? tr + 2 : tr * sub + 2;  // staged rows of a patch
+  T->TW = tw; T->TR = tr; T->TI = ti;
+  T->dpat = make_kdiv((uint32_t)px);
+  T->dcol = make_kdiv((uint32_t)(pool ? (tw + 1) / 2 : tw));
+  T->dsp = make_kdiv((uint32_t)(srows * (tw + 2)));
+  T->dsr = make_kdiv((uint32_t)(tw + 2));
+  ntr = (ntr + sub - 1) / sub;
+  T->dhp = make_kdiv((uint32_t)(ti > 1 ? 1 : ntr * ntc));
+  T->dtc = make_kdiv((uint32_t)ntc);
+  T->npat = px * ti;
+  T->sub = sub;
+  T->subn = ti > 1 ? ti : 0;
+  T->suby = ti > 1 ? 0 : tr;
+  T->ns = (ti > 1 ? ti * sub : 1) * srows * (tw + 2);
+  T->ntiles = ti > 1 ? (uint32_t)((N + ti * sub - 1) / (ti * sub)) : (uint32_t)((size_t)N * ntr * ntc);
 }
 
-bool mfma_conv_fits(int cout, int H, int W, int epi) {
-  return cout % 64 == 0 && (epi == EPI_FOLD || epi == EPI_POOL) && mfma_tile(H, W, epi, nullptr);
+// LDS bytes of a layer's block; fills the regions' offsets
+static size_t mfma_lds(const MfmaConv& mc, int cw, MfmaTile* T) {
+  T->ps = cw < 4 ? cw : 4;
+  T->planes = cw < 4 ? 1 : (cw + 3) / 4;
+  T->subl = (T->subn ? T->subn * T->dsp.d : T->suby * T->dsr.d) * (uint32_t)T->ps * 4;
+  T->plane_b = ((uint32_t)T->ns * T->ps * 4 + 15) & ~15u;
+  T->steps = mc.steps;
+  T->slots = mc.slots;
+  T->ncg = mc.coutp / (16 * mc.mt);
+  const size_t wb = (size_t)mc.steps * mc.mt * 1024;
+  T->resident = wb <= kResident;
+  T->off_tab = T->planes * T->plane_b;
+  T->off_s = T->off_tab + (uint32_t)mc.steps * 16;
+  T->off_a = T->off_s + (uint32_t)mc.mt * 19 * 64;
+  return T->off_a + (T->resident ? wb : (size_t)2 * kPhase * mc.mt * 1024);
 }
 
-hipError_t launch_bconv_mfma(const BconvArgs& a, const MfmaConv& mc, int epi, bool dump, hipStream_t s) {
-  if (a.N <= 0 || a.H <= 0 || a.W <= 0) return hipSuccess;
+bool mfma_conv_fits(const MfmaConv& mc, int cw, int N, int H, int W, int epi) {
+  if (!mc.w || H <= 0 || W <= 0) return false;
+  if (epi != EPI_FOLD && epi != EPI_POOL && epi != EPI_HEAD && epi != EPI_P) return false;
+  if (epi == EPI_HEAD && mc.mt > 2) return false;
+  if (epi != EPI_P && !mc.r1) return false;
+  if (epi == EPI_POOL && !mc.r2) return false;
   MfmaTile T{};
-  if ((epi != EPI_FOLD && epi != EPI_POOL) || !mc.w || !mc.s || a.cout % 64 || !mfma_tile(a.H, a.W, epi, &T))
-    return hipErrorInvalidValue;
-  if (a.in1 && a.padoff != 0x80000000u) return hipErrorInvalidValue;  // v1 concat semantics only
-  if (dump && (!a.P || (epi == EPI_POOL && !a.P2))) return hipErrorInvalidValue;  // dumps need their targets
+  mfma_tile(std::max(N, 1), H, W, cw, epi == EPI_POOL, 256, 1, &T);
+  return mfma_lds(mc, cw, &T) <= 160 * 1024;
+}
+
+namespace {
+using MfmaFn = void (*)(const MfmaParams);
+template <int MT, int G, bool RES>
+MfmaFn mfma_fn(int epi) {
+  switch (epi) {
+    case EPI_FOLD: return k_bconv_mfma<MT, G, EPI_FOLD, RES>;
+    case EPI_POOL: return k_bconv_mfma<MT, G, EPI_POOL, RES>;
+    case EPI_P: return k_bconv_mfma<MT, G, EPI_P, RES>;
+    case EPI_HEAD:
+      if constexpr (MT <= 2 && G == 4) return k_bconv_mfma<MT, G, EPI_HEAD, RES>;
+      break;
+  }
+  return nullptr;
+}
+template <bool RES>
+MfmaFn mfma_fn(int mt, int G, int epi) {
+  if (G == 4) return mt == 1 ? mfma_fn<1, 4, RES>(epi) : mt == 2 ? mfma_fn<2, 4, RES>(epi) : mfma_fn<4, 4, RES>(epi);
+  return mt == 1 ? mfma_fn<1, 2, RES>(epi) : mt == 2 ? mfma_fn<2, 2, RES>(epi) : mfma_fn<4, 2, RES>(epi);
+}
+}  // namespace
+
+hipError_t launch_bconv_mfma(const BconvArgs& a, const MfmaConv& mc, int epi, hipStream_t s) {
+  if (a.N <= 0 || a.H <= 0 || a.W <= 0) return hipSuccess;
+  const int cw = a.cw0 + a.cw1;
+  if (!mfma_conv_fits(mc, cw, a.N, a.H, a.W, epi) || a.cout > mc.coutp) return hipErrorInvalidValue;
+  if (mc.slots != mfma_nslots(a.cw0, a.cw1, a.pair)) return hipErrorInvalidValue;
+  if (epi == EPI_P && !a.P) return hipErrorInvalidValue;
+  if (epi == EPI_POOL && !a.out2) return hipErrorInvalidValue;
+  if (epi == EPI_FOLD && !a.out) return hipErrorInvalidValue;
   const size_t npix = (size_t)a.N * a.H * a.W;
   if (npix * a.cw0 * 4 >= 0x80000000ull) return hipErrorInvalidValue;
   if (a.in1 && (size_t)a.N * a.h1 * a.w1 * a.cw1 * 4 >= 0x80000000ull) return hipErrorInvalidValue;
-  T.npair = mc.npair;
-  T.nc0 = (a.cw0 + 1) / 2;
-  T.nch = mfma_nchunk(a.cw0, a.in1 ? a.cw1 : 0);
-  if (T.npair != 18 * T.nch) return hipErrorInvalidValue;
-  const size_t wbytes = (size_t)a.cout * T.npair * 32;
-  if (wbytes + 64 * 32 >= 0x80000000ull) return hipErrorInvalidValue;
-  T.wbytes = (uint32_t)wbytes;
-  const size_t per = (size_t)1 << T.lti;  // patches per tile
-  const size_t ntiles = T.lti ? (a.N + per - 1) / per : (size_t)a.N * T.hpt;
-  if (ntiles >= 0x7FFFFFFFull) return hipErrorInvalidValue;
-  T.ntiles = (uint32_t)ntiles;
-  const uint32_t b0 = (uint32_t)(npix * a.cw0 * 4);
-  const uint32_t b1 = a.in1 ? (uint32_t)((size_t)a.N * a.h1 * a.w1 * a.cw1 * 4) : 0u;
-  const size_t lds = (size_t)2 * ((size_t)T.ps << T.lti) + kAring;
+  int dev = 0;
+  if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
+  const int cus = device_cus();
+  const bool pool = epi == EPI_POOL;
+  const size_t waves = mfma_waves(mc.mt, epi);  // blocks a CU holds by registers
+  MfmaTile T{};
+  mfma_tile(a.N, a.H, a.W, cw, pool, 256, 1, &T);
+  size_t lds = mfma_lds(mc, cw, &T);
+  int G = 4;
+  if (epi != EPI_HEAD && (size_t)T.ntiles * T.ncg < 2 * (size_t)cus) {
+    // 32 pixels a wave where 64 leave CUs without a block
+    MfmaTile T2{};
+    mfma_tile(a.N, a.H, a.W, cw, pool, 128, 1, &T2);
+    const size_t l2 = mfma_lds(mc, cw, &T2);
+    if (l2 <= 160 * 1024) { T = T2; lds = l2; G = 2; }
+  } else {
+    // two or four tiles staged together where that costs no round of blocks
+    // (a tile's staging costs about one and a half times its sums)
+    double best = 0.0;
+    MfmaTile T2{};
+    for (int sub = 1; sub <= 4; sub *= 2) {
+      mfma_tile(a.N, a.H, a.W, cw, pool, 256, sub, &T2);
+      const size_t l2 = mfma_lds(mc, cw, &T2);
+      if (T2.sub != sub || (sub > 1 && l2 > 53 * 1024)) break;
+      const size_t slots = std::max<size_t>(1, std::min<size_t>(waves, 160 * 1024 / l2)) * cus;
+      const double t = (double)(((size_t)T2.ntiles * T2.ncg + slots - 1) / slots) * (sub + 1.5);
+      if (sub == 1 || t < best) { best = t; T = T2; lds = l2; }
+    }
+  }
+  if ((size_t)a.N * T.dhp.d >= 0x7FFFFFFFull) return hipErrorInvalidValue;
+  const MfmaFn fn = T.resident ? mfma_fn<true>(mc.mt, G, epi) : mfma_fn<false>(mc.mt, G, epi);
+  if (!fn) return hipErrorInvalidValue;
   // more than 64 KB of LDS: allowed once per variant and device (bit d of
   // the variant's mask for device d)
-  using Fn = void (*)(const BconvArgs, const int8_t*, const int32_t*, const MfmaTile, uint32_t, uint32_t);
-  static const Fn fns[4] = {k_bconv_mfma<EPI_FOLD, false>, k_bconv_mfma<EPI_FOLD, true>, k_bconv_mfma<EPI_POOL, false>,
-                            k_bconv_mfma<EPI_POOL, true>};
-  static std::atomic<uint64_t> attr[4];
-  const int var = (epi == EPI_POOL ? 2 : 0) + (dump ? 1 : 0);
-  // as many blocks as fit on the chip at once (LDS, and three waves per
-  // SIMD by registers), each walking items blockIdx.x, + gridDim.x, ...
-  int dev = 0, cus = 0;
-  if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+  static std::atomic<uint64_t> attr[2][3][2][4];
+  std::atomic<uint64_t>& at = attr[T.resident][mc.mt >> 1][G >> 2][epi];
   const uint64_t bit = 1ull << (dev & 63);
-  if (!(attr[var].load(std::memory_order_acquire) & bit)) {
-    if (hipError_t e = hipFuncSetAttribute((const void*)fns[var], hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  if (!(at.load(std::memory_order_acquire) & bit)) {
+    if (hipError_t e = hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         e != hipSuccess)
       return e;
-    attr[var].fetch_or(bit, std::memory_order_acq_rel);
+    at.fetch_or(bit, std::memory_order_acq_rel);
   }
-  const size_t per_cu = std::min<size_t>(3, (160 * 1024) / lds);
-  const size_t items = ntiles * (size_t)(a.cout / 64);
-  if (items >= 0xFFFFFFFFull) return hipErrorInvalidValue;
-  // (a multiple of 8 blocks for the XCD-aware item order; blocks without
-  // an item exit)
-  const dim3 grid((unsigned)((std::min<size_t>(items, per_cu * cus) + 7) / 8 * 8));
-  hipLaunchKernelGGL(fns[var], grid, dim3(256), lds, s, a, mc.w, mc.s, T, b0, b1);
+  // as many blocks as fit on the chip at once (LDS, registers), the tiles
+  // spread evenly over them
+  const size_t per_cu = std::max<size_t>(1, std::min<size_t>(waves, (160 * 1024) / lds));
+  const uint32_t t8 = (T.ntiles + 7) / 8;
+  const uint32_t most = std::max<uint32_t>(1, (uint32_t)(per_cu * cus / 8 / T.ncg));
+  const uint32_t rounds = (t8 + most - 1) / most, nts = (t8 + rounds - 1) / rounds;
+  const uint32_t b0 = (uint32_t)(npix * a.cw0 * 4);
+  // (a v3 tensor's pad pixel lies just past its last one)
+  const uint32_t b1 = a.in1 ? (uint32_t)((size_t)a.N * a.h1 * a.w1 * a.cw1 * 4) : 0u;
+  hipLaunchKernelGGL(fn, dim3(8 * (unsigned)T.ncg * nts), dim3(256), lds, s, MfmaParams{a, mc, T, b0, b1});
   return hipGetLastError();
 }
 

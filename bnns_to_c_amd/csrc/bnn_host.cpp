@@ -345,12 +345,10 @@ FoldHost canon_fold(const Act& a, int coutp) {
   return f;
 }
 
-// Which binary convs run on the int8 matrix cores (same results as the
-// popcount kernel either way): by default a fold or pool conv with
-// cout % 64 == 0, an image tile that fits (mfma_conv_fits), rows at least 16
-// wide and 64 or more input channels (use_mfma).  BNN_BCONV_MFMA=0 keeps every conv on the popcount
-// kernel, =2 takes the matrix cores wherever they fit (both read when a
-// model or layer is created).
+// Which binary convs run on the matrix cores (same results as the popcount
+// kernel either way; use_mfma).  BNN_BCONV_MFMA=0 keeps them all on the
+// popcount kernel, =2 takes the matrix cores wherever a tile fits (both read
+// when a model or layer is created).
 int mfma_conv_mode() {
   const char* e = getenv("BNN_BCONV_MFMA");
   if (e && !strcmp(e, "0")) return 0;
@@ -372,7 +370,7 @@ struct DevBconv {
   int cin = 0, cout = 0, cs = 0, cw0 = 0, cw1 = 0;
   uint32_t* wt = nullptr;
   FoldDev f1{}, f2{};
-  MfmaConv mc{};  // int8 matrix-core tables when cout % 64 == 0 (mc.w null otherwise)
+  MfmaConv mc{};  // matrix-core tables (mc.w null: the popcount kernel only)
   int mfma = 0;   // mfma_conv_mode() at creation
   int pair = 0;   // cin <= 16, no concat: wt holds tap pairs, 5 words per channel
   uint32_t* mw = nullptr;  // the fused middle's table [words][channel group][9][64] (mid layers only)
@@ -406,20 +404,31 @@ bool cert_mode() {
   return !(e && !strcmp(e, "0"));
 }
 
-// The int8 matrix-core conv by default where whole forwards measure it
-// faster than the popcount kernel: every fold or pool layer that fits with
-// rows at least 16 pixels wide and at least two input words (a 64-channel
-// K chunk filled).  Config 4 (256 x 256, base 32: thirteen such layers at
-// 128, 64, 32 and 16 wide) 2.34 ms against 2.79 with the popcount kernel
-// everywhere (dec4.c1 116 against 223 us, dec2.c1 130 against 190); the
-// isolated 128 -> 128 pool layer at 32 x 32 (benchmark config 2) 210
-// against 288 us.  A 32-channel input fills half a chunk (config 4's
-// enc2.c1: 61 against 46 us), and at 8 x 8 (the headline's level 2 when its
-// layers run one by one) a tile's staging and epilogue outweigh its one to
-// three chunks (enc3.c1 15 against 8 us, forward 0.342 against 0.320 ms).
-// BNN_BCONV_MFMA=2 takes it wherever it fits.
-bool use_mfma(const DevBconv& L, int epi, int H, int W) {
-  return L.mc.w && mfma_conv_fits(L.cout, H, W, epi) && (L.mfma == 2 || (W >= 16 && L.cw0 + L.cw1 >= 2));
+// Fold and pool layers of full 64-channel groups from 64 or more input
+// channels with rows a power of two at least 16 wide.
+bool wide_layer(const DevBconv& L, int epi, int W) {
+  return L.cout % 64 == 0 && (epi == EPI_FOLD || epi == EPI_POOL) && W >= 16 && (W & (W - 1)) == 0 &&
+         L.cw0 + L.cw1 >= 2;
+}
+// The matrix-core conv by default where it measured faster than the popcount
+// kernel, which starts a launch sooner (about 2 us) but counts a word at a
+// time.  Event times, matrix cores against popcount:
+//  * 256 x 256 tiles, base 32, batch 64: 16-77 against 38-227 us a layer,
+//    every layer (2.4e9 to 1.3e11 bit-MACs);
+//  * 1024 patches of 32 x 32: 48 -> 16 channels (7.2e9) 20.0 against 24.5,
+//    16 -> 16 (2.4e9) 17.9 against 16.8;
+//  * pooled layers from 96 channels, 0.5e9: 7.7-10.6 against 9.2-13.8.
+// Wide layers (wide_layer) have always run there.
+bool use_mfma(const DevBconv& L, int epi, int N, int H, int W) {
+  if (!mfma_conv_fits(L.mc, L.cw0 + L.cw1, N, H, W, epi)) return false;
+  const double macs = 9.0 * N * H * W * L.cin * L.cout;
+  return L.mfma == 2 || wide_layer(L, epi, W) || macs >= 4e9 || (epi == EPI_POOL && L.cin >= 96 && macs >= 3e8);
+}
+// The profiler's name of a matrix-core layer: "_mfma" marks the wide layers,
+// as it always has (under BNN_BCONV_MFMA=2 every fold or pool layer of whole
+// 64-channel groups); the others keep their plain name.
+bool named_mfma(const DevBconv& L, int epi, int W) {
+  return wide_layer(L, epi, W) || (L.mfma == 2 && L.cout % 64 == 0 && (epi == EPI_FOLD || epi == EPI_POOL));
 }
 
 struct Workspace {
@@ -436,6 +445,8 @@ struct BnnDevice {
   int device = 0;
   hipStream_t stream = nullptr;
   std::vector<void*> allocs;
+  uint8_t* chunk = nullptr;  // the rest of the last allocation of tables (dev_upload)
+  size_t chunk_left = 0;
   // the first stage: v1 enc1.conv1 (3x3) or the v2 stem (1x1), real conv + real fold
   bool stem = false;
   int rcin = 0, rcout = 0;
@@ -487,11 +498,23 @@ namespace {
 
 template <class T>
 int dev_upload(BnnDevice* D, T** dst, const T* src, size_t n) {
-  void* p = nullptr;
-  HIP_TRY(hipMalloc(&p, n ? n * sizeof(T) : 4));
-  D->allocs.push_back(p);
+  // tables share allocations of at least kTableChunk bytes, each table on a
+  // 256-byte boundary (a model has some two hundred of them)
+  constexpr size_t kTableChunk = 256u << 10;
+  const size_t b = std::max<size_t>(256, (n * sizeof(T) + 255) & ~(size_t)255);
+  if (b > D->chunk_left) {
+    void* p = nullptr;
+    const size_t c = std::max(b, kTableChunk);
+    HIP_TRY(hipMalloc(&p, c));
+    D->allocs.push_back(p);
+    D->chunk = (uint8_t*)p;
+    D->chunk_left = c;
+  }
+  T* const p = (T*)D->chunk;
+  D->chunk += b;
+  D->chunk_left -= b;
   if (n) HIP_TRY(hipMemcpy(p, src, n * sizeof(T), hipMemcpyHostToDevice));
-  *dst = (T*)p;
+  *dst = p;
   return BNN_OK;
 }
 
@@ -503,6 +526,60 @@ int upload_fold(BnnDevice* D, FoldDev* fd, const Act& a, int coutp) {
   if ((rc = dev_upload(D, &lo, f.lo.data(), f.lo.size()))) return rc;
   if ((rc = dev_upload(D, &wid, f.wid.data(), f.wid.size()))) return rc;
   fd->lo = lo; fd->wid = wid;
+  return BNN_OK;
+}
+
+// the matrix-core conv's operands, border sums and rules
+int upload_mfma(BnnDevice* D, DevBconv* L, const Conv& c, int cs, const Act* a1, const Act* a2) {
+  std::vector<uint32_t> w, slot;
+  std::vector<int32_t> S;
+  mfma_conv_tables(c.packed, c.Cin, c.Cout, cs, L->pair, &w, &S, &slot);
+  const int cp = mfma_coutp(c.Cout), K = 9 * c.Cin;
+  MfmaConv& m = L->mc;
+  std::vector<float> ctr[2], rad[2];
+  std::vector<uint32_t> inv[2];
+  for (int k = 0; k < 2; ++k) {
+    const Act* a = k ? a2 : a1;
+    ctr[k].assign(cp, 0.0f);
+    rad[k].assign(cp, -1.0f);
+    inv[k].assign((cp + 31) / 32, 0u);
+    if (!a) continue;
+    const FoldHost f = canon_fold(*a, cp);
+    for (int co = 0; co < c.Cout; ++co) {
+      bool iv;
+      mfma_rule(f.lo[co], f.wid[co], K, &ctr[k][co], &rad[k][co], &iv);
+      if (iv) inv[k][co / 32] |= 1u << (co % 32);
+    }
+  }
+  std::vector<float> s(S.size());
+  for (size_t i = 0; i < S.size(); ++i) s[i] = -(float)S[i] - ctr[0][i % cp];
+  // one upload: the operands first, the smaller tables after them
+  std::vector<uint32_t> all = w;
+  auto add = [&](const void* src, size_t n) {
+    all.resize((all.size() + 3) & ~(size_t)3);
+    const size_t at = all.size();
+    all.resize(at + n);
+    std::memcpy(all.data() + at, src, n * 4);
+    return at;
+  };
+  std::vector<float> c12(cp);
+  for (int co = 0; co < cp; ++co) c12[co] = ctr[0][co] - ctr[1][co];
+  const size_t o_s = add(s.data(), s.size()), o_c1 = add(ctr[0].data(), cp), o_r1 = add(rad[0].data(), cp),
+               o_c12 = add(c12.data(), cp), o_r2 = add(rad[1].data(), cp), o_i1 = add(inv[0].data(), inv[0].size()),
+               o_i2 = add(inv[1].data(), inv[1].size()), o_sl = add(slot.data(), slot.size());
+  uint32_t* d;
+  int rc;
+  if ((rc = dev_upload(D, &d, all.data(), all.size()))) return rc;
+  m.s = (const float*)(d + o_s);
+  m.c1 = (const float*)(d + o_c1);
+  m.slot = d + o_sl;
+  if (a1) { m.r1 = (const float*)(d + o_r1); m.inv1 = d + o_i1; }
+  if (a1 && a2) { m.c12 = (const float*)(d + o_c12); m.r2 = (const float*)(d + o_r2); m.inv2 = d + o_i2; }
+  m.coutp = cp;
+  m.mt = mfma_mt(c.Cout);
+  m.slots = mfma_nslots(L->cw0, L->cw1, L->pair);
+  m.steps = (m.slots + 3) / 4;
+  m.w = d;
   return BNN_OK;
 }
 
@@ -521,16 +598,7 @@ int upload_bconv(BnnDevice* D, DevBconv* L, const Conv& c, int cs, const Act* a1
   if (a1 && (rc = upload_fold(D, &L->f1, *a1, coutp))) return rc;
   if (a2 && (rc = upload_fold(D, &L->f2, *a2, coutp))) return rc;
   L->mfma = mfma_conv_mode();
-  if (c.Cout % 64 == 0 && L->mfma) {
-    std::vector<int8_t> w8(mfma_w_len(c.Cin, c.Cout, cs));
-    std::vector<int32_t> st(mfma_s_len(c.Cout));
-    mfma_conv_tables(c.packed, c.Cin, c.Cout, cs, w8.data(), st.data());
-    int8_t* dw;
-    int32_t* ds;
-    if ((rc = dev_upload(D, &dw, w8.data(), w8.size()))) return rc;
-    if ((rc = dev_upload(D, &ds, st.data(), st.size()))) return rc;
-    L->mc = MfmaConv{dw, ds, mfma_npair(L->cw0, L->cw1)};
-  }
+  if (L->mfma) return upload_mfma(D, L, c, cs, a1, a2);
   return BNN_OK;
 }
 
@@ -935,9 +1003,14 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
       a.P = dmp->P[pi++];
       if (epi == EPI_POOL) a.P2 = dmp->P2[lvl];
     }
-    const bool mm = use_mfma(L, epi, a.H, a.W);
+    const bool mm = use_mfma(L, epi, cnt, a.H, a.W);
     if (mm) {
-      HIP_TRY(launch_bconv_mfma(a, L.mc, epi, dump, st));
+      if (dump) {
+        // the debug forward's P: the same sums with the integer epilogue
+        HIP_TRY(launch_bconv_mfma(a, L.mc, EPI_P, st));
+        if (epi == EPI_POOL) HIP_TRY(launch_maxpool(a.P, a.P2, cnt * L.cout, a.H, a.W, 2, 2, st));
+      }
+      HIP_TRY(launch_bconv_mfma(a, L.mc, epi, st));
     } else {
       int mt, cog;
       // the shape the whole batch would take: the parts run side by side,
@@ -945,9 +1018,10 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
       pick_shape(epi, N, a.H, a.W, L.cout, &mt, &cog);
       HIP_TRY(launch_bconv(a, epi, mt, cog, dump, st));
     }
-    const char* ot = epi == EPI_POOL ? (mm ? "bconv_pool_mfma" : "bconv_pool")
+    const bool nm = mm && named_mfma(L, epi, a.W);
+    const char* ot = epi == EPI_POOL ? (nm ? "bconv_pool_mfma" : "bconv_pool")
                      : epi == EPI_HEAD ? "bconv_head"
-                                       : (mm ? "bconv_mfma" : "bconv");
+                                       : (nm ? "bconv_mfma" : "bconv");
     return mark(label, ot, (double)N * L.cout * a.H * a.W, (double)L.cin * 9);
   };
 
@@ -2023,6 +2097,10 @@ int bnn_layer_P_device(const BnnConvLayer* L, const uint32_t* d_act, int N, int 
   int rc;
   if ((rc = layer_args(L, d_act, N, H, W, &a))) return rc;
   a.P = d_P;
+  if (use_mfma(L->L, EPI_P, N, H, W)) {
+    HIP_TRY(launch_bconv_mfma(a, L->L.mc, EPI_P, (hipStream_t)stream));
+    return BNN_OK;
+  }
   int mt, cog;
   pick_shape(EPI_P, N, H, W, a.cout, &mt, &cog);
   HIP_TRY(launch_bconv(a, EPI_P, mt, cog, false, (hipStream_t)stream));
@@ -2037,8 +2115,8 @@ int bnn_layer_fold_pool_device(const BnnConvLayer* L, const uint32_t* d_act, int
   if (!L->L.f1.lo || !L->L.f2.lo) return set_err(BNN_EARG, "layer was created without both rules");
   if (H < 2 || W < 2) return set_err(BNN_EARG, "pool needs H, W >= 2");
   a.out = d_skip; a.out2 = d_down;
-  if (use_mfma(L->L, EPI_POOL, H, W)) {
-    HIP_TRY(launch_bconv_mfma(a, L->L.mc, EPI_POOL, false, (hipStream_t)stream));
+  if (use_mfma(L->L, EPI_POOL, N, H, W)) {
+    HIP_TRY(launch_bconv_mfma(a, L->L.mc, EPI_POOL, (hipStream_t)stream));
     return BNN_OK;
   }
   int mt, cog;

@@ -422,49 +422,81 @@ hipError_t launch_conv3_chain(const float* x, const int8_t* wsign, const float* 
 hipError_t launch_bconv(const BconvArgs& a, int epi, int mt, int cog, bool dump,
                         hipStream_t s);
 
-// Binary conv on the int8 matrix cores (v_mfma_i32_16x16x64_i8), for
-// cout % 64 == 0 and the EPI_FOLD / EPI_POOL epilogues.  With activation
-// bits alpha in {0,1} (0 for taps outside the image) and weights w in
-// {-1,+1}, D = sum over valid taps of w*alpha and
+// Binary conv on the matrix cores (FP4 operands, FP32 sums; the kernel's file
+// says how).  With activation bits alpha in {0,1} (0 for taps outside the
+// image) and weights w in {-1,+1}, D = sum over valid taps of w*alpha and
 //   P = sum over valid taps of w*(2*alpha - 1) = 2*D - S,
 // S = sum of w over the valid taps, which depends only on which taps are
 // valid: 16 border classes (row pattern x column pattern, each of: all
-// valid, first invalid, last invalid, both invalid).  K runs over chunks of
-// two activation words (64 channels) of one input segment, a concat's
-// upsampled segment after the first (an odd segment's last chunk has an
-// empty second word); within a chunk over the 9 taps, and within a tap over
-// the two words: pair (chunk * 9 + tap) * 2 + word, 32 channels each.
+// valid, first invalid, last invalid, both invalid).  K runs over slots of 32
+// terms, four to a matrix op: the words in planes of four (a concat's
+// upsampled words after the skip's), within a plane the 9 taps, within a tap
+// the plane's words; a first segment of at most 16 channels (pair) puts six
+// slots of word 0 first instead, tap pairs (row, columns 0 and 1) and single
+// taps (row, column 2) in turn.
 struct MfmaConv {
-  const int8_t* w;      // [coutp][npair][32] int8, +-1, 0 for padded channels and empty words
-  const int32_t* s;     // [16][coutp] S per border class
-  int npair;
+  const uint32_t* w;    // FP4 operands [coutp / (16 mt)][steps][mt][64 lanes][4]
+  const float* s;       // [16][coutp]: -S - c1
+  const float* c1;      // [coutp] rule 1: bit = (|P - c1| < r1) ^ inv1; 0 without a rule
+  const float* r1;      // null without a rule
+  const float* c12;     // rule 2 (null without): c1 - c2, r2, inv2
+  const float* r2;
+  const uint32_t *inv1, *inv2;  // [coutp / 32], bit c % 32 of word c / 32
+  const uint32_t* slot;  // [slots] tap | word << 8
+  int coutp, mt, steps, slots;
 };
-inline int mfma_nchunk(int cw0, int cw1) { return (cw0 + 1) / 2 + (cw1 + 1) / 2; }
-inline int mfma_npair(int cw0, int cw1) { return 18 * mfma_nchunk(cw0, cw1); }
-// kidx sign bits -> the int8 weight table; channel layout as repack_bin
-// (a concat's upsampled channels start at word cw0)
-inline void mfma_conv_tables(const uint64_t* kbits, int cin, int cout, int cs, int8_t* w, int32_t* stab) {
-  const int cw0 = (cs ? cs : cin) / 32 + ((cs ? cs : cin) % 32 != 0);
-  const int cw1 = cs ? (cin - cs + 31) / 32 : 0;
-  const int npair = mfma_npair(cw0, cw1), nc0 = (cw0 + 1) / 2;
-  const int coutp = (cout + 63) / 64 * 64, nw = (cin * 9 + 63) / 64;
-  for (size_t i = 0; i < (size_t)coutp * npair * 32; ++i) w[i] = 0;
-  std::vector<long> T((size_t)coutp * 9, 0);
+inline int mfma_nslots(int cw0, int cw1, int pair) { return 9 * (cw0 + cw1) - (pair ? 3 : 0); }
+// channels of a wave in 16s: as many as fill the group, unless half of a
+// last group of 64 would be padding
+inline int mfma_mt(int cout) { return cout <= 16 ? 1 : cout <= 32 || (cout + 63) / 64 * 64 - cout >= 32 ? 2 : 4; }
+inline int mfma_coutp(int cout) {
+  const int g = 16 * mfma_mt(cout);
+  return (cout + g - 1) / g * g;
+}
+// kidx sign bits -> the operand table and S; channel layout as repack_bin (a
+// concat's upsampled channels start at word cw0)
+inline void mfma_conv_tables(const uint64_t* kbits, int cin, int cout, int cs, bool pair, std::vector<uint32_t>* w,
+                             std::vector<int32_t>* stab, std::vector<uint32_t>* slot) {
+  const int c0 = cs ? cs : cin, cw0 = (c0 + 31) / 32, cw1 = cs ? (cin - cs + 31) / 32 : 0, cw = cw0 + cw1;
+  const int mt = mfma_mt(cout), coutp = mfma_coutp(cout), nw = (cin * 9 + 63) / 64;
+  // slot -> (word, tap, taps in it)
+  struct Slot { int wd, t, n; };
+  std::vector<Slot> sl;
+  if (pair)
+    for (int k = 0; k < 6; ++k) sl.push_back({0, (k >> 1) * 3 + (k & 1) * 2, k & 1 ? 1 : 2});
+  for (int p = 0; p < (cw + 3) / 4; ++p)
+    for (int t = 0; t < 9; ++t)
+      for (int wd = p == 0 && pair ? 1 : 4 * p; wd < cw && wd < 4 * p + 4; ++wd) sl.push_back({wd, t, 1});
+  const int steps = ((int)sl.size() + 3) / 4;
+  slot->clear();
+  for (const Slot& s : sl) slot->push_back((uint32_t)(s.t | s.wd << 8));
+  auto sign = [&](int co, int ci, int t) {
+    const int k = ci * 9 + t;
+    return ((kbits[(size_t)co * nw + (k >> 6)] >> (k & 63)) & 1ull) ? 1 : -1;
+  };
+  // FP4 codes of 4, 2, 1, 4: times the activation nibble's 0.5, 1, 2, 0.5
+  static const uint32_t code[4] = {6, 4, 2, 6};
+  w->assign((size_t)coutp / 16 * steps * 64 * 4, 0u);
   for (int co = 0; co < cout; ++co)
-    for (int ci = 0; ci < cin; ++ci) {
-      int wd, b, c;  // word within its segment, bit, chunk
-      if (!cs || ci < cs) { wd = ci >> 5; b = ci & 31; c = wd >> 1; }
-      else { wd = (ci - cs) >> 5; b = (ci - cs) & 31; c = nc0 + (wd >> 1); }
-      for (int t = 0; t < 9; ++t) {
-        const int k = ci * 9 + t;
-        const int v = ((kbits[(size_t)co * nw + (k >> 6)] >> (k & 63)) & 1ull) ? 1 : -1;
-        const int pr = (c * 9 + t) * 2 + (wd & 1);
-        w[((size_t)co * npair + pr) * 32 + b] = (int8_t)v;
-        T[(size_t)co * 9 + t] += v;
+    for (size_t k = 0; k < sl.size(); ++k) {
+      const int lane = 16 * (int)(k % 4) + co % 16, m = co / 16 % mt;
+      uint32_t* d = w->data() + ((((size_t)(co / (16 * mt)) * steps + k / 4) * mt + m) * 64 + lane) * 4;
+      for (int b = 0; b < 32; ++b) {
+        const Slot& s = sl[k];
+        const int wb = pair && s.wd == 0 ? b % 16 : b, tap = s.t + (pair && s.wd == 0 ? b / 16 : 0);
+        if (pair && s.wd == 0 && b / 16 >= s.n) continue;
+        const int ci = s.wd < cw0 ? s.wd * 32 + wb : c0 + (s.wd - cw0) * 32 + wb;
+        if (s.wd < cw0 ? ci >= c0 : ci >= cin) continue;
+        d[b & 3] |= (code[b & 3] | (sign(co, ci, tap) < 0 ? 8u : 0u)) << (4 * (b >> 2));
       }
     }
+  std::vector<long> T((size_t)coutp * 9, 0);
+  for (int co = 0; co < cout; ++co)
+    for (int ci = 0; ci < cin; ++ci)
+      for (int t = 0; t < 9; ++t) T[(size_t)co * 9 + t] += sign(co, ci, t);
   // valid rows / columns of the 3x3 window for patterns 0..3
   static const int valid[4][3] = {{1, 1, 1}, {0, 1, 1}, {1, 1, 0}, {0, 1, 0}};
+  stab->assign((size_t)16 * coutp, 0);
   for (int rp = 0; rp < 4; ++rp)
     for (int cp = 0; cp < 4; ++cp)
       for (int co = 0; co < coutp; ++co) {
@@ -472,18 +504,37 @@ inline void mfma_conv_tables(const uint64_t* kbits, int cin, int cout, int cs, i
         for (int ky = 0; ky < 3; ++ky)
           for (int kx = 0; kx < 3; ++kx)
             if (valid[rp][ky] && valid[cp][kx]) sum += T[(size_t)co * 9 + ky * 3 + kx];
-        stab[(size_t)(rp * 4 + cp) * coutp + co] = (int32_t)sum;
+        (*stab)[(size_t)(rp * 4 + cp) * coutp + co] = (int32_t)sum;
       }
 }
-inline size_t mfma_w_len(int cin, int cout, int cs) {
-  const int cw0 = ((cs ? cs : cin) + 31) / 32, cw1 = cs ? (cin - cs + 31) / 32 : 0;
-  return (size_t)(cout + 63) / 64 * 64 * mfma_npair(cw0, cw1) * 32;
+// A canonical interval rule over the sums |P| <= K as bit = (|P - c| < r) ^ inv:
+// the interval's part inside [-K, K] is one run (c its middle, r half its
+// length and a half more), nothing (r = -1), or the two ends, which are the
+// complement of the run between them.
+inline void mfma_rule(int32_t lo, uint32_t wid, int K, float* c, float* r, bool* inv) {
+  long run[2][2];
+  int n = 0;
+  for (int k = -1; k <= 1; ++k) {
+    const long u = std::max<long>(-K, (long)lo + k * 4294967296l);
+    const long v = std::min<long>(K, (long)lo + k * 4294967296l + (long)wid - 1);
+    if (u > v) continue;
+    if (n && run[n - 1][1] + 1 == u) run[n - 1][1] = v;
+    else if (n < 2) { run[n][0] = u; run[n][1] = v; ++n; }
+  }
+  long a = 0, b = -2;
+  *inv = n == 2;
+  if (n == 1) { a = run[0][0]; b = run[0][1]; }
+  if (n == 2) { a = run[0][1] + 1; b = run[1][0] - 1; }
+  *c = n ? 0.5f * (float)(a + b) : 0.0f;
+  *r = n ? 0.5f * (float)(b - a) + 0.5f : -1.0f;
 }
-inline size_t mfma_s_len(int cout) { return (size_t)16 * ((cout + 63) / 64 * 64); }
-// Whether launch_bconv_mfma takes a layer of this shape (cout % 64 == 0 and
-// an image narrow enough for its LDS tile).
-bool mfma_conv_fits(int cout, int H, int W, int epi);
-hipError_t launch_bconv_mfma(const BconvArgs& a, const MfmaConv& m, int epi, bool dump, hipStream_t s);
+// Whether launch_bconv_mfma takes a layer of cw input words a pixel (every
+// shape whose tile, operand and tables fit a CU's LDS; the head in one wave's
+// channels; the rules the epilogue needs).
+// compute units of the current device (cached per device)
+int device_cus();
+bool mfma_conv_fits(const MfmaConv& mc, int cw, int N, int H, int W, int epi);
+hipError_t launch_bconv_mfma(const BconvArgs& a, const MfmaConv& m, int epi, hipStream_t s);
 hipError_t launch_real(const RealArgs& a, hipStream_t s);
 
 // Simple kernels behind the reference's batch-1 kernel ABI.

@@ -1,4 +1,4 @@
-"""The binary 3x3 conv on the int8 matrix cores (bnn_bconv_mfma.hip).
+"""The binary 3x3 conv on the matrix cores (bnn_bconv_mfma.hip).
 
 The kernel computes the same P as csrc/bnn_conv.c:23-36 (P = 2*D - S with
 D the int8 product of 0/1 activation bytes and +-1 weights, S the weight sum
@@ -124,3 +124,70 @@ def test_layer_fold_pool_matches_popcount(monkeypatch, N, H, W, c):
         L.close()
     assert np.array_equal(outs["0"][0], outs["2"][0])
     assert np.array_equal(outs["0"][1], outs["2"][1])
+
+
+def _act(torch, seed, N, H, W, c):
+    """Random packed bits, the unused high bits of the last word 0."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    a = torch.randint(-2**31, 2**31, (N, H, W, (c + 31) // 32), generator=g, device="cuda", dtype=torch.int64)
+    a = a.to(torch.int32)
+    if c % 32:
+        a[..., -1] &= (1 << c % 32) - 1
+    return a
+
+
+# tiles of whole patches (1 to 64 of them, a partial last one), of whole rows
+# (odd widths and heights, an even split), of columns (67, 130 wide); one to
+# four tiles staged together; paired taps (16 and fewer channels); 1 to 12
+# input words, planes of four with a remainder; channel groups of 16, 32 and
+# 64 with a partial last one; weights kept in LDS and streamed through it
+SHAPES = [(700, 2, 2, 256, 256), (9, 5, 3, 40, 24), (37, 4, 4, 384, 128), (3, 13, 9, 40, 96), (2, 33, 47, 8, 16),
+          (5, 45, 51, 24, 24), (2, 64, 67, 96, 48), (1, 31, 130, 72, 160), (1100, 32, 32, 16, 16),
+          (70, 64, 64, 32, 32), (1, 7, 200, 200, 72), (400, 8, 8, 64, 64), (1, 1, 1, 33, 7), (3, 3, 64, 129, 65)]
+
+
+@pytest.mark.parametrize("N,H,W,cin,cout", SHAPES)
+def test_layer_shapes_match_popcount(monkeypatch, N, H, W, cin, cout):
+    """P, skip bits and pooled bits of an isolated layer: the matrix cores
+    against the popcount kernel, every rule type, bit for bit."""
+    import torch
+    act = _act(torch, 50 + cin, N, H, W, cin)
+    w = B.pack_kidx(synth.make_signs(51, cout, cin))
+    r1 = synth.make_rules(52, cout, cin * 9, coverage=True)
+    r2 = synth.make_rules(53, cout, cin * 9, coverage=True)
+    cwo = (cout + 31) // 32
+    outs = {}
+    for mode in ("0", "2"):
+        monkeypatch.setenv("BNN_BCONV_MFMA", mode)
+        L = E.ConvLayer(w, cin, cout, r1, r2)
+        P = torch.full((N, cout, H, W), -7, dtype=torch.int32, device="cuda")
+        L.P_device(act.data_ptr(), N, H, W, P.data_ptr(), None)
+        got = [P]
+        if H >= 2 and W >= 2:
+            skip = torch.full((N, H, W, cwo), -1, dtype=torch.int32, device="cuda")
+            down = torch.full((N, H // 2, W // 2, cwo), -1, dtype=torch.int32, device="cuda")
+            only = torch.full((N, H // 2, W // 2, cwo), -1, dtype=torch.int32, device="cuda")
+            L.fold_pool_device(act.data_ptr(), N, H, W, skip.data_ptr(), down.data_ptr(), None)
+            L.fold_pool_device(act.data_ptr(), N, H, W, None, only.data_ptr(), None)
+            got += [skip, down, only]
+        torch.cuda.synchronize()
+        outs[mode] = [t.cpu().numpy() for t in got]
+        L.close()
+    for a, b in zip(outs["0"], outs["2"]):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("base,N,H,W", [(8, 3, 35, 41), (16, 2, 32, 32), (24, 2, 45, 51), (20, 1, 70, 83)])
+def test_forced_forward_vs_checker(tmp_path, orc, monkeypatch, base, N, H, W):
+    """Whole forwards with every layer on the matrix cores (the concat layers
+    with an upsample that leaves odd edges uncovered, the head): every stage
+    against the checker."""
+    monkeypatch.setenv("BNN_BCONV_MFMA", "2")
+    monkeypatch.setenv("BNN_MID", "0")
+    b = synth.make_blob(seed=60 + base, base=base, coverage=True)
+    p = tmp_path / "m.blob"
+    p.write_bytes(B.to_bytes(b))
+    eng = E.Engine(str(p))
+    _check_stages(eng, orc.parse(B.to_bytes(b)), synth.make_input(160, N, 120, H, W))
+    eng.close()
