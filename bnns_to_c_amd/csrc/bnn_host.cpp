@@ -61,17 +61,28 @@ std::vector<uint32_t> repack_bin(const uint64_t* kbits, int cin, int cout, int t
   const int cw0 = words(cs ? cs : cin), cw1 = cs ? words(cin - cs) : 0;
   const int coutp = pad32(cout);
   std::vector<uint32_t> wt((size_t)(cw0 + cw1) * coutp * taps, 0u);
-  for (int co = 0; co < cout; ++co)
-    for (int ci = 0; ci < cin; ++ci) {
-      int w, b;
-      if (!cs || ci < cs) { w = ci >> 5; b = ci & 31; }
-      else { w = cw0 + ((ci - cs) >> 5); b = (ci - cs) & 31; }
-      for (int t = 0; t < taps; ++t) {
-        const int k = ci * taps + t;
-        if ((kbits[(size_t)co * nw + (k >> 6)] >> (k & 63)) & 1ull)
-          wt[((size_t)w * coutp + co) * taps + t] |= 1u << b;
+  // where bit k of a channel's words goes: offset from the channel's first word, bit
+  std::vector<uint32_t> off((size_t)cin * taps), bit((size_t)cin * taps);
+  for (int ci = 0; ci < cin; ++ci) {
+    int w, b;
+    if (!cs || ci < cs) { w = ci >> 5; b = ci & 31; }
+    else { w = cw0 + ((ci - cs) >> 5); b = (ci - cs) & 31; }
+    for (int t = 0; t < taps; ++t) {
+      off[(size_t)ci * taps + t] = (uint32_t)(w * coutp * taps + t);
+      bit[(size_t)ci * taps + t] = 1u << b;
+    }
+  }
+  for (int co = 0; co < cout; ++co) {
+    uint32_t* const row = wt.data() + (size_t)co * taps;
+    for (int i = 0; i < nw; ++i) {
+      uint64_t v = kbits[(size_t)co * nw + i];
+      if (i == nw - 1 && cin * taps % 64) v &= (1ull << (cin * taps % 64)) - 1;
+      for (; v; v &= v - 1) {
+        const int k = i * 64 + __builtin_ctzll(v);
+        row[off[k]] |= bit[k];
       }
     }
+  }
   return wt;
 }
 
@@ -369,6 +380,7 @@ constexpr int kMidExtMin = 256;
 struct DevBconv {
   int cin = 0, cout = 0, cs = 0, cw0 = 0, cw1 = 0;
   uint32_t* wt = nullptr;
+  std::vector<uint32_t> words;  // repack_bin's table, while a model is built
   FoldDev f1{}, f2{};
   MfmaConv mc{};  // matrix-core tables (mc.w null: the popcount kernel only)
   int mfma = 0;   // mfma_conv_mode() at creation
@@ -392,6 +404,15 @@ bool mid_mode() {
 // them as per-layer kernels.
 bool midx_mode() {
   const char* e = getenv("BNN_MIDX");
+  return !(e && !strcmp(e, "0"));
+}
+
+// For 32x32 patches every binary layer runs in one kernel (launch_tail) where
+// the fused middle and its level-1 layers would and the widths fit
+// (tail_fits); BNN_TAIL=0, like BNN_MIDX=0, BNN_MID=0 and BNN_BCONV_MFMA=0,
+// keeps the layers apart.
+bool tail_mode() {
+  const char* e = getenv("BNN_TAIL");
   return !(e && !strcmp(e, "0"));
 }
 
@@ -464,6 +485,12 @@ struct BnnDevice {
   DevBconv e1[4], e2[4], b1, b2, d1[4], d2[4];
   bool mid = false;  // the fused middle applies (mid_fits at load, and mid_mode())
   bool midx = false; // and takes the level-1 layers too (mid_ext_fits, midx_mode())
+  // every binary layer of a 32x32 patch as one kernel (tail_fits at load,
+  // mid_mode(), midx_mode(), the matrix cores on): its layers with their LDS
+  // places for 1 and 2 patches a block
+  bool tail = false;
+  TailArgs ta[2];
+  float* hl = nullptr;  // its head's sums over the first eight channels, by sign pattern
   float *hw = nullptr, *hb = nullptr;
   int ncls = 0;
   Workspace ws;
@@ -530,11 +557,14 @@ int upload_fold(BnnDevice* D, FoldDev* fd, const Act& a, int coutp) {
 }
 
 // the matrix-core conv's operands, border sums and rules
-int upload_mfma(BnnDevice* D, DevBconv* L, const Conv& c, int cs, const Act* a1, const Act* a2) {
+int upload_mfma(BnnDevice* D, DevBconv* L, const Conv& c, int cs, const Act* a1, const Act* a2,
+                const std::vector<uint32_t>& wt) {
+  const BinWords bw{wt.data(), c.Cin, c.Cout, cs, L->cw0, L->cw1, pad32(c.Cout)};
   std::vector<uint32_t> w, slot;
   std::vector<int32_t> S;
-  mfma_conv_tables(c.packed, c.Cin, c.Cout, cs, L->pair, &w, &S, &slot);
   const int cp = mfma_coutp(c.Cout), K = 9 * c.Cin;
+  mfma_conv_tables(bw, L->pair, &w, &slot);
+  mfma_border_sums(bw, cp, &S);
   MfmaConv& m = L->mc;
   std::vector<float> ctr[2], rad[2];
   std::vector<uint32_t> inv[2];
@@ -589,16 +619,17 @@ int upload_bconv(BnnDevice* D, DevBconv* L, const Conv& c, int cs, const Act* a1
   L->cw1 = cs ? words(c.Cin - cs) : 0;
   std::vector<uint32_t> wt = repack_bin(c.packed, c.Cin, c.Cout, 9, cs);
   L->pair = (cs ? cs : c.Cin) <= 16;
-  if (L->pair) wt = pair_taps(wt, c.Cout);
+  L->mfma = mfma_conv_mode();
   int rc;
+  if (L->mfma && (rc = upload_mfma(D, L, c, cs, a1, a2, wt))) return rc;
+  L->words = wt;
+  if (L->pair) wt = pair_taps(wt, c.Cout);
   if ((rc = dev_upload(D, &L->wt, wt.data(), wt.size()))) return rc;
   // rules padded to 64 channels (width 0 past cout): the fused middle reads
   // one per lane of a 64-channel group
   const int coutp = (c.Cout + 63) & ~63;
   if (a1 && (rc = upload_fold(D, &L->f1, *a1, coutp))) return rc;
   if (a2 && (rc = upload_fold(D, &L->f2, *a2, coutp))) return rc;
-  L->mfma = mfma_conv_mode();
-  if (L->mfma) return upload_mfma(D, L, c, cs, a1, a2);
   return BNN_OK;
 }
 
@@ -607,7 +638,7 @@ int upload_bconv(BnnDevice* D, DevBconv* L, const Conv& c, int cs, const Act* a1
 // of a group read consecutive words for one tap and the taps lie at fixed
 // distances
 int upload_mid_w(BnnDevice* D, DevBconv* L, const Conv& c, int cs) {
-  const std::vector<uint32_t> wt = repack_bin(c.packed, c.Cin, c.Cout, 9, cs);
+  const std::vector<uint32_t>& wt = L->words;
   const int nwd = L->cw0 + L->cw1, cp32 = pad32(c.Cout), ncg = (c.Cout + 63) / 64;
   std::vector<uint32_t> mw((size_t)nwd * ncg * 9 * 64, 0u);
   for (int w = 0; w < nwd; ++w)
@@ -647,6 +678,174 @@ bool mid_ext_fits(BnnDevice* D) {
   return D->e1[1].cw0 == words(D->e2[0].cout) && D->e2[1].cw0 == words(D->e1[1].cout) &&
          D->d1[2].cw0 == words(D->e2[1].cout) && D->d1[2].cw1 == words(D->d2[1].cout) &&
          D->d2[2].cw0 == words(D->d1[2].cout);
+}
+
+// Whether the whole-patch kernel takes this model: at most 16, 32, 64, 128,
+// 256 channels at the five levels (a stem too), concats as the topology has
+// them, a head over the last layer.
+bool tail_fits(const Model* m, const BnnDevice* D) {
+  for (int i = 0; i < 4; ++i) {
+    const int c = 16 << i;
+    if ((i || D->stem) && D->e1[i].cout > c) return false;
+    if (D->e2[i].cout > c || D->d1[3 - i].cout > c || D->d2[3 - i].cout > c) return false;
+    if (D->d1[3 - i].cs != D->e2[i].cout) return false;
+    if (D->d1[3 - i].cin - D->d1[3 - i].cs != (i < 3 ? D->d2[2 - i].cout : D->b2.cout)) return false;
+  }
+  return D->rcout <= 16 && D->b1.cout <= 256 && D->b2.cout <= 256 && m->head_Cin == D->d2[3].cout;
+}
+
+// the whole-patch kernel's tables
+int upload_tail(const Model* m, BnnDevice* D) {
+  struct Spec {
+    const DevBconv* L;
+    const Conv* c;
+    const Act *a1, *a2;
+    int lvl, kind;
+    int in;        // LDS tensor read (a concat: its skip), words, of them the skip's
+    int wds, cw0;
+    bool pair;     // the first word is a pair word
+    int out, down;
+  };
+  // LDS tensors [level, words]; a concat's upsampled planes follow its skip's
+  enum { ACT, ACT2, SK1, UP1, D1, H2, SK2, UP2, D2, H3, SK3, UP3, D3, H4, SK4, UP4, D4, B1, NT };
+  static const int tl[NT] = {0, 0, 0, 0, 1, 1, 1, 1, 2, 2, 2, 2, 3, 3, 3, 3, 4, 4};
+  const int tw[NT] = {1, D->stem ? 1 : 0, 1, 1, 1, 1, 1, 2, 1, 2, 2, 4, 2, 4, 4, 8, 4, 8};
+  std::vector<Spec> sp;
+  if (D->stem)
+    sp.push_back({&D->e1[0], &m->enc_conv1[0], &m->enc_act1[0], nullptr, 0, TAIL_FOLD, ACT, 1, 1, true, ACT2, -1});
+  const int H[4] = {ACT, H2, H3, H4}, SK[4] = {SK1, SK2, SK3, SK4}, UP[4] = {UP1, UP2, UP3, UP4}, DN[4] = {D1, D2, D3, D4};
+  for (int i = 0; i < 4; ++i) {
+    const int w = 1 << std::max(0, i - 1);  // words of the level's tensors: 1, 1, 2, 4
+    if (i)
+      sp.push_back({&D->e1[i], &m->enc_conv1[i], &m->enc_act1[i], nullptr, i, TAIL_FOLD, DN[i - 1], i < 3 ? 1 : 2,
+                    i < 3 ? 1 : 2, i == 1, H[i], -1});
+    sp.push_back({&D->e2[i], &m->enc_conv2[i], &m->enc_act2_skip[i], &m->enc_act2_down[i], i, TAIL_POOL,
+                  i ? H[i] : (D->stem ? ACT2 : ACT), w, w, i == 0, SK[i], DN[i]});
+  }
+  sp.push_back({&D->b1, &m->bott_conv1, &m->bott_act1, nullptr, 4, TAIL_FOLD, D4, 4, 4, false, B1, -1});
+  sp.push_back({&D->b2, &m->bott_conv2, &m->bott_act2, nullptr, 4, TAIL_UP, B1, 8, 8, false, UP4, -1});
+  for (int i = 0; i < 4; ++i) {
+    const int lv = 3 - i, w = 1 << std::max(0, lv - 1);
+    sp.push_back({&D->d1[i], &m->dec_conv1[i], &m->dec_act1[i], nullptr, lv, TAIL_FOLD, SK[lv], w + (lv ? 2 * w : 1), w,
+                  lv == 0, H[lv], -1});
+    sp.push_back({&D->d2[i], &m->dec_conv2[i], &m->dec_act2[i], nullptr, lv, i < 3 ? TAIL_UP : TAIL_HEAD, H[lv], w, w,
+                  lv == 0, i < 3 ? UP[lv - 1] : -1, -1});
+  }
+  // K slots: (word, tap, taps in the word), wd < 0 past the last
+  struct Slot { int wd, t, n; };
+  auto slots_of = [](const Spec& s) {
+    std::vector<Slot> v;
+    const Slot none{-1, 0, 0};
+    int t1 = 0;  // taps of word 1 taken by the pair's free slot
+    if (s.pair) {
+      for (int r = 0; r < 3; ++r) v.push_back({0, 3 * r, 2});
+      v.push_back(s.wds > 1 ? Slot{1, t1++, 1} : none);
+      for (int r = 0; r < 3; ++r) v.push_back({0, 3 * r + 2, 1});
+      v.push_back(none);
+      for (int wd = 1; wd < s.wds; ++wd)
+        for (int t = wd == 1 ? t1 : 0; t < 9; ++t) v.push_back({wd, t, 1});
+    } else {
+      for (int p = 0; p < s.wds; p += 4)
+        for (int t = 0; t < 9; ++t)
+          for (int wd = p; wd < s.wds && wd < p + 4; ++wd) v.push_back({wd, t, 1});
+    }
+    while (v.size() % 4) v.push_back(none);
+    return v;
+  };
+  std::vector<int> tab[2];
+  TailArgs base{};
+  base.nlayers = (int)sp.size();
+  std::vector<TailLayer> lay;
+  for (const Spec& s : sp) {
+    const Conv& c = *s.c;
+    const int cs = s.L->cs, C = 16 << s.lvl, nct = C / 16;
+    const std::vector<Slot> sl = slots_of(s);
+    const int steps = (int)sl.size() / 4;
+    const BinWords bw{s.L->words.data(), c.Cin, c.Cout, cs, s.L->cw0, s.L->cw1, pad32(c.Cout)};
+    std::vector<uint32_t> w((size_t)nct * steps * 64, 0u);
+    for (size_t k = 0; k < sl.size(); ++k) {
+      // the model's word: the skip's and the upsampled words may be fewer than the level's
+      const Slot& x = sl[k];
+      if (x.wd < 0 || (x.wd < s.cw0 ? x.wd >= bw.cw0 : x.wd - s.cw0 >= bw.cw1)) continue;
+      const int wd = x.wd < s.cw0 ? x.wd : bw.cw0 + x.wd - s.cw0;
+      for (int co = 0; co < c.Cout; ++co) {
+        uint32_t v = bw.neg(wd, co, x.t);  // FP4's sign bit: set for a weight of -1
+        if (x.n == 2) v |= bw.neg(wd, co, x.t + 1) << 16;
+        w[((size_t)(co / 16) * steps + k / 4) * 64 + 16 * (k % 4) + co % 16] = v;
+      }
+    }
+    // border sums and rules, padded to the level's channels
+    std::vector<int32_t> S;
+    mfma_border_sums(bw, C, &S);
+    const int ni = std::max(1, C / 32);
+    std::vector<float> tb((size_t)19 * C + 2 * ni, 0.0f);
+    std::vector<uint32_t> inv(2 * ni, 0u);
+    const FoldHost f1 = canon_fold(*s.a1, C);
+    FoldHost f2;
+    if (s.a2) f2 = canon_fold(*s.a2, C);
+    for (int co = 0; co < C; ++co) {
+      float c1 = 0.0f, r1 = -1.0f, c2 = 0.0f, r2 = -1.0f;
+      bool i1 = false, i2 = false;
+      if (co < c.Cout) {
+        mfma_rule(f1.lo[co], f1.wid[co], 9 * c.Cin, &c1, &r1, &i1);
+        if (s.a2) mfma_rule(f2.lo[co], f2.wid[co], 9 * c.Cin, &c2, &r2, &i2);
+      }
+      for (int k = 0; k < 16; ++k) tb[(size_t)k * C + co] = (co < c.Cout ? -(float)S[(size_t)k * C + co] : 0.0f) - c1;
+      tb[(size_t)16 * C + co] = r1;
+      tb[(size_t)17 * C + co] = c1 - c2;
+      tb[(size_t)18 * C + co] = r2;
+      if (i1) inv[co / 32] |= 1u << (co % 32);
+      if (i2) inv[ni + co / 32] |= 1u << (co % 32);
+    }
+    std::memcpy(&tb[(size_t)19 * C], inv.data(), inv.size() * 4);
+    TailLayer t{};
+    uint32_t* dw;
+    float* dt;
+    int rc;
+    if ((rc = dev_upload(D, &dw, w.data(), w.size()))) return rc;
+    if ((rc = dev_upload(D, &dt, tb.data(), tb.size()))) return rc;
+    t.w = dw; t.tabs = dt;
+    t.lvl = s.lvl; t.kind = s.kind; t.steps = steps;
+    t.slot = (int)tab[0].size() / 4;
+    lay.push_back(t);
+    for (int v = 0; v < 2; ++v) {
+      const int np = 1 << v, d = 32 >> s.lvl, p = d + 2;
+      int off[NT], o = 0;
+      for (int i = 0; i < NT; ++i) { off[i] = o * 4; o += tw[i] * tail_plane(np, tl[i]); }
+      for (const Slot& x : sl)
+        tab[v].push_back(x.wd < 0 ? INT32_MIN
+                                  : off[s.in] + (x.wd * tail_plane(np, s.lvl) + x.t / 3 * p + x.t % 3) * 4);
+      TailLayer& q = D->ta[v].L[lay.size() - 1];
+      q = t;
+      q.out = s.out >= 0 ? off[s.out] : 0;
+      q.down = s.down >= 0 ? off[s.down] : 0;
+      q.opair = s.out == ACT || s.out == ACT2 || s.out == SK1;
+      q.dpair = s.down == D1;
+      D->ta[v].off_in = off[ACT];
+      D->ta[v].off_tab = (o + 3) / 4 * 16;
+      D->ta[v].lds_words = (o + 3) / 4 * 4;
+      D->ta[v].nlayers = (int)sp.size();
+    }
+  }
+  // the head's first eight steps (bias, then fused steps in order) for each of
+  // their 256 bit patterns
+  std::vector<float> hl((size_t)m->head_Cout * 256);
+  for (int t = 0; t < m->head_Cout; ++t)
+    for (int o = 0; o < 256; ++o) {
+      float a = m->head_bias[t];
+      for (int c = 0; c < 8 && c < m->head_Cin; ++c)
+        a = std::fma(m->head_W[(size_t)t * m->head_Cin + c], (o >> c) & 1 ? 1.0f : -1.0f, a);
+      hl[(size_t)t * 256 + o] = a;
+    }
+  if (int rc = dev_upload(D, &D->hl, hl.data(), hl.size())) return rc;
+  for (int v = 0; v < 2; ++v) {
+    int* d;
+    int rc;
+    if ((rc = dev_upload(D, &d, tab[v].data(), tab[v].size()))) return rc;
+    D->ta[v].slots = d;
+    D->ta[v].nslot = (int)tab[v].size();
+  }
+  return BNN_OK;
 }
 
 // real conv weights.  v2 stem: lane masks of the 1x1 matrix-core kernel
@@ -802,9 +1001,14 @@ int build_device(Model* m, const StemPart* st = nullptr) {
     for (int l = 0; l < kMidLayers; ++l)
       if ((rc = upload_mid_w(D, L[l], *cv[l], L[l]->cs))) return rc;
   }
+  D->tail = D->midx && D->e2[0].mfma && tail_mode() && tail_fits(m, D);
+  if (D->tail && (rc = upload_tail(m, D))) return rc;
   D->ncls = m->head_Cout;
   if ((rc = dev_upload(D, &D->hw, m->head_W, (size_t)m->head_Cout * m->head_Cin))) return rc;
   if ((rc = dev_upload(D, &D->hb, m->head_bias, (size_t)m->head_Cout))) return rc;
+  for (DevBconv* L : {&D->b1, &D->b2}) L->words = {};
+  for (int i = 0; i < 4; ++i)
+    for (DevBconv* L : {&D->e1[i], &D->e2[i], &D->d1[i], &D->d2[i]}) L->words = {};
   HIP_TRY(hipDeviceSynchronize());
   return BNN_OK;
 }
@@ -1116,10 +1320,25 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
   static const char* enc_c2[4] = {"enc1.c2", "enc2.c2", "enc3.c2", "enc4.c2"};
   static const char* dec_c1[4] = {"dec4.c1", "dec3.c1", "dec2.c1", "dec1.c1"};
   static const char* dec_c2[4] = {"dec4.c2", "dec3.c2", "dec2.c2", "dec1.c2"};
+  // every binary layer of a 32x32 patch as one kernel; with per-kernel events
+  // (one kernel has no time per layer) or debug dumps the layers run apart
+  const bool use_tail = D->tail && H == 32 && W == 32 && !evs && !dump;
+  auto tail = [&]() -> int {
+    const int np = tail_np(cnt);
+    TailArgs a = D->ta[np - 1];
+    a.in = at(w.a1, 0, 1);
+    a.N = cnt;
+    a.hw = D->hw; a.hl = D->hl; a.ncls = D->ncls; a.hc = m->head_Cin;
+    a.logits = sc ? d_logits : d_logits + (size_t)nb * D->ncls * H * W;
+    if (sc) { a.sH = sc->sH; a.sW = sc->sW; a.pcols = sc->pcols; a.prow0 = sc->prow0 + nb / sc->pcols; }
+    HIP_TRY(launch_tail(a, np, st));
+    return BNN_OK;
+  };
   int stage = 3;  // what part() enqueues: 1 the first conv, 2 the binary layers
   auto part = [&]() -> int {
   if ((stage & 1) && (rc = first_conv())) return rc;
   if (!(stage & 2)) return BNN_OK;
+  if (use_tail) return tail();
   const uint32_t* x = w.a1;
   for (int i = 0; i < (use_ext ? 1 : use_mid ? 2 : 4); ++i) {
     const uint32_t* hin = x;
@@ -1183,9 +1402,11 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
   // stream instead, the wait for it at the end and for the caller's stream
   // at the start left the GPU idle for 17 us a forward at batch 1024).  A
   // scene splits at whole patch rows.  One stream with per-kernel events or
-  // debug dumps.
+  // debug dumps, and where one kernel runs the binary layers: its blocks' time
+  // is the same for half the patches (batch 1024: 238.7 us against 289 as two
+  // parts; the scene 203 against 215).
   int parts = 1;
-  if (!dump && !evs)
+  if (!dump && !evs && !use_tail)
     while (parts < std::min(kSplitMax, max_parts) && N >= kSplitMin * parts * 2) parts *= 2;
   // a scene splits at whole patch rows (its patches are numbered row by row)
   const int unit = sc ? sc->pcols : 1;

@@ -453,12 +453,42 @@ inline int mfma_coutp(int cout) {
   const int g = 16 * mfma_mt(cout);
   return (cout + g - 1) / g * g;
 }
-// kidx sign bits -> the operand table and S; channel layout as repack_bin (a
-// concat's upsampled channels start at word cw0)
-inline void mfma_conv_tables(const uint64_t* kbits, int cin, int cout, int cs, bool pair, std::vector<uint32_t>* w,
-                             std::vector<int32_t>* stab, std::vector<uint32_t>* slot) {
-  const int c0 = cs ? cs : cin, cw0 = (c0 + 31) / 32, cw1 = cs ? (cin - cs + 31) / 32 : 0, cw = cw0 + cw1;
-  const int mt = mfma_mt(cout), coutp = mfma_coutp(cout), nw = (cin * 9 + 63) / 64;
+// The weights of a layer as the popcount kernel's table has them: +1 bits,
+// word w of channel co at tap t at ((w * coutp) + co) * 9 + t (coutp: cout
+// rounded up to 32; a concat's upsampled channels start at word cw0).
+struct BinWords {
+  const uint32_t* wt;
+  int cin, cout, cs, cw0, cw1, coutp;
+  uint32_t valid(int w) const {  // the channels a word holds
+    const int c0 = cs ? cs : cin, n = w < cw0 ? c0 - 32 * w : cin - c0 - 32 * (w - cw0);
+    return n <= 0 ? 0u : n >= 32 ? ~0u : (1u << n) - 1u;
+  }
+  uint32_t neg(int w, int co, int t) const { return ~wt[((size_t)w * coutp + co) * 9 + t] & valid(w); }
+};
+// S per border class, [16][coutp of the caller], 0 past cout
+inline void mfma_border_sums(const BinWords& b, int coutp, std::vector<int32_t>* stab) {
+  stab->assign((size_t)16 * coutp, 0);
+  // valid rows / columns of the 3x3 window for patterns 0..3
+  static const int valid[4][3] = {{1, 1, 1}, {0, 1, 1}, {1, 1, 0}, {0, 1, 0}};
+  for (int co = 0; co < b.cout; ++co) {
+    int T[9];
+    for (int t = 0; t < 9; ++t) {
+      int neg = 0;
+      for (int w = 0; w < b.cw0 + b.cw1; ++w) neg += __builtin_popcount(b.neg(w, co, t));
+      T[t] = b.cin - 2 * neg;
+    }
+    for (int rp = 0; rp < 4; ++rp)
+      for (int cp = 0; cp < 4; ++cp) {
+        int sum = 0;
+        for (int t = 0; t < 9; ++t)
+          if (valid[rp][t / 3] && valid[cp][t % 3]) sum += T[t];
+        (*stab)[(size_t)(rp * 4 + cp) * coutp + co] = sum;
+      }
+  }
+}
+// the operand table and the slots (tap | word << 8)
+inline void mfma_conv_tables(const BinWords& b, bool pair, std::vector<uint32_t>* w, std::vector<uint32_t>* slot) {
+  const int cw = b.cw0 + b.cw1, mt = mfma_mt(b.cout), coutp = mfma_coutp(b.cout);
   // slot -> (word, tap, taps in it)
   struct Slot { int wd, t, n; };
   std::vector<Slot> sl;
@@ -470,42 +500,19 @@ inline void mfma_conv_tables(const uint64_t* kbits, int cin, int cout, int cs, b
   const int steps = ((int)sl.size() + 3) / 4;
   slot->clear();
   for (const Slot& s : sl) slot->push_back((uint32_t)(s.t | s.wd << 8));
-  auto sign = [&](int co, int ci, int t) {
-    const int k = ci * 9 + t;
-    return ((kbits[(size_t)co * nw + (k >> 6)] >> (k & 63)) & 1ull) ? 1 : -1;
-  };
   // FP4 codes of 4, 2, 1, 4: times the activation nibble's 0.5, 1, 2, 0.5
   static const uint32_t code[4] = {6, 4, 2, 6};
   w->assign((size_t)coutp / 16 * steps * 64 * 4, 0u);
-  for (int co = 0; co < cout; ++co)
+  for (int co = 0; co < b.cout; ++co)
     for (size_t k = 0; k < sl.size(); ++k) {
+      const Slot& s = sl[k];
+      const bool two = pair && s.wd == 0 && s.n == 2;
+      uint32_t v = b.valid(s.wd), g = b.neg(s.wd, co, s.t);
+      if (two) { v |= v << 16; g |= b.neg(s.wd, co, s.t + 1) << 16; }
       const int lane = 16 * (int)(k % 4) + co % 16, m = co / 16 % mt;
       uint32_t* d = w->data() + ((((size_t)(co / (16 * mt)) * steps + k / 4) * mt + m) * 64 + lane) * 4;
-      for (int b = 0; b < 32; ++b) {
-        const Slot& s = sl[k];
-        const int wb = pair && s.wd == 0 ? b % 16 : b, tap = s.t + (pair && s.wd == 0 ? b / 16 : 0);
-        if (pair && s.wd == 0 && b / 16 >= s.n) continue;
-        const int ci = s.wd < cw0 ? s.wd * 32 + wb : c0 + (s.wd - cw0) * 32 + wb;
-        if (s.wd < cw0 ? ci >= c0 : ci >= cin) continue;
-        d[b & 3] |= (code[b & 3] | (sign(co, ci, tap) < 0 ? 8u : 0u)) << (4 * (b >> 2));
-      }
+      for (int j = 0; j < 4; ++j) d[j] = ((v >> j) & 0x11111111u) * code[j] | ((g >> j) & 0x11111111u) << 3;
     }
-  std::vector<long> T((size_t)coutp * 9, 0);
-  for (int co = 0; co < cout; ++co)
-    for (int ci = 0; ci < cin; ++ci)
-      for (int t = 0; t < 9; ++t) T[(size_t)co * 9 + t] += sign(co, ci, t);
-  // valid rows / columns of the 3x3 window for patterns 0..3
-  static const int valid[4][3] = {{1, 1, 1}, {0, 1, 1}, {1, 1, 0}, {0, 1, 0}};
-  stab->assign((size_t)16 * coutp, 0);
-  for (int rp = 0; rp < 4; ++rp)
-    for (int cp = 0; cp < 4; ++cp)
-      for (int co = 0; co < coutp; ++co) {
-        long sum = 0;
-        for (int ky = 0; ky < 3; ++ky)
-          for (int kx = 0; kx < 3; ++kx)
-            if (valid[rp][ky] && valid[cp][kx]) sum += T[(size_t)co * 9 + ky * 3 + kx];
-        (*stab)[(size_t)(rp * 4 + cp) * coutp + co] = (int32_t)sum;
-      }
 }
 // A canonical interval rule over the sums |P| <= K as bit = (|P - c| < r) ^ inv:
 // the interval's part inside [-K, K] is one run (c its middle, r half its
@@ -611,6 +618,37 @@ struct MidArgs {
   int xoff[kMidXTensors], xcw[kMidXTensors];
 };
 hipError_t launch_mid(const MidArgs& a, bool dump, hipStream_t s);
+
+// Every binary layer of 32x32 patches in one kernel (bnn_tail.hip), for models
+// of at most 16, 32, 64, 128, 256 channels at the five levels (kTailC; a
+// narrower layer runs padded to them).
+constexpr int kTailLayers = 18;  // enc1.c1 (stem models only), enc1.c2 .. dec1.c2
+enum TailKind : int { TAIL_FOLD = 0, TAIL_POOL = 1, TAIL_UP = 2, TAIL_HEAD = 3 };
+struct TailLayer {
+  const uint32_t* w;   // sign bits [tile of 16 channels][step][64 lanes]: lane 16q + i, K slot 4 step + q, channel i
+  const float* tabs;   // C = the level's channels: [16][C] -S - c1; [C] r1, c1 - c2, r2; then inv1, inv2 [max(1, C / 32)]
+  int lvl, kind, steps;
+  int slot;            // first step in the slot table
+  int out, opair;      // LDS bytes of the output (TAIL_UP: at the level above), written as a pair tensor
+  int down, dpair;     // TAIL_POOL: the pooled output
+};
+struct TailArgs {
+  TailLayer L[kTailLayers];
+  int nlayers, nslot, lds_words, off_tab, off_in;
+  const int* slots;    // [step][4] LDS byte offset from a pixel's window corner, bit 31: no slot
+  const uint32_t* in;  // [N][32][32] bits of the first tensor (at most 16 channels)
+  int N;
+  const float* hw;     // head [ncls][hc]
+  const float* hl;     // [ncls][256]: bias and the first eight channels' steps, by their bits
+  int ncls, hc;
+  float* logits;       // [N][ncls][32][32], or the scene map [ncls][sH][sW]
+  int sH, sW, pcols, prow0;  // scene mode (pcols > 0), as in RealArgs
+};
+// patches a block for a launch of N: 1 or 2
+int tail_np(int N);
+// LDS words of one plane (all of a block's patches) at a level
+int tail_plane(int np, int lvl);
+hipError_t launch_tail(const TailArgs& a, int np, hipStream_t s);
 
 // the certified first conv (bits only; RealArgs with cwb, cws, out, no f32)
 hipError_t launch_real_cert(const RealArgs& a, hipStream_t s);
