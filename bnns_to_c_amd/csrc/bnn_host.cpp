@@ -870,9 +870,9 @@ int upload_real(BnnDevice* D, const Conv& c, const Act& a) {
     std::vector<uint64_t> wm(real_conv_masks_len(c.Cout, c.Cin));
     real_conv_masks(c.wsign, c.Cout, c.Cin, wm.data());
     if ((rc = dev_upload(D, &D->rwm, wm.data(), wm.size()))) return rc;
-    if (c.Cin <= 128 && c.Cin % 4 == 0) {
-      std::vector<uint16_t> cb(real_cert_b_len(c.Cout));
-      std::vector<uint32_t> cs(real_cert_s_len(c.Cout));
+    if (c.Cin <= 256) {
+      std::vector<uint16_t> cb(real_cert_b_len(c.Cout, c.Cin));
+      std::vector<uint32_t> cs(real_cert_s_len(c.Cout, c.Cin));
       real_cert_tables(c.wsign, c.Cout, c.Cin, cb.data(), cs.data());
       if ((rc = dev_upload(D, &D->rcwb, cb.data(), cb.size()))) return rc;
       if ((rc = dev_upload(D, &D->rcws, cs.data(), cs.size()))) return rc;
@@ -1155,9 +1155,7 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
     if (D->stem) {
       HIP_TRY(launch_stem(ra, st));
       if ((rc = mark("stem.conv", "conv_real", (double)N * D->rcout * H * W, (double)D->rcin))) return rc;
-    } else if (D->cert && real_cert_fits(D->rcin, W, sc ? sc->sW : W) && (uintptr_t)ra.x % 16 == 0) {
-      // (the certified kernel stages 16-byte groups; an input that is not
-      // 16-byte aligned takes the exact-order kernel below)
+    } else if (D->cert && real_cert_takes(ra)) {
       if (dump) {
         RealArgs rf = ra;
         rf.out = nullptr;
@@ -1449,9 +1447,12 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
   // (launch_real_cert; config 3's 660 patches as 506 + 154 instead of two
   // half-full rounds of 330)
   long cut = rows / 2;
-  if (parts == 2 && !D->stem && D->cert && real_cert_fits(D->rcin, W, sc ? sc->sW : W) &&
-      (uintptr_t)d_in % 16 == 0) {
-    const long round = real_cert_round(D->rcin, D->rcout, W) / unit;
+  RealArgs whole{};
+  whole.x = d_in;
+  whole.N = N; whole.H = H; whole.W = W; whole.cin = D->rcin; whole.cout = D->rcout;
+  if (sc) { whole.sH = sc->sH; whole.sW = sc->sW; whole.pcols = sc->pcols; }
+  if (parts == 2 && !D->stem && D->cert && real_cert_takes(whole)) {
+    const long round = real_cert_round(whole) / unit;
     if (round > 0 && rows > round && 2 * (rows - round) <= round) cut = round;
   }
   for (int k = 0; k < parts; ++k) {

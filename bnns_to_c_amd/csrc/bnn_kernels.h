@@ -193,32 +193,36 @@ inline void real_conv_masks(const int8_t* wsign, int cout, int cin, uint64_t* ou
           out[((size_t)(co / 16) * cp + ci) * 3 + t / 4] |= 1ull << (16 * (t % 4) + co % 16);
 }
 
-// Tables of the certified first conv (all signs +-1, cin <= 128):
+// Tables of the certified first conv (all signs +-1, cin <= 256; nw waves a
+// block, each with cpw = ceil(cin / nw) input channels):
 //  * operand table [16-channel group][wave w][tap][lane][8] fp16 bit
 //    patterns: lane l holds output channel 16 g + l % 16 and, in element j,
-//    input channel cin / 4 * w + 4 j + l / 16 when 4 j + l / 16 < cin / 4
-//    (+1 -> 0x3C00, -1 -> 0xBC00; other elements and channels past cout -> 0);
-//  * sign masks [cout padded to 16][tap][4] words: bit ci % 32 of word
+//    input channel cpw * w + 4 j + l / 16 when 4 j + l / 16 < cpw (+1 ->
+//    0x3C00, -1 -> 0xBC00; other elements, channels past cin or cout -> 0);
+//  * sign masks [cout padded to 16][tap][nw] words: bit ci % 32 of word
 //    ci / 32 set iff the weight is +1.
-inline size_t real_cert_b_len(int cout) { return (size_t)((cout + 15) / 16) * 4 * 9 * 64 * 8; }
-inline size_t real_cert_s_len(int cout) { return (size_t)((cout + 15) / 16) * 16 * 9 * 4; }
+inline int real_cert_waves(int cin) { return cin <= 128 ? 4 : 8; }
+inline size_t real_cert_b_len(int cout, int cin) {
+  return (size_t)((cout + 15) / 16) * real_cert_waves(cin) * 9 * 64 * 8;
+}
+inline size_t real_cert_s_len(int cout, int cin) { return (size_t)((cout + 15) / 16) * 16 * 9 * real_cert_waves(cin); }
 inline void real_cert_tables(const int8_t* wsign, int cout, int cin, uint16_t* b, uint32_t* s) {
-  const int ng = (cout + 15) / 16;
+  const int ng = (cout + 15) / 16, nw = real_cert_waves(cin), cpw = (cin + nw - 1) / nw;
   for (int g = 0; g < ng; ++g)
-    for (int w = 0; w < 4; ++w)
+    for (int w = 0; w < nw; ++w)
       for (int t = 0; t < 9; ++t)
         for (int l = 0; l < 64; ++l)
           for (int j = 0; j < 8; ++j) {
-            const int co = 16 * g + l % 16, cl = 4 * j + l / 16, ci = cin / 4 * w + cl;
+            const int co = 16 * g + l % 16, cl = 4 * j + l / 16, ci = cpw * w + cl;
             uint16_t v = 0;
-            if (co < cout && cl < cin / 4) v = wsign[((size_t)co * cin + ci) * 9 + t] > 0 ? 0x3C00 : 0xBC00;
-            b[((((size_t)g * 4 + w) * 9 + t) * 64 + l) * 8 + j] = v;
+            if (co < cout && cl < cpw && ci < cin) v = wsign[((size_t)co * cin + ci) * 9 + t] > 0 ? 0x3C00 : 0xBC00;
+            b[((((size_t)g * nw + w) * 9 + t) * 64 + l) * 8 + j] = v;
           }
-  for (size_t i = 0; i < real_cert_s_len(cout); ++i) s[i] = 0;
+  for (size_t i = 0; i < real_cert_s_len(cout, cin); ++i) s[i] = 0;
   for (int co = 0; co < cout; ++co)
     for (int t = 0; t < 9; ++t)
-      for (int ci = 0; ci < cin && ci < 128; ++ci)
-        if (wsign[((size_t)co * cin + ci) * 9 + t] > 0) s[((size_t)co * 9 + t) * 4 + ci / 32] |= 1u << (ci % 32);
+      for (int ci = 0; ci < cin; ++ci)
+        if (wsign[((size_t)co * cin + ci) * 9 + t] > 0) s[((size_t)co * 9 + t) * nw + ci / 32] |= 1u << (ci % 32);
 }
 // The real fold's bit as a function of the tap sum v, in the reference's
 // float steps (csrc/bnn_fold.c:62-77, A * o + B fused): o = al * v,
@@ -307,12 +311,6 @@ inline void real_fold_switches(float al, float A, float B, float sl, float rs, f
   *b0 = base ? 1.0f : 0.0f;
   *dc = d;
 }
-// whether launch_real_cert takes a layer of this shape (rows wider than 32
-// run as tiles of 32 columns with a one-column halo either side)
-inline bool real_cert_fits(int cin, int W, int rowlen) {
-  return cin >= 4 && cin <= 128 && cin % 4 == 0 && W >= 4 && W % 4 == 0 && rowlen % 4 == 0;
-}
-
 // 1x1 stem weights (v2 models; signs +1, -1 or 0): 64-bit lane masks
 // [group of four input channels q][16-channel group g][2]; bit 16k + i of
 // mask 0 is set iff w[16g + i][4q + k] > 0, of mask 1 iff it is nonzero.
@@ -652,9 +650,12 @@ hipError_t launch_tail(const TailArgs& a, int np, hipStream_t s);
 
 // the certified first conv (bits only; RealArgs with cwb, cws, out, no f32)
 hipError_t launch_real_cert(const RealArgs& a, hipStream_t s);
-// how many patches of this shape one round of the certified kernel holds
+// whether it takes a launch of this shape and input (N, H, W, cin, cout, x and
+// the scene fields): any width and row length, up to 256 input channels
+bool real_cert_takes(const RealArgs& a);
+// how many patches of such a launch one round of the certified kernel holds
 // (its blocks resident on the device at once), 0 if it cannot tell
-long real_cert_round(int cin, int cout, int W);
+long real_cert_round(const RealArgs& a);
 
 // The 1x1 head as its own kernel (heads over more than 32 channels, which
 // one epilogue group cannot hold): input the head layer's packed bits

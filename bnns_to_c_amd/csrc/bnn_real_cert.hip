@@ -23,7 +23,7 @@
 // are recombined (2048 Zh + Zl) and scaled back by 2^(e - 21) in fp32.
 //
 // E = 2^-24 (1 + 2^-8) A + (1 + 2^-8) Q + 2^-109, rounded up, with
-//  * A = sum over the output's 3 x 3 x cin window of (cin - ci + 16) |x|,
+//  * A = sum over the output's 3 x 3 x cin window of (cin - ci + 12 + NW) |x|,
 //    ci the input channel;
 //  * Q = half a grid step 2^(e-21) per term: 48 * 2^(e-21) per (input row,
 //    wave) of the window;
@@ -32,22 +32,24 @@
 //    sum_(k >= 2) 2^-24 |s_k|, and |s_k| <= (1 + 2^-24)^k sum_(i <= k) |t_i|,
 //    so by at most 2^-24 (1 + 2^-16) sum_i (cin - i + 1) |t_i|; the nine
 //    tap sums add 8 2^-24 (1 + 2^-16) sum |x| more;
-//  * this kernel's: recombination, two row adds, three adds of the
-//    four-wave reduction (each at most 2^-24 (sum |x| + Q)); the weight's
-//    "+ 16" covers these and the tap adds, 2^-8 the (1 + 2^-16) factors and
-//    the roundings of A itself, 2^-110 underflow.
+//  * this kernel's: recombination, two row adds, NW - 1 adds of the
+//    reduction over the NW waves (each at most 2^-24 (sum |x| + Q)); the
+//    weight's "+ 12 + NW" covers these and the eight tap adds, 2^-8 the
+//    (1 + 2^-16) factors and the roundings of A itself, 2^-110 underflow.
 //
-// Work split: one block of four waves per (patch, 16-channel group, tile
-// of 32 columns); wave w converts a quarter of the input channels.  Rows stream through a ring of
-// four LDS row buffers by 16-byte LDS DMA, one row ahead.  Each step
+// Work split: one block of NW waves, four, or eight above 128 input channels,
+// per (patch, 16-channel group, tile of 32 columns); wave w converts its NW-th
+// of the input channels (at most 32).  Rows stream through a ring of
+// four LDS row buffers by 16-byte LDS DMA
+// (4-byte where rows are not multiples of 16 bytes), one row ahead.  Each step
 // converts one input row into digits (the shifted operands of the kx = 0 and
 // kx = 2 taps come from DPP row shifts, the 16-lane rows being the operand's
 // pixel rows), runs 36 MFMAs into per-ky digit sums and adds them into three
 // rolling output-row partials.  An output row is complete one step after its
 // last input row: each wave writes its partial, its window sum of |x| and
 // its Q to LDS (plain stores; float atomics on LDS are several times slower
-// here), and after a barrier each wave adds the four in wave order for a
-// quarter of the row, folds, certifies and writes the bits.
+// here), and after a barrier each of four waves adds the NW in wave order
+// for a quarter of the row, folds, certifies and writes the bits.
 //
 // Rows wider than 32 (HALO): each block takes 32 output columns, its window
 // the same 32 columns (128-byte aligned rows of each channel), and the two
@@ -87,8 +89,8 @@ __device__ __forceinline__ uint32_t dmov(uint32_t src) {
   return (uint32_t)__builtin_amdgcn_mov_dpp((int)src, CTRL, 0xF, 0xF, true);
 }
 constexpr int kShl1 = 0x101, kShr1 = 0x111, kRor1 = 0x121;
-// halo of one ring slot: [channel 128][side 2] floats
-constexpr uint32_t kHaloSlot = 128 * 2 * 4;
+// halo of one ring slot: [channel 32 NW][side 2] floats
+constexpr uint32_t halo_slot(int nw) { return (uint32_t)nw * 32 * 2 * 4; }
 
 // Pixel layout of the operands: lane p of a 16-lane row holds pixel 2p of
 // the even segment (s = 0) and pixel 2p + 1 of the odd segment (s = 1).
@@ -194,7 +196,8 @@ __device__ __forceinline__ void window3(const float (&v)[2], float h, float (&o)
 // 16-byte store
 __device__ __forceinline__ int part_idx(int s, int g, int c) { return ((s * 4 + g) * 16 + c) * 4; }
 
-// Wave w converts input channels cpw * w .. cpw * w + cpw - 1 (cpw = cin / 4):
+// Wave w converts input channels cpw * w .. cpw * w + cpw - 1 (cpw = cin / NW,
+// rounded up; channels from cin on hold zeros in LDS and zero weights):
 // element j of lane (p, gq) is channel cpw * w + 4 j + gq, column 16 s + p;
 // elements past the wave's channels read as 0.  GUARD: such elements may
 // occur for j < 7 (cpw < 28); otherwise only element 7 can be one.
@@ -204,13 +207,23 @@ __device__ __forceinline__ int part_idx(int s, int g, int c) { return ((s * 4 + 
 // partial sets in LDS, one whole output word per pixel); its recompute
 // reads the sign masks and the halo columns from global memory, which
 // leaves LDS room for two blocks per CU.
-template <bool GUARD, bool HALO, int G>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+//
+// NW: waves per block, 4 (up to 128 input channels) or 8 (up to 256).
+//
+// DW: rows arrive by 4-byte instead of 16-byte LDS DMA, so that any row
+// length, width and 4-byte aligned input is taken (four times the load
+// instructions, the same bytes and LDS layout).  Against the order-exact
+// kernel, which such inputs and more than 128 bands took before: a forward of
+// 48 patches 45x51 of 103 bands, 24 channels 220 -> 186 us, a 301x217 scene
+// of 120 bands (rows of 868 bytes) 83 -> 66 us.
+template <bool GUARD, bool HALO, int G, int NW, bool DW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
 void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
+  constexpr uint32_t kHaloSlot = halo_slot(NW);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int p = lane & 15, gq = lane >> 4;
-  const int H = a.H, W = a.W, cin = a.cin, cpw = cin >> 2;
+  const int H = a.H, W = a.W, cin = a.cin, cpw = (cin + NW - 1) / NW;
   // rows up to 32 wide: one block per patch, window column = image column;
   // wider rows (HALO): tiles of 32 columns, the window the tile itself
   // (columns outside the image read 0)
@@ -240,13 +253,13 @@ void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
   const int vhi = HALO ? min(32, W - wx0) : W;  // output window columns 0 .. vhi - 1
   const uint32_t rb = (uint32_t)nld * 1024u;  // bytes per row buffer
   float* opart = cert_lds + (size_t)kCertRing * rb / 4;  // [group][wave][512]
-  float* absw = opart + G * 4 * 512;                     // [wave][32]
-  float* qw = absw + 4 * 32;                             // [wave]
-  uint32_t* wsl = reinterpret_cast<uint32_t*>(qw + 4);   // G = 1: [channel][tap][4] sign masks
-  // HALO: [slot][channel 128][side 2], at byte hal_off, one slot per ring
+  float* absw = opart + G * NW * 512;                    // [wave][32]
+  float* qw = absw + NW * 32;                            // [wave]
+  uint32_t* wsl = reinterpret_cast<uint32_t*>(qw + NW);  // G = 1: [channel][tap][NW] sign masks
+  // HALO: [slot][channel 32 NW][side 2], at byte hal_off, one slot per ring
   // row (G = 1) or two (G = 2: the conversion's and the next row's)
   constexpr int kHS = G == 1 ? kCertRing : 2;
-  const uint32_t hal_off = (uint32_t)kCertRing * rb + (G * 4 * 512 + 4 * 32 + 4 + (G == 1 ? 16 * 36 : 0)) * 4u;
+  const uint32_t hal_off = (uint32_t)kCertRing * rb + (G * NW * 512 + NW * 32 + NW + (G == 1 ? 16 * 9 * NW : 0)) * 4u;
   const float* hal = cert_lds + hal_off / 4;
   // G = 2: the 32 channels' fold parameters, [parameter 9][channel 32]
   // (alpha, A, B, slope, rsign, t1, t2, dc, b0), after the halo slots
@@ -258,7 +271,7 @@ void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
   cert_f16x8 Bw[G][9];
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    const uint4* src = reinterpret_cast<const uint4*>(a.cwb) + ((size_t)((grp * G + g) * 4 + wv) * 9) * 64 + lane;
+    const uint4* src = reinterpret_cast<const uint4*>(a.cwb) + ((size_t)((grp * G + g) * NW + wv) * 9) * 64 + lane;
 #pragma unroll
     for (int t = 0; t < 9; ++t) {
       const uint4 v = src[t * 64];
@@ -266,25 +279,36 @@ void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
     }
   }
 
-  // G = 1: the group's sign masks (16 channels x 9 taps x 4 words) for the
+  // G = 1: the group's sign masks (16 channels x 9 taps x NW words) for the
   // reference-order recompute; the first row barrier orders them
   if constexpr (G == 1)
-    for (int i = tid; i < 16 * 36; i += 256) wsl[i] = a.cws[(size_t)grp * 16 * 36 + i];
+    for (int i = tid; i < 16 * 9 * NW; i += 64 * NW) wsl[i] = a.cws[(size_t)grp * 16 * 9 * NW + i];
 
-  // DMA: wave w issues the row's 1 KiB loads k = w, w + 4, ... < nld; lane L
+  // DMA: wave w issues the row's 1 KiB loads k = w, w + NW, ... < nld; lane L
   // of load k fetches 16 bytes: channel 8 k + L / 8, column group (L % 8)
-  // swapped as in row_off
+  // swapped as in row_off.  DW: 256-byte loads k = w, w + NW, ... < 4 nld,
+  // lane L one float of channel 2 k + L / 32; a step of NW loads is 2 NW
+  // channels, a multiple of 4, so a lane's column is the same in all of them
   const InGeom ig = in_geom(a, n);
   const uint32_t rstr4 = (uint32_t)ig.rstride * 4u;
-  uint32_t doff[4];
+  constexpr int kLd = DW ? 16 : 4;  // loads of a wave: at most 32 NW channels
+  const int nk = DW ? 4 * nld : nld;
+  const int dci = DW ? 2 * wv + (lane >> 5) : 8 * wv + (lane >> 3);
+  const uint32_t cs4 = (uint32_t)ig.cstride * 4u;
+  uint32_t doff[DW ? 1 : kLd];
+  if constexpr (DW) {
+    const int col = wx0 + ((((lane >> 2) & 7) ^ (int)(row_swz(dci) << 2)) << 2) + (lane & 3);
+    doff[0] = col < ig.xlim ? (uint32_t)(ig.base + (size_t)dci * ig.cstride + col) * 4u : kCertFar;
+  } else {
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const int k = wv + 4 * m;
-    const int ci = 8 * k + (lane >> 3);
-    const int g4 = (lane & 7) ^ (int)(row_swz(ci) << 2);
-    const int cg = wx0 + 4 * g4;  // image column of the 16-byte group
-    const bool ok = k < nld && ci < cin && cg >= 0 && cg < ig.xlim;
-    doff[m] = ok ? (uint32_t)(ig.base + (size_t)ci * ig.cstride + cg) * 4u : kCertFar;
+    for (int m = 0; m < kLd; ++m) {
+      const int k = wv + NW * m;
+      const int ci = dci + 8 * NW * m;
+      const int g4 = (lane & 7) ^ (int)(row_swz(ci) << 2);
+      const int cg = wx0 + 4 * g4;  // image column of the 16-byte group
+      const bool ok = k < nld && ci < cin && cg < ig.xlim;
+      doff[m] = ok ? (uint32_t)(ig.base + (size_t)ci * ig.cstride + cg) * 4u : kCertFar;
+    }
   }
   // HALO: wave w's one load per row brings channels 32 w .. 32 w + 31, lane
   // L channel 32 w + L / 2 at window column -1 (L even) or 32 (L odd)
@@ -301,17 +325,32 @@ void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
     const uint32_t slot = lds0 + (uint32_t)(y % kCertRing) * rb;
     const bool inrow = y < ig.ylim;
     const uint32_t ro = (uint32_t)y * rstr4;
+    // (DW: compared in each step, so that no sixteen masks live across them)
+    int dlim = 0;
+    if constexpr (DW) {
+      dlim = inrow && doff[0] != kCertFar ? cin : 0;
+      asm volatile("" : "+v"(dlim));
+    }
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const int k = wv + 4 * m;
-      if (k >= nld) break;
-      const uint32_t m0v = uni(slot + (uint32_t)k * 1024u);
-      const uint32_t vo = (inrow && doff[m] != kCertFar) ? doff[m] + ro : kCertFar;
+    for (int m = 0; m < kLd; ++m) {
+      const int k = wv + NW * m;
+      if (k >= nk) break;
+      const uint32_t m0v = uni(slot + (uint32_t)k * (DW ? 256u : 1024u));
       const dma_u32x4 rd = xsrc;
-      asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                   :
-                   : "s"(m0v), "v"(vo), "s"(rd)
-                   : "memory");
+      if constexpr (DW) {
+        // (channels from cin on read 0, like columns outside the input)
+        const uint32_t vo = dci + 2 * NW * m < dlim ? doff[0] + ro + (uint32_t)(2 * NW * m) * cs4 : kCertFar;
+        asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+                     :
+                     : "s"(m0v), "v"(vo), "s"(rd)
+                     : "memory");
+      } else {
+        const uint32_t vo = (inrow && doff[m] != kCertFar) ? doff[m] + ro : kCertFar;
+        asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :
+                     : "s"(m0v), "v"(vo), "s"(rd)
+                     : "memory");
+      }
     }
     if (HALO && 32 * wv < cin) {
       const uint32_t m0h = uni(lds0 + hal_off + (uint32_t)(y % kHS) * kHaloSlot + (uint32_t)wv * 256u);
@@ -330,11 +369,11 @@ void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
   uint32_t jvalid = 0;
 #pragma unroll
   for (int j = 0; j < 8; ++j) jvalid |= (4 * j + gq < cpw ? 1u : 0u) << j;
-  // weight of element j's |x| in the window sum: cin - ci + 16 for its
+  // weight of element j's |x| in the window sum: cin - ci + 12 + NW for its
   // channel ci (the bound's weighted sum; exact small integers)
   float wsum[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) wsum[j] = (float)(cin + 16 - (cpw * wv + 4 * j + gq));
+  for (int j = 0; j < 8; ++j) wsum[j] = (float)(cin + 12 + NW - (cpw * wv + 4 * j + gq));
 
   // finalize: lane -> output channel fc of each group, pixels fpx0 and
   // fpx0 + 1.  The fold's bit along [-dc, dc] as at most two change points
@@ -555,7 +594,7 @@ void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
       const int r = yi - 1;
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        float* mine = opart + (g * 4 + wv) * 512;
+        float* mine = opart + (g * NW + wv) * 512;
 #pragma unroll
         for (int s = 0; s < 2; ++s)
           *reinterpret_cast<float4*>(&mine[part_idx(s, gq, p)]) =
@@ -569,10 +608,13 @@ void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
       __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
       block_barrier();
 
-      // finalize: the four partials in wave order
+      // finalize: the NW partials in wave order, by the first four waves (of
+      // eight, those that hold no more than their share of the row steps'
+      // work either way)
+      if (NW == 4 || wv < 4) {
       float v[G][2], Aw[2] = {0.0f, 0.0f};
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
+      for (int w = 0; w < NW; ++w) {
         const float2 u = *reinterpret_cast<const float2*>(&absw[w * 32 + fpx0]);
         Aw[0] = __fadd_rn(Aw[0], u.x);
         Aw[1] = __fadd_rn(Aw[1], u.y);
@@ -581,14 +623,18 @@ void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
       for (int g = 0; g < G; ++g) {
         v[g][0] = v[g][1] = 0.0f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          const float t0 = opart[(g * 4 + w) * 512 + i0], t1 = opart[(g * 4 + w) * 512 + i0 + 256];
+        for (int w = 0; w < NW; ++w) {
+          const float t0 = opart[(g * NW + w) * 512 + i0], t1 = opart[(g * NW + w) * 512 + i0 + 256];
           v[g][0] = __fadd_rn(v[g][0], t0);
           v[g][1] = __fadd_rn(v[g][1], t1);
         }
       }
-      const float4 qq = *reinterpret_cast<const float4*>(qw);
-      const float Qs = __fadd_rn(__fadd_rn(qq.x, qq.y), __fadd_rn(qq.z, qq.w));
+      float Qs = 0.0f;
+#pragma unroll
+      for (int w = 0; w < NW; w += 4) {
+        const float4 qq = *reinterpret_cast<const float4*>(qw + w);
+        Qs = __fadd_rn(Qs, __fadd_rn(__fadd_rn(qq.x, qq.y), __fadd_rn(qq.z, qq.w)));
+      }
       // the row's quantisation part of E with its margins, and 2^-109 for
       // underflow
       const float Qc = __fadd_rn(__fmul_rn(Qs, 1.0f + 0x1p-9f + 0x1p-19f), 0x1p-109f);
@@ -672,19 +718,20 @@ void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
         const int ky = tap / 3, kx = tap - 3 * (tap / 3);
         const int iy = r + ky - 1, ix = upx + kx - 1;
         if (kk < nb && iy >= 0 && iy < H && wx0 + ix >= 0 && wx0 + ix < W) {
-          // lane t sums tap t % 9: its four sign-mask words, then the
+          // lane t sums tap t % 9: its NW sign-mask words, then the
           // channels in batches of 32 read ahead of their adds (channels
           // 4 m, 4 m + 3 at column offset c0, 4 m + 1, 4 m + 2 at the
           // swapped one, as row_off lays them out).  A last partial batch
-          // reads up to 28 channels past cin, inside the block's LDS (a row
+          // reads up to 31 channels past cin, inside the block's LDS (a row
           // buffer holds at least cin channels and 11 KiB of partials follow
           // the ring), and adds +0 for them, which leaves a sum that started
           // at +0 unchanged.  HALO: a column outside the window (-1 or 32)
           // reads the row's halo, [channel][side] (G = 1), or global memory
           // (G = 2), instead.
-          const uint4 m4 = G == 1 ? *reinterpret_cast<const uint4*>(&wsl[((li & 15) * 9 + tap) * 4])
-                                  : *reinterpret_cast<const uint4*>(
-                                        &a.cws[(((size_t)(grp * G + g) * 16 + (li & 15)) * 9 + tap) * 4]);
+          const uint32_t* mp = G == 1 ? &wsl[((li & 15) * 9 + tap) * NW]
+                                      : &a.cws[(((size_t)(grp * G + g) * 16 + (li & 15)) * 9 + tap) * NW];
+          uint4 m4 = *reinterpret_cast<const uint4*>(mp), m8 = m4;
+          if constexpr (NW == 8) m8 = *reinterpret_cast<const uint4*>(mp + 4);
           const bool hcol = HALO && (ix < 0 || ix > 31);
           const int ixr = hcol ? 0 : ix;
           const float* rowp = cert_lds + (size_t)(iy % kCertRing) * rb / 4;
@@ -696,7 +743,6 @@ void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
           const uint32_t goff = iy < ig.ylim && wx0 + ix < ig.xlim
                                     ? (uint32_t)(ig.base + (size_t)iy * ig.rstride + (wx0 + ix)) * 4u
                                     : kCertFar;
-          const uint32_t cs4 = (uint32_t)ig.cstride * 4u;
           for (int cb = 0; cb < cin; cb += 32) {
             float xb[32];
 #pragma unroll
@@ -720,7 +766,9 @@ void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
             }
             // -x for a clear mask bit: bit j of the inverted word moved to
             // the sign position
-            const uint32_t nw = ~(cb < 32 ? m4.x : cb < 64 ? m4.y : cb < 96 ? m4.z : m4.w);
+            if (NW == 8 && cb == 128) m4 = m8;
+            const int cq = cb & 127;
+            const uint32_t nw = ~(cq < 32 ? m4.x : cq < 64 ? m4.y : cq < 96 ? m4.z : m4.w);
             if (cin - cb >= 32) {
 #pragma unroll
               for (int j = 0; j < 32; ++j) st = __fadd_rn(st, f32_of(bits_of(xb[j]) ^ ((nw << (31 - j)) & 0x80000000u)));
@@ -781,6 +829,7 @@ void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
           else *reinterpret_cast<uint16_t*>(dst) = (uint16_t)word;
         }
       }
+      }  // NW == 4 || wv < 4
     }
     // next step: output rows yi + 1 and yi, input rows yi - 1 and yi
 #pragma unroll
@@ -804,34 +853,60 @@ void k_real_cert(const RealArgs a, uint32_t xbytes, int nld, uint32_t nitems) {
 namespace {
 
 using CertFn = void (*)(const RealArgs, uint32_t, int, uint32_t);
-const CertFn kCertFns[8] = {k_real_cert<false, false, 1>, k_real_cert<true, false, 1>, k_real_cert<false, true, 1>,
-                            k_real_cert<true, true, 1>,   k_real_cert<false, false, 2>, k_real_cert<true, false, 2>,
-                            k_real_cert<false, true, 2>,  k_real_cert<true, true, 2>};
+// index: guard, halo, G = 2 bits (4 waves, 16-byte loads); then halo, G = 2
+// (4 waves, 4-byte loads); then halo, G = 2, 4-byte loads (8 waves)
+constexpr int kCertVars = 20;
+const CertFn kCertFns[kCertVars] = {
+    k_real_cert<false, false, 1, 4, false>, k_real_cert<true, false, 1, 4, false>,
+    k_real_cert<false, true, 1, 4, false>,  k_real_cert<true, true, 1, 4, false>,
+    k_real_cert<false, false, 2, 4, false>, k_real_cert<true, false, 2, 4, false>,
+    k_real_cert<false, true, 2, 4, false>,  k_real_cert<true, true, 2, 4, false>,
+    k_real_cert<true, false, 1, 4, true>,   k_real_cert<true, true, 1, 4, true>,
+    k_real_cert<true, false, 2, 4, true>,   k_real_cert<true, true, 2, 4, true>,
+    k_real_cert<true, false, 1, 8, false>,  k_real_cert<true, true, 1, 8, false>,
+    k_real_cert<true, false, 2, 8, false>,  k_real_cert<true, true, 2, 8, false>,
+    k_real_cert<true, false, 1, 8, true>,   k_real_cert<true, true, 1, 8, true>,
+    k_real_cert<true, false, 2, 8, true>,   k_real_cert<true, true, 2, 8, true>};
 
-// A launch's shape: the variant (guard, halo, G = 2 bits), its LDS bytes and
-// work items (blocks of a whole patch) per patch.
+// A launch's shape: the variant, its LDS bytes, waves a block and work items
+// (blocks of a whole patch) per patch.  dw: rows by 4-byte loads.
 struct CertShape {
-  int var, nld, G;
+  int var, nld, G, nw;
   size_t lds;
   long per_patch;
 };
-CertShape cert_shape(int cin, int cout, int W) {
+CertShape cert_shape(int cin, int cout, int W, bool dw) {
   CertShape c{};
   c.nld = (cin + 7) / 8;
-  const bool guard = cin / 4 < 28, halo = W > 32;
-  // 17 to 32 output channels: both 16-channel groups in one block
-  c.G = cout > 16 && cout <= 32 ? 2 : 1;
-  c.lds = (size_t)kCertRing * c.nld * 1024 + (c.G * 4 * 512 + 4 * 32 + 4 + (c.G == 1 ? 16 * 36 : 0)) * 4 +
-          (halo ? (c.G == 1 ? kCertRing : 2) * kHaloSlot : 0) + (c.G == 2 ? 9 * 32 * 4 : 0);
-  c.var = (guard ? 1 : 0) + (halo ? 2 : 0) + (c.G == 2 ? 4 : 0);
+  c.nw = real_cert_waves(cin);
+  const bool guard = (cin + 3) / 4 < 28, halo = W > 32;
+  auto lds = [&](int G) {
+    return (size_t)kCertRing * c.nld * 1024 + (G * c.nw * 512 + c.nw * 32 + c.nw + (G == 1 ? 16 * 9 * c.nw : 0)) * 4 +
+           (halo ? (G == 1 ? kCertRing : 2) * halo_slot(c.nw) : 0) + (G == 2 ? 9 * 32 * 4 : 0);
+  };
+  // 17 to 32 output channels: both 16-channel groups in one block, where
+  // their partials fit (up to 240 input channels)
+  c.G = cout > 16 && cout <= 32 && lds(2) <= 160 * 1024 ? 2 : 1;
+  c.lds = lds(c.G);
+  const int h = halo ? 1 : 0, g2 = c.G == 2 ? 1 : 0;
+  c.var = c.nw == 8 ? 12 + h + 2 * g2 + 4 * (dw ? 1 : 0) : dw ? 8 + h + 2 * g2 : (guard ? 1 : 0) + 2 * h + 4 * g2;
   c.per_patch = (halo ? (W + 31) / 32 : 1) * (long)((cout + 16 * c.G - 1) / (16 * c.G));
   return c;
+}
+CertShape cert_shape(const RealArgs& a) {
+  // 16-byte loads need every row of every channel, and every tile's edge, at
+  // a multiple of 16 bytes
+  const int rowlen = a.pcols > 0 ? a.sW : a.W;
+  return cert_shape(a.cin, a.cout, a.W, a.W % 4 != 0 || rowlen % 4 != 0 || (uintptr_t)a.x % 16 != 0);
+}
+size_t cert_in_bytes(const RealArgs& a) {
+  return a.pcols > 0 ? (size_t)a.cin * a.sH * a.sW * 4 : (size_t)a.N * a.cin * a.H * a.W * 4;
 }
 
 // The kernel asks for more than 64 KiB of LDS: allow it once per variant and
 // device (bit d of the variant's mask for device d).
 hipError_t cert_attr(int var) {
-  static std::atomic<uint64_t> attr[8];
+  static std::atomic<uint64_t> attr[kCertVars];
   int dev = 0;
   if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
   const uint64_t bit = 1ull << (dev & 63);
@@ -849,14 +924,14 @@ hipError_t cert_attr(int var) {
 // times the blocks one CU holds at these LDS bytes), cached per variant and
 // row-buffer count (the devices of one process are alike); 0 if unknown.
 long cert_slots(const CertShape& c) {
-  static std::atomic<long> cache[8][17];
-  if (c.nld < 1 || c.nld > 16) return 0;
+  static std::atomic<long> cache[kCertVars][33];
+  if (c.nld < 1 || c.nld > 32) return 0;
   long v = cache[c.var][c.nld].load(std::memory_order_acquire);
   if (v) return v;
   int dev = 0, ncu = 0, per_cu = 0;
   if (cert_attr(c.var) != hipSuccess || hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)kCertFns[c.var], 256, c.lds) != hipSuccess)
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)kCertFns[c.var], 64 * c.nw, c.lds) != hipSuccess)
     return 0;
   v = (long)ncu * per_cu;
   cache[c.var][c.nld].store(v, std::memory_order_release);
@@ -870,8 +945,14 @@ long cert_slots(const CertShape& c) {
 // empty launch, a row step 2.1)
 constexpr double kCertStart = 2.0;
 
-long real_cert_round(int cin, int cout, int W) {
-  const CertShape c = cert_shape(cin, cout, W);
+// (32-bit byte offsets, and a grid of fewer than 2^32 threads)
+bool real_cert_takes(const RealArgs& a) {
+  return a.cin >= 1 && a.cin <= 256 && (uintptr_t)a.x % 4 == 0 && cert_in_bytes(a) < kCertFar &&
+         (double)a.N * cert_shape(a).per_patch * 64 * cert_shape(a).nw < 4e9;
+}
+
+long real_cert_round(const RealArgs& a) {
+  const CertShape c = cert_shape(a);
   const long slots = cert_slots(c);
   return slots > 0 ? slots / c.per_patch : 0;
 }
@@ -879,11 +960,9 @@ long real_cert_round(int cin, int cout, int W) {
 hipError_t launch_real_cert(const RealArgs& a, hipStream_t s) {
   if ((long)a.N * a.H * a.W <= 0) return hipSuccess;
   if (!a.cwb || !a.cws || !a.ct1 || !a.ct2 || !a.cb0 || !a.cdc || !a.out || a.f32 || a.hout) return hipErrorInvalidValue;
-  const int rowlen = a.pcols > 0 ? a.sW : a.W;
-  if (!real_cert_fits(a.cin, a.W, rowlen) || (uintptr_t)a.x % 16) return hipErrorInvalidValue;
-  const size_t xbytes = a.pcols > 0 ? (size_t)a.cin * a.sH * a.sW * 4 : (size_t)a.N * a.cin * a.H * a.W * 4;
-  if (xbytes >= kCertFar) return hipErrorInvalidValue;
-  const CertShape c = cert_shape(a.cin, a.cout, a.W);
+  if (!real_cert_takes(a)) return hipErrorInvalidValue;
+  const size_t xbytes = cert_in_bytes(a);
+  const CertShape c = cert_shape(a);
   if (hipError_t e = cert_attr(c.var); e != hipSuccess) return e;
   const long npatch_items = (long)a.N * c.per_patch;
   // Row parts: a block's time is its row steps (the kernel is latency-bound,
@@ -917,7 +996,7 @@ hipError_t launch_real_cert(const RealArgs& a, hipStream_t s) {
   // a multiple of 8 blocks (one per XCD in turn); the padding ones exit
   const bool xorder = c.per_patch > 1 || a.cout > 16 || S > 1;
   const dim3 grid((unsigned)(xorder ? (nitems + 7) / 8 * 8 : nitems));
-  hipLaunchKernelGGL(kCertFns[c.var], grid, dim3(256), c.lds, s, b, (uint32_t)xbytes, c.nld, (uint32_t)nitems);
+  hipLaunchKernelGGL(kCertFns[c.var], grid, dim3(64 * c.nw), c.lds, s, b, (uint32_t)xbytes, c.nld, (uint32_t)nitems);
   return hipGetLastError();
 }
 

@@ -312,3 +312,51 @@ def test_cert_unaligned_input(tmp_path):
     want = eng.forward_batch(x)
     assert _bits_equal(y.cpu().numpy(), want)
     eng.close()
+
+
+@pytest.mark.parametrize("nb,base,H,W", [
+    (120, 16, 20, 30), (120, 32, 17, 33), (103, 16, 45, 51), (61, 8, 19, 67), (111, 16, 16, 35), (127, 24, 16, 31),
+    (1, 8, 16, 17), (2, 16, 18, 64), (97, 32, 16, 65),
+    (129, 16, 16, 32), (144, 32, 20, 64), (200, 16, 24, 40), (224, 32, 16, 37), (230, 24, 20, 65), (232, 32, 16, 64),
+    (235, 32, 16, 34), (256, 16, 16, 33), (255, 32, 18, 31)])
+def test_cert_any_rows_and_bands(tmp_path, orc, nb, base, H, W):
+    """Row lengths and band counts that are not multiples of 4 (rows by 4-byte
+    loads) and more than 128 bands (eight waves a block; from 241 bands on
+    one 16-channel group a block also for 32 channels): folds on ties of +-1
+    inputs, an infinity and a NaN, each bit against the checker."""
+    b = synth.make_blob(seed=70 + nb, base=base, n_bands=nb)
+    rng = np.random.default_rng(71 + nb)
+    x = rng.choice(np.array([-1.0, 1.0], np.float32), size=(2, nb, H, W))
+    model = orc.parse(B.to_bytes(b))
+    _, ref = model.forward(x[0], stages=True)
+    act = b.enc_act1[0]
+    A = act.A.astype(np.float32)
+    Bv = act.B.copy()
+    for c in range(len(Bv)):
+        Bv[c] = np.float32(-(A[c] * ref["enc1.conv1"][c, 5 + c % 8, 3 + c % 8]))
+    act.B = Bv.astype(np.float32)
+    act.rsign = np.where(np.arange(len(Bv)) % 2 == 0, np.float32(0.0), np.float32(1e-30)).astype(np.float32)
+    x[1, nb - 1, H - 1, W - 1] = np.inf
+    x[1, nb // 2, H // 2, W // 2] = np.nan
+    model = orc.parse(B.to_bytes(b))
+    eng = _engine(tmp_path, b)
+    eng.cert_stats()
+    _check(eng, model, x)
+    und, outs = eng.cert_stats()
+    assert und > 0 and outs == 2 * x.shape[0] * base * H * W  # the debug and the plain forward
+    eng.close()
+
+
+@pytest.mark.parametrize("nb,base,Hs,Ws", [(120, 16, 65, 67), (200, 16, 70, 61), (61, 32, 66, 97)])
+def test_cert_scene_odd_rows(tmp_path, orc, nb, base, Hs, Ws):
+    """A cube whose rows are not a multiple of 4 long: every map value equals
+    the exact-order kernel's."""
+    b = synth.make_blob(seed=75, base=base, n_bands=nb)
+    cube = synth.make_input(76, 1, nb, Hs, Ws)[0]
+    eng = _engine(tmp_path, b)
+    plain = _engine(tmp_path, b, name="p.blob", cert=False)
+    try:
+        assert _bits_equal(eng.forward_patched(cube, 32), plain.forward_patched(cube, 32))
+    finally:
+        eng.close()
+        plain.close()
