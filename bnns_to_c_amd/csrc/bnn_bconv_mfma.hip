@@ -57,8 +57,7 @@ struct KDiv {
   uint32_t d, mul, sh;
 };
 inline KDiv make_kdiv(uint32_t d) {
-  KDiv f{d, 0u, 0u};
-  while ((1ull << f.sh) < d) ++f.sh;
+  KDiv f{d, 0u, d > 1 ? 32u - (uint32_t)__builtin_clz(d - 1) : 0u};
   f.mul = (uint32_t)(((1ull << (31 + f.sh)) + d - 1) / d);
   return f;
 }

@@ -432,18 +432,42 @@ bool wide_layer(const DevBconv& L, int epi, int W) {
          L.cw0 + L.cw1 >= 2;
 }
 // The matrix-core conv by default where it measured faster than the popcount
-// kernel, which starts a launch sooner (about 2 us) but counts a word at a
-// time.  Event times, matrix cores against popcount:
-//  * 256 x 256 tiles, base 32, batch 64: 16-77 against 38-227 us a layer,
-//    every layer (2.4e9 to 1.3e11 bit-MACs);
-//  * 1024 patches of 32 x 32: 48 -> 16 channels (7.2e9) 20.0 against 24.5,
-//    16 -> 16 (2.4e9) 17.9 against 16.8;
-//  * pooled layers from 96 channels, 0.5e9: 7.7-10.6 against 9.2-13.8.
+// kernel, which starts a launch about 2 us sooner but counts a word at a time
+// (macs: the whole batch's bit-MACs, also for a part of it, since the parts
+// run side by side).  Times in us, matrix cores against popcount:
+//  * fold: from 2e9 every layer wins or ties (256 -> 256 at 1.9e9 11.0 : 16.2,
+//    96 -> 32 at 2.2e9 8.3 : 8.8; below, 24 -> 48 at 8.3e8 8.0 : 7.0, 144 -> 48
+//    at 1.6e9 9.3 : 8.4), and so do deep layers on few pixels, where a
+//    popcount wave walks all words of a pixel (256 -> 256 at 2.8e8 9.4 : 10.7,
+//    512 -> 512 at 9e6 11.6 : 14.0, but 192 -> 384 at 1.9e8 10.4 : 7.6);
+//  * pool: from 96 channels at any size (96 -> 40 at 2.4e7 7.2 : 7.6, 248 ->
+//    192 at 4.5e7 8.5 : 14.6), else from 2.5e9 (24 -> 24 at 3.7e9 18.2 : 23.1,
+//    16 -> 16 at 2.4e9 17.9 : 16.8);
+//  * head: 32 -> 32 at 4.8e9 14.0 : 16.9; 24 -> 24 at 3.7e9 31.8 : 24.4;
+//  * P: its stores bind, and rows of other lengths than whole groups of 16
+//    leave lanes and lines partly filled, so shallow layers take the matrix
+//    cores only with such rows (64 -> 64, 64 x 64, 75 : 89; 16 -> 128 there
+//    143 : 95; 64 -> 64, 45 x 51, 52 : 41), those from 96 channels also where
+//    many rounds of blocks even the last one out (152 -> 40, 3.4e5 pixels, 43 :
+//    62; 152 -> 64, 1.2e5 pixels, 36 : 28), deep ones always (232 -> 24 at
+//    1.6e9 10.2 : 15.4, 456 -> 168 at 1.2e9 16.3 : 10.3).
 // Wide layers (wide_layer) have always run there.
+bool mfma_pays(const DevBconv& L, int epi, int N, int H, int W) {
+  if (L.mfma == 2 || wide_layer(L, epi, W)) return true;
+  const double px = (double)N * H * W, macs = 9.0 * px * L.cin * L.cout;
+  switch (epi) {
+    case EPI_FOLD: return macs >= 2e9 || (L.cw1 == 0 && L.cin >= 256 && (macs >= 2.5e8 || L.cin >= 512));
+    case EPI_POOL: return macs >= 2.5e9 || L.cin >= 96;
+    case EPI_HEAD: return macs >= 4e9 && L.cin >= 32;
+  }
+  if (L.cin >= 224) return macs >= 1.5e9;
+  if (L.cin >= 176) return macs >= 4e9;
+  if (W % 16 == 0 && L.cin >= 48 && macs >= 8e9) return true;
+  return L.cin >= 96 && macs >= 4e9 && px * ((L.cout + 63) / 64) >= 3e5;
+}
 bool use_mfma(const DevBconv& L, int epi, int N, int H, int W) {
-  if (!mfma_conv_fits(L.mc, L.cw0 + L.cw1, N, H, W, epi)) return false;
-  const double macs = 9.0 * N * H * W * L.cin * L.cout;
-  return L.mfma == 2 || wide_layer(L, epi, W) || macs >= 4e9 || (epi == EPI_POOL && L.cin >= 96 && macs >= 3e8);
+  // (the tile is worked out only where it could run: 0.4 us of the host)
+  return L.mc.w && mfma_pays(L, epi, N, H, W) && mfma_conv_fits(L.mc, L.cw0 + L.cw1, N, H, W, epi);
 }
 // The profiler's name of a matrix-core layer: "_mfma" marks the wide layers,
 // as it always has (under BNN_BCONV_MFMA=2 every fold or pool layer of whole
@@ -1205,7 +1229,7 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
       a.P = dmp->P[pi++];
       if (epi == EPI_POOL) a.P2 = dmp->P2[lvl];
     }
-    const bool mm = use_mfma(L, epi, cnt, a.H, a.W);
+    const bool mm = use_mfma(L, epi, N, a.H, a.W);  // (the whole batch, as pick_shape below)
     if (mm) {
       if (dump) {
         // the debug forward's P: the same sums with the integer epilogue

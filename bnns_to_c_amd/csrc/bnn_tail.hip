@@ -154,7 +154,7 @@ __device__ __forceinline__ void tail_fetch(__amdgpu_buffer_rsrc_t wu, int steps,
 }
 
 // One layer of level LV, of 2^LV tiles of 16 channels.  A group is four 2x2
-// blocks in a row of blocks (level 3: a patch, level 4: four patches), so
+// blocks in a row of blocks (level 3: a patch, level 4: the block's patches), so
 // where a lane reads and writes is a constant of the lane and the level plus
 // the group's corner, which is scalar.
 template <int NP, int NW, int LV>
@@ -215,7 +215,7 @@ __device__ __forceinline__ void tail_layer(TailKarg kp, int li, uint8_t* smem, i
     lu = 2 * (2 * by + r) * p2 + 2 * (2 * bx + c);
     ld = by * p1 + bx;
   } else {
-    const int n = NP == 4 ? b4 : b4 & (NP - 1);  // (fewer than 16 pixels: the rest repeat)
+    const int n = b4 & (NP - 1);  // (fewer than 16 pixels: the rest repeat)
     lc = n * p * p + r * p + c;
     lu = n * p2 * p2 + 2 * r * p2 + 2 * c;
     ld = 0;

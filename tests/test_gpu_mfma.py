@@ -178,6 +178,35 @@ def test_layer_shapes_match_popcount(monkeypatch, N, H, W, cin, cout):
         assert np.array_equal(a, b)
 
 
+# both sides of the default rule's lines: P by depth, row length and pixels,
+# pools by depth and size
+@pytest.mark.parametrize("N,H,W,cin,cout", [(5220, 10, 5, 56, 32), (70, 64, 64, 64, 64), (60, 64, 64, 64, 64),
+                                            (300, 31, 41, 104, 24), (60, 31, 41, 104, 24), (246, 6, 17, 368, 56),
+                                            (7, 22, 20, 248, 176), (14, 22, 20, 248, 176), (45, 33, 93, 80, 24),
+                                            (45, 33, 93, 88, 24), (2, 49, 7, 96, 40)])
+def test_default_rule_layers_match_popcount(monkeypatch, N, H, W, cin, cout):
+    import torch
+    act = _act(torch, 55, N, H, W, cin)
+    w = B.pack_kidx(synth.make_signs(56, cout, cin))
+    r1 = synth.make_rules(57, cout, cin * 9, coverage=True)
+    r2 = synth.make_rules(58, cout, cin * 9, coverage=True)
+    cwo = (cout + 31) // 32
+    outs = {}
+    for mode in ("0", "1"):
+        monkeypatch.setenv("BNN_BCONV_MFMA", mode)
+        L = E.ConvLayer(w, cin, cout, r1, r2)
+        P = torch.full((N, cout, H, W), -7, dtype=torch.int32, device="cuda")
+        skip = torch.full((N, H, W, cwo), -1, dtype=torch.int32, device="cuda")
+        down = torch.full((N, H // 2, W // 2, cwo), -1, dtype=torch.int32, device="cuda")
+        L.P_device(act.data_ptr(), N, H, W, P.data_ptr(), None)
+        L.fold_pool_device(act.data_ptr(), N, H, W, skip.data_ptr(), down.data_ptr(), None)
+        torch.cuda.synchronize()
+        outs[mode] = [t.cpu().numpy() for t in (P, skip, down)]
+        L.close()
+    for a, b in zip(outs["0"], outs["1"]):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("base,N,H,W", [(8, 3, 35, 41), (16, 2, 32, 32), (24, 2, 45, 51), (20, 1, 70, 83)])
 def test_forced_forward_vs_checker(tmp_path, orc, monkeypatch, base, N, H, W):
     """Whole forwards with every layer on the matrix cores (the concat layers

@@ -1,6 +1,6 @@
 """Every binary layer of a 32x32 patch in one kernel (bnn_tail.hip), for v1 and
 stem models of at most 16, 32, 64, 128, 256 channels at the five levels, with
-1, 2 or 4 patches a block by the launch's size.  BNN_TAIL=0 keeps the layers
+1 or 2 patches a block by the launch's size.  BNN_TAIL=0 keeps the layers
 apart; the logits are the same bit for bit, and the checker's."""
 import numpy as np
 import pytest
@@ -28,7 +28,7 @@ def _bits(a):
     return np.ascontiguousarray(a).view(np.uint32)
 
 
-# one patch, a few, a partial last block of two and of four, more than a round
+# one patch, a few, a partial last block of two, more than a round
 @pytest.mark.parametrize("base,N,cov", [(16, 1, False), (16, 5, True), (16, 301, False), (16, 515, True),
                                          (16, 1031, True), (8, 2, True), (12, 3, True), (4, 1, True), (8, 601, False)])
 def test_tail_equals_layers(tmp_path, monkeypatch, orc, base, N, cov):
