@@ -932,7 +932,7 @@ def main() -> int:
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "fp32 first conv (certified: fp16 matrix-core digit sums, exact fp32 recompute where undecided) "
-                 "+ xnor-popcount (u32) binary convs",
+                 "+ binary convs exact (FP4 matrix cores, FP32 integer sums)",
         "data": "synthetic: seeded random blob (base 16, Bernoulli sign weights, U[-fan_in/4,fan_in/4] "
                 "ge/lt thresholds) and x ~ N(0,1) patches, resident in HBM",
         "config": {"workload": "v1 Bi-Real binary UNet forward (nearest upsampler), 32x32x120 patches",

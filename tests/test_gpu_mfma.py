@@ -1,15 +1,13 @@
 """The binary 3x3 conv on the matrix cores (bnn_bconv_mfma.hip).
 
 The kernel computes the same P as csrc/bnn_conv.c:23-36 (P = 2*D - S with
-D the int8 product of 0/1 activation bytes and +-1 weights, S the weight sum
-over the in-image taps), with the rule and the 2x2 max-pool of
+D the FP4 product of 0/1 activations and +-1 weights, S the weight sum over
+the in-image taps), with the rule and the 2x2 max-pool of
 csrc/bnn_fold.c:37-60 and csrc/bnn_maxpool.c:28-48 fused.  BNN_BCONV_MFMA=2
-routes every conv it fits (cout % 64 == 0, W a power of two in 8..64, rows
-that tile) through it; every stage of the forward must then equal the
-checker's bit for bit, as on the popcount path.  The default rule (at least
-four 64-channel input chunks) is checked to pick exactly the layers it
-names, and the isolated layer entry point must agree with the popcount
-kernel on the benchmark's fused config and smaller shapes.
+routes every conv through it; every stage of the forward must then equal the
+checker's bit for bit, as on the popcount path.  The default rule is checked
+on the wide layers that it names and on both sides of its lines, and the
+isolated layer entry point must agree with the popcount kernel.
 """
 import numpy as np
 import pytest
