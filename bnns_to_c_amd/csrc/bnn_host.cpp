@@ -417,12 +417,15 @@ bool tail_mode() {
 }
 
 // The certified first conv (launch_real_cert) makes the v1 enc1.conv1 bits
-// whenever its shape fits (real_cert_fits); BNN_CERT=0 keeps the exact-order
-// matrix-core kernel for them.  The debug forward's float conv output always
-// comes from the exact-order kernel.
-bool cert_mode() {
+// of a launch that fits (real_cert_takes) where it is the faster kernel
+// (real_cert_pays); BNN_CERT=0 keeps the exact-order matrix-core kernel for
+// them, =2 takes the certified one wherever it fits.  The debug forward's
+// float conv output always comes from the exact-order kernel.
+int cert_mode() {
   const char* e = getenv("BNN_CERT");
-  return !(e && !strcmp(e, "0"));
+  if (e && !strcmp(e, "0")) return 0;
+  if (e && !strcmp(e, "2")) return 2;
+  return 1;
 }
 
 // Fold and pool layers of full 64-channel groups from 64 or more input
@@ -497,11 +500,11 @@ struct BnnDevice {
   int rcin = 0, rcout = 0;
   uint64_t* rwm = nullptr;  // lane-mask weights (v1: all signs +-1, else null and rw is used)
   float *rw = nullptr, *ralpha = nullptr, *rA = nullptr, *rB = nullptr, *rslope = nullptr, *rrsign = nullptr;
-  // the certified first conv's tables (v1, all signs +-1, cin <= 128, cin % 4 == 0), and cert_mode()
+  // the certified first conv's tables (v1, all signs +-1, cin <= 256), and cert_mode()
   uint16_t* rcwb = nullptr;
   uint32_t* rcws = nullptr;
   float *rct1 = nullptr, *rct2 = nullptr, *rcb0 = nullptr, *rcdc = nullptr;  // its fold summary
-  bool cert = false;
+  int cert = 0;
   // outputs the certified conv recomputed (device) and certified in all
   // (host), since the last bnn_cert_stats
   unsigned long long* rcnt = nullptr;
@@ -539,6 +542,11 @@ struct BnnDevice {
   uint8_t* scratch = nullptr;
   std::string scratch_err;
 };
+
+// whether a launch of the first conv takes the certified kernel
+static bool use_cert(const BnnDevice* D, const RealArgs& a) {
+  return D->cert && real_cert_takes(a) && (D->cert == 2 || real_cert_pays(a));
+}
 
 struct BnnConvLayer {
   BnnDevice dev;   // owns the allocations
@@ -1016,7 +1024,7 @@ int build_device(Model* m, const StemPart* st = nullptr) {
   }
   D->mid = mid_mode() && mid_fits(D);
   D->midx = D->mid && midx_mode() && mid_ext_fits(D);
-  D->cert = cert_mode() && D->rcwb && D->rcws && D->rct1;
+  D->cert = D->rcwb && D->rcws && D->rct1 ? cert_mode() : 0;
   if (D->mid) {
     const auto L = mid_layers(D);
     const Conv* cv[kMidLayers] = {&m->enc_conv1[2], &m->enc_conv2[2], &m->enc_conv1[3], &m->enc_conv2[3],
@@ -1179,7 +1187,7 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
     if (D->stem) {
       HIP_TRY(launch_stem(ra, st));
       if ((rc = mark("stem.conv", "conv_real", (double)N * D->rcout * H * W, (double)D->rcin))) return rc;
-    } else if (D->cert && real_cert_takes(ra)) {
+    } else if (use_cert(D, ra)) {
       if (dump) {
         RealArgs rf = ra;
         rf.out = nullptr;
@@ -1475,7 +1483,7 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
   whole.x = d_in;
   whole.N = N; whole.H = H; whole.W = W; whole.cin = D->rcin; whole.cout = D->rcout;
   if (sc) { whole.sH = sc->sH; whole.sW = sc->sW; whole.pcols = sc->pcols; }
-  if (parts == 2 && !D->stem && D->cert && real_cert_takes(whole)) {
+  if (parts == 2 && !D->stem && use_cert(D, whole)) {
     const long round = real_cert_round(whole) / unit;
     if (round > 0 && rows > round && 2 * (rows - round) <= round) cut = round;
   }

@@ -653,6 +653,19 @@ hipError_t launch_real_cert(const RealArgs& a, hipStream_t s);
 // whether it takes a launch of this shape and input (N, H, W, cin, cout, x and
 // the scene fields): any width and row length, up to 256 input channels
 bool real_cert_takes(const RealArgs& a);
+// estimated times of the certified and the order-exact matrix-core kernel
+double real_cert_us(const RealArgs& a);
+double real_exact_us(const RealArgs& a);
+// Whether the certified kernel is to run: its estimated time against the
+// order-exact kernel's, both fitted (eight in ten within 15%) to the two
+// kernels' times of 1,260 launches of 16 to 256 bands, 8 to 32 output
+// channels, batches, images and scenes of any row length.  The certified conv's time hardly depends on the bands up to
+// 128 (120 bands of 1,024 32x32 patches 150 : 325 us), so few bands run in
+// order (19 bands, 154 patches 100x108, 351 : 172 us), and from 129 on a CU
+// holds one block of it for two (136 bands, 27 patches 110x98, 215 : 153 us;
+// 224 bands, 7 patches 32x32, 18 : 52).  Over those launches the rule takes
+// 81.7 ms, the certified kernel alone 87.3, the better of the two 81.5.
+inline bool real_cert_pays(const RealArgs& a) { return real_cert_us(a) <= real_exact_us(a); }
 // how many patches of such a launch one round of the certified kernel holds
 // (its blocks resident on the device at once), 0 if it cannot tell
 long real_cert_round(const RealArgs& a);

@@ -2236,6 +2236,16 @@ int device_cus() {
   return cus[dev];
 }
 
+// The order-exact matrix-core conv's time in us: 6 for the launch; two blocks
+// a CU hold 8 x 32 pixels of 16 channels each, a round of them 3.3 and 2.63 a
+// chunk of 8 input channels (1.59 where each CU has one).
+double real_exact_us(const RealArgs& a) {
+  const long cus = device_cus(), chunks = (a.cin + kRealMfmaCI - 1) / kRealMfmaCI;
+  const long blocks = (long)a.N * ((a.H + 7) / 8) * ((a.W + 31) / 32) * ((a.cout + 15) / 16);
+  const long full = blocks / (2 * cus), rest = blocks % (2 * cus);
+  return 6.0 + (double)full * (3.3 + 2.63 * chunks) + (rest > cus ? 3.3 + 2.63 * chunks : rest ? 3.3 + 1.59 * chunks : 0.0);
+}
+
 hipError_t launch_real(const RealArgs& a, hipStream_t s) {
   if ((long)a.N * a.H * a.W <= 0) return hipSuccess;
   const size_t xbytes = a.pcols > 0 ? (size_t)a.cin * a.sH * a.sW * 4 : (size_t)a.N * a.cin * a.H * a.W * 4;

@@ -60,6 +60,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -940,10 +941,66 @@ long cert_slots(const CertShape& c) {
 
 }  // namespace
 
+namespace {
+
 // row steps a block's time holds beyond its rows' (launch, tables, first row:
 // a two-row part of one 32x32 patch, three row steps, measured 5.7 us above an
 // empty launch, a row step 2.1)
-constexpr double kCertStart = 2.0;
+constexpr int kCertStart = 2;
+
+// A launch's row parts: a block's time is its row steps (the kernel is
+// latency-bound, a block alone on its CU takes about as long as two), so each
+// patch's rows are split over S blocks where that fills the device better.  A
+// part of rh rows takes rh + 1 row steps (it re-reads the input row above it)
+// and about kCertStart of them before its first row; the S taken has the least
+// rounds x steps, the fewest blocks among equals.  Against halves and
+// quarters within one round only, conv time by events: one 32x32 patch
+// 19.0 -> 10.3 us (16 parts for 4), 64 patches 29.4 -> 21.4 (8 for 4), one
+// 512x512 image 285 -> 68 us (32 parts for 4, 64 blocks of 512 possible).
+struct CertParts {
+  int S, rh;
+  long slots;
+};
+CertParts cert_parts(const RealArgs& a, const CertShape& c) {
+  CertParts p{1, a.H, cert_slots(c)};
+  if (p.slots <= 0) return p;
+  const long items = (long)a.N * c.per_patch;
+  double best = 0.0;
+  // (each count of parts with its fewest rows a part: 2 sqrt(H) of them)
+  for (int rh = a.H; rh >= 2; --rh) {
+    const int parts = (a.H + rh - 1) / rh;
+    rh = (a.H + parts - 1) / parts;
+    const double t = (double)((items * parts + p.slots - 1) / p.slots) * (rh + 1 + kCertStart);
+    if (parts == 1 || t < 0.98 * best) {
+      best = t;
+      p.S = parts;
+      p.rh = rh;
+    }
+  }
+  return p;
+}
+
+// us of a row step with one, two and three blocks on a CU, by variant
+constexpr double kCertStep[kCertVars][3] = {
+    {1.47, 2.05, 2.50}, {1.47, 2.05, 2.50}, {1.86, 2.83, 2.83}, {1.86, 2.83, 2.83},  // 4 waves: one group, tiles
+    {2.16, 2.85, 2.85}, {2.16, 2.85, 2.85}, {3.20, 3.88, 3.88}, {3.20, 3.88, 3.88},  // two groups, tiles
+    {1.81, 2.29, 2.29}, {2.44, 3.08, 3.08}, {2.52, 3.07, 3.07}, {3.39, 4.11, 4.11},  // the four by 4-byte loads
+    {2.67, 2.67, 2.67}, {3.84, 3.84, 3.84}, {3.94, 3.94, 3.94}, {5.09, 5.09, 5.09},  // 8 waves
+    {3.03, 3.03, 3.03}, {4.08, 4.08, 4.08}, {4.13, 4.13, 4.13}, {5.35, 5.35, 5.35}};  // 8 waves, 4-byte loads
+
+}  // namespace
+
+// The launch's time in us: 6 for the launch, then each round's blocks (the
+// last one's by how many share a CU) their row steps.
+double real_cert_us(const RealArgs& a) {
+  const CertShape c = cert_shape(a);
+  const CertParts p = cert_parts(a, c);
+  if (p.slots <= 0) return 0.0;
+  const long cus = device_cus(), per_cu = std::max(1l, p.slots / cus);
+  const long items = (long)a.N * c.per_patch * p.S, full = items / p.slots, rest = items % p.slots;
+  auto step = [&](long k) { return kCertStep[c.var][std::min(k, 3l) - 1]; };
+  return 6.0 + (p.rh + 1 + kCertStart) * ((double)full * step(per_cu) + (rest ? step((rest + cus - 1) / cus) : 0.0));
+}
 
 // (32-bit byte offsets, and a grid of fewer than 2^32 threads)
 bool real_cert_takes(const RealArgs& a) {
@@ -964,32 +1021,8 @@ hipError_t launch_real_cert(const RealArgs& a, hipStream_t s) {
   const size_t xbytes = cert_in_bytes(a);
   const CertShape c = cert_shape(a);
   if (hipError_t e = cert_attr(c.var); e != hipSuccess) return e;
-  const long npatch_items = (long)a.N * c.per_patch;
-  // Row parts: a block's time is its row steps (the kernel is latency-bound,
-  // a block alone on its CU takes about as long as two), so each patch's rows
-  // are split over S blocks where that fills the device better.  A part of
-  // rh rows takes rh + 1 row steps (it re-reads the input row above it) and
-  // about kCertStart of them before its first row; the S taken has the least
-  // rounds x steps, the fewest blocks among equals.  Against halves and
-  // quarters within one round only, conv time by events: one 32x32 patch
-  // 19.0 -> 10.3 us (16 parts for 4), 64 patches 29.4 -> 21.4 (8 for 4), one
-  // 512x512 image 285 -> 68 us (32 parts for 4, 64 blocks of 512 possible).
-  const long slots = cert_slots(c);
-  int S = 1;
-  if (slots > 0) {
-    double best = 0.0;
-    for (int rh = a.H; rh >= 2; --rh) {
-      const int parts = (a.H + rh - 1) / rh;
-      if ((a.H + parts - 1) / parts != rh) continue;  // a smaller rh has as many parts
-      const long items = npatch_items * parts;
-      const double t = (double)((items + slots - 1) / slots) * (rh + 1 + kCertStart);
-      if (rh == a.H || t < 0.98 * best) {
-        best = t;
-        S = parts;
-      }
-    }
-  }
-  const long nitems = npatch_items * S;
+  const int S = cert_parts(a, c).S;
+  const long nitems = (long)a.N * c.per_patch * S;
   if (nitems >= 0x7FFFFFF0) return hipErrorInvalidValue;
   RealArgs b = a;
   b.rsplit = S;

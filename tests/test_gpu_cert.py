@@ -14,7 +14,9 @@ bound cannot decide many outputs and the reference-order recompute must:
 The debug forward reports the act1 bits of the certified kernel (its float
 conv output comes from the exact-order kernel); the plain forward's logits
 must match too, and a model loaded with BNN_CERT=0 (exact-order kernel for
-the bits) must give bit-identical logits on a larger batch.
+the bits) must give bit-identical logits on a larger batch.  The models here
+are loaded with BNN_CERT=2, which takes the certified kernel wherever it
+fits; test_cert_taken_where_it_pays loads them as a program does.
 """
 import os
 
@@ -33,10 +35,10 @@ def _engine(tmp_path, b, name="m.blob", cert=True):
     p = tmp_path / name
     p.write_bytes(B.to_bytes(b))
     old = os.environ.get("BNN_CERT")
-    if cert:
+    if cert is None:  # whichever kernel is the faster one
         os.environ.pop("BNN_CERT", None)
     else:
-        os.environ["BNN_CERT"] = "0"
+        os.environ["BNN_CERT"] = "2" if cert else "0"
     try:
         return E.Engine(str(p))
     finally:
@@ -294,9 +296,8 @@ def test_cert_stats_counts(tmp_path):
 
 
 def test_cert_unaligned_input(tmp_path):
-    """An input that is not 16-byte aligned runs (on the exact-order kernel,
-    the certified one stages 16-byte groups) with the same logits as an
-    aligned copy."""
+    """An input that is not 16-byte aligned runs (its rows by 4-byte loads)
+    with the same logits as an aligned copy."""
     import torch
 
     b = synth.make_blob(seed=57)
@@ -360,3 +361,25 @@ def test_cert_scene_odd_rows(tmp_path, orc, nb, base, Hs, Ws):
     finally:
         eng.close()
         plain.close()
+
+
+# few bands, and 129 and more on many pixels, where the order-exact kernel is
+# the faster one; 120 bands, and many bands on few pixels, where it is not
+@pytest.mark.parametrize("nb,base,N,H,W,takes", [
+    (23, 16, 64, 28, 90, False), (22, 16, 1, 213, 565, False), (16, 8, 1, 118, 21, False),
+    (136, 16, 1, 213, 470, False), (144, 16, 26, 63, 43, False), (136, 16, 27, 110, 98, False),
+    (120, 16, 64, 32, 32, True), (120, 16, 1, 32, 32, True), (120, 16, 2, 300, 217, True),
+    (136, 16, 1, 32, 32, True), (224, 16, 7, 32, 32, True), (220, 16, 4, 81, 27, True), (178, 16, 2, 35, 28, True)])
+def test_cert_taken_where_it_pays(tmp_path, nb, base, N, H, W, takes):
+    """The default takes the faster of the two first convs (real_cert_pays);
+    the logits are the same either way."""
+    b = synth.make_blob(seed=57, base=base, n_bands=nb)
+    x = synth.make_input(58, N, nb, H, W)
+    eng = _engine(tmp_path, b, cert=None)
+    eng.cert_stats()
+    got = eng.forward_batch(x)
+    assert eng.cert_stats()[1] == (N * base * H * W if takes else 0)
+    other = _engine(tmp_path, b, "o.blob", cert=not takes)
+    assert _bits_equal(got, other.forward_batch(x))
+    eng.close()
+    other.close()
