@@ -49,8 +49,8 @@ before each other configuration.  Prints ONE JSON line on stdout:
                 against the FP4 peak, and the bit-packed popcount kernel
                 (BNN_BCONV_MFMA=0) against the VALU-popcount peak
   cfg4          benchmark config 4: 256x256x120 patches, batch 64, base 32;
-                per-kernel times, the wide matrix-core convs against the
-                dense FP4 peak
+                per-kernel times, the matrix-core convs against the dense
+                FP4 peak
   scene         benchmark config 3: a 956x684x120 scene by 32x32 patches,
                 device-resident and from host memory (PCIe included)
   v2_stem       the v2 spectral-stem model (16-channel 1x1 stem, then the
@@ -965,8 +965,7 @@ def main() -> int:
             "cfg4": {"config": "large tiles: 256x256x120, batch 64, base 32 (512 channels at the bottleneck)",
                      "ms_per_step": round(cfg4_ms, 4), "patches_s": round(N4 / cfg4_ms * 1e3, 1),
                      "kernels": cfg4_kern,
-                     "mfma_rule": "every binary layer; \"_mfma\" marks fold and pool convs with cout % 64 == 0, "
-                                  "rows at least 16 wide and 64+ input channels (enc2.c2 .. dec2.c2 here)"},
+                     "mfma_rule": "\"_mfma\" names the matrix-core kernel, the others ran on the popcount kernel"},
             "scene": {"config": f"{SH}x{SW}x{b.n_bands} cube, {PS}x{PS} patches ({npatch}, edge patches zero "
                                 "past the scene), benchmark config 3",
                       "device_ms": round(scene_dev_ms, 4), "device_patches_s": round(npatch / scene_dev_ms * 1e3, 1),

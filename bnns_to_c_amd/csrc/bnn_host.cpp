@@ -472,13 +472,6 @@ bool use_mfma(const DevBconv& L, int epi, int N, int H, int W) {
   // (the tile is worked out only where it could run: 0.4 us of the host)
   return L.mc.w && mfma_pays(L, epi, N, H, W) && mfma_conv_fits(L.mc, L.cw0 + L.cw1, N, H, W, epi);
 }
-// The profiler's name of a matrix-core layer: "_mfma" marks the wide layers,
-// as it always has (under BNN_BCONV_MFMA=2 every fold or pool layer of whole
-// 64-channel groups); the others keep their plain name.
-bool named_mfma(const DevBconv& L, int epi, int W) {
-  return wide_layer(L, epi, W) || (L.mfma == 2 && L.cout % 64 == 0 && (epi == EPI_FOLD || epi == EPI_POOL));
-}
-
 struct Workspace {
   int N = 0, H = 0, W = 0;
   uint8_t* base = nullptr;
@@ -1252,10 +1245,9 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
       pick_shape(epi, N, a.H, a.W, L.cout, &mt, &cog);
       HIP_TRY(launch_bconv(a, epi, mt, cog, dump, st));
     }
-    const bool nm = mm && named_mfma(L, epi, a.W);
-    const char* ot = epi == EPI_POOL ? (nm ? "bconv_pool_mfma" : "bconv_pool")
-                     : epi == EPI_HEAD ? "bconv_head"
-                                       : (nm ? "bconv_mfma" : "bconv");
+    const char* ot = epi == EPI_POOL   ? (mm ? "bconv_pool_mfma" : "bconv_pool")
+                     : epi == EPI_HEAD ? (mm ? "bconv_head_mfma" : "bconv_head")
+                                       : (mm ? "bconv_mfma" : "bconv");
     return mark(label, ot, (double)N * L.cout * a.H * a.W, (double)L.cin * 9);
   };
 

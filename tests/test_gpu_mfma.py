@@ -80,7 +80,8 @@ def test_forced_mfma_stages_vs_checker(tmp_path, orc, monkeypatch, seed, base, N
 
 def test_default_rule_picks_wide_layers(tmp_path, orc, monkeypatch):
     """Default: the matrix cores for fold and pool layers with cout % 64 == 0,
-    rows at least 16 wide and at least 64 input channels."""
+    rows at least 16 wide and at least 64 input channels, and for deep folds;
+    a layer's op names the kernel that ran."""
     monkeypatch.delenv("BNN_BCONV_MFMA", raising=False)
     b = synth.make_blob(seed=26, base=32)
     p = tmp_path / "m.blob"
@@ -89,9 +90,11 @@ def test_default_rule_picks_wide_layers(tmp_path, orc, monkeypatch):
     x = synth.make_input(126, 1, 120, 128, 128)
     ops = _ops(eng, x)
     # base 32 at 128x128: levels 1, 2, 3 are 64, 32 and 16 wide with 64,
-    # 128 and 256 channels; level 0 (128 wide, 32 channels), enc2.c1 (32
-    # input channels) and the 8 x 8 bottleneck stay on the popcount kernel
+    # 128 and 256 channels, bott.c2 has 512; level 0 (128 wide, 32 channels),
+    # enc2.c1 (32 input channels) and bott.c1 (256 to 512 on 8 x 8 pixels)
+    # stay on the popcount kernel
     want = {f"{lv}.c{k}" for lv in ("enc2", "enc3", "enc4", "dec4", "dec3", "dec2") for k in (1, 2)} - {"enc2.c1"}
+    want |= {"bott.c2"}
     got = {lab for lab, op in ops.items() if op.endswith("_mfma")}
     assert got == want, (got, ops)
     _check_stages(eng, orc.parse(B.to_bytes(b)), x)
