@@ -8,6 +8,7 @@
 // (-mllvm -amdgpu-mfma-vgpr-form): the epilogue reads all of them.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 
 #include "bnn_device.h"
 #include "bnn_kernels.h"
@@ -707,6 +708,108 @@ bool mfma_conv_fits(const MfmaConv& mc, int cw, int N, int H, int W, int epi) {
   return mfma_lds(mc, cw, &T) <= 160 * 1024;
 }
 
+// A launch: its tile, the pixel groups a wave (G), LDS bytes, the blocks a CU
+// holds of it, and the tile slots (blocks per channel group and XCD) and
+// rounds over them.
+struct MfmaPlan {
+  MfmaTile T;
+  int G;
+  size_t lds, per_cu;
+  uint32_t nts, rounds;
+};
+static MfmaPlan mfma_plan(const MfmaConv& mc, int cw, int N, int H, int W, int epi, int cus) {
+  const bool pool = epi == EPI_POOL;
+  const size_t waves = mfma_waves(mc.mt, epi);  // blocks a CU holds by registers
+  MfmaPlan p{};
+  mfma_tile(N, H, W, cw, pool, 256, 1, &p.T);
+  p.lds = mfma_lds(mc, cw, &p.T);
+  p.G = 4;
+  if (epi != EPI_HEAD && (size_t)p.T.ntiles * p.T.ncg < 2 * (size_t)cus) {
+    // 32 pixels a wave where 64 leave CUs without a block
+    MfmaTile T2{};
+    mfma_tile(N, H, W, cw, pool, 128, 1, &T2);
+    const size_t l2 = mfma_lds(mc, cw, &T2);
+    if (l2 <= 160 * 1024) { p.T = T2; p.lds = l2; p.G = 2; }
+  } else {
+    // two or four tiles staged together where that costs no round of blocks
+    // (a tile's staging costs about one and a half times its sums)
+    double best = 0.0;
+    MfmaTile T2{};
+    for (int sub = 1; sub <= 4; sub *= 2) {
+      mfma_tile(N, H, W, cw, pool, 256, sub, &T2);
+      const size_t l2 = mfma_lds(mc, cw, &T2);
+      if (T2.sub != sub || (sub > 1 && l2 > 53 * 1024)) break;
+      const size_t slots = std::max<size_t>(1, std::min<size_t>(waves, 160 * 1024 / l2)) * cus;
+      const double t = (double)(((size_t)T2.ntiles * T2.ncg + slots - 1) / slots) * (sub + 1.5);
+      if (sub == 1 || t < best) { best = t; p.T = T2; p.lds = l2; }
+    }
+  }
+  // as many blocks as fit on the chip at once (LDS, registers), the tiles
+  // spread evenly over them
+  p.per_cu = std::max<size_t>(1, std::min<size_t>(waves, (160 * 1024) / p.lds));
+  const uint32_t t8 = (p.T.ntiles + 7) / 8;
+  const uint32_t most = std::max<uint32_t>(1, (uint32_t)(p.per_cu * cus / 8 / p.T.ncg));
+  p.rounds = (t8 + most - 1) / most;
+  p.nts = (t8 + p.rounds - 1) / p.rounds;
+  return p;
+}
+
+// Folds and pools: the lesser of both kernels' estimated times in us, fitted
+// to 2,238 layers timed on both (8 to 1,152 input channels, 8 to 768 output
+// channels, 1 to 67,000 patches of 1 to 640 rows; eight times in ten within 9%
+// here, 13% for popcount).  Summed over the layers the choice takes 20.6 ms,
+// the better of the two 20.5, the popcount kernel alone 27.5, this one 22.7.
+//  * popcount: a wave counts its words (9 a tap word, 5 a pair) over cog
+//    channels x 1 or 4 pixels, the waves over the 1,024 SIMDs; from 60 words
+//    on, and with the weights' bytes, its weight loads show;
+//  * here: K steps and rounds of tiles, by the blocks that share a CU: staging
+//    by pixels and planes, sums by operands, the epilogue by outputs.
+// Pairs (us, popcount : here): folds 64 -> 64, one 128x128 image, 5.0 : 7.1,
+// 96 -> 192, 32x32, 5.2 : 8.1, 48 -> 16, 61 patches 113x73, 12.7 : 16.9, 256
+// -> 256, 148 of 4x4, 16.4 : 10.5, 512 -> 512, 32x32, 33.8 : 12.4; pools 16 ->
+// 16, 1,618 patches 70x25, 31 : 45, 32 -> 8, 6,154 of 15x19, 17 : 39, 40 ->
+// 192, 192 of 35x4, 16.1 : 10.1.
+// The head and P go by lines through the same pairs of times:
+//  * head: 32 -> 32 at 4.8e9 bit-MACs 16.9 : 14.0; 24 -> 24 at 3.7e9 24.4 :
+//    31.8;
+//  * P: its stores bind, and rows of other lengths than whole groups of 16
+//    leave lanes and lines partly filled, so shallow layers run here only with
+//    such rows (64 -> 64, 64 x 64, 89 : 75; 16 -> 128 there 95 : 143; 64 -> 64,
+//    45 x 51, 41 : 52), those from 96 channels also where many rounds of blocks
+//    even the last one out (152 -> 40, 3.4e5 pixels, 62 : 43; 152 -> 64, 1.2e5
+//    pixels, 28 : 36), from 224 channels at 1.5e9 bit-MACs (232 -> 24 at 1.6e9
+//    15.4 : 10.2; 456 -> 168 at 1.2e9 10.3 : 16.3).
+bool mfma_conv_pays(const MfmaConv& mc, int cin, int cout, int cw, bool pair, int epi, int N, int H, int W) {
+  const double px = (double)N * H * W, macs = 9.0 * px * cin * cout;
+  if (epi == EPI_HEAD || epi == EPI_P) {
+    const bool pays = epi == EPI_HEAD ? macs >= 4e9 && cin >= 32
+                      : cin >= 224    ? macs >= 1.5e9
+                      : cin >= 176    ? macs >= 4e9
+                                      : (W % 16 == 0 && cin >= 48 && macs >= 8e9) ||
+                                         (cin >= 96 && macs >= 4e9 && px * ((cout + 63) / 64) >= 3e5);
+    return pays && mfma_conv_fits(mc, cw, N, H, W, epi);
+  }
+  const bool pool = epi == EPI_POOL;
+  const int cus = device_cus();
+  int mt, cog;
+  bconv_shape(epi, N, H, W, cout, &mt, &cog);
+  const long waves = ((long)N * ((H + mt - 1) / mt) * ((W + mt - 1) / mt) + 63) / 64 * ((cout + cog - 1) / cog);
+  const double words = 9 * cw - (pair ? 4 : 0), ws = (double)waves / (4 * cus);
+  const double turns = ws < 2 ? std::ceil(ws) : ws, out = turns * cog * mt * mt;
+  const double deep = turns * std::max(0.0, words - 60), kw = words * cout / 1024;
+  const double pop = pool ? 4.91 + out * (0.0035 * words + 0.0188) + 0.27 * kw + 0.048 * deep
+                          : 4.33 + out * (0.0036 * words + 0.0085) + 0.088 * kw + 0.021 * deep;
+  const double start = pool ? 5.87 + 0.093 * mc.steps : 5.19 + 0.071 * mc.steps;
+  if (pop <= start || !mfma_conv_fits(mc, cw, N, H, W, epi)) return false;
+  const MfmaPlan p = mfma_plan(mc, cw, N, H, W, epi, cus);
+  const double blocks = 8.0 * p.T.ncg * p.nts, planes = (cw + 3) / 4, loads = cw < 4 ? cw : 0;
+  const double share = blocks <= (double)p.per_cu * cus ? std::min((double)p.per_cu, std::ceil(blocks / cus)) : blocks / cus;
+  const double stage = p.rounds * share * p.T.ns / 256, sums = p.rounds * share * p.T.sub * mc.mt * p.G;
+  const double here = pool ? start + stage * (0.287 * planes + 0.0218 * loads) + sums * (0.0077 * mc.steps + 0.0348) + 0.33 * p.rounds * planes
+                           : start + stage * 0.378 * planes + sums * (0.0100 * mc.steps + 0.0286) + 0.28 * p.rounds * planes;
+  return here < pop;
+}
+
 namespace {
 using MfmaFn = void (*)(const MfmaParams);
 template <int MT, int G, bool RES>
@@ -741,40 +844,15 @@ hipError_t launch_bconv_mfma(const BconvArgs& a, const MfmaConv& mc, int epi, hi
   if (a.in1 && (size_t)a.N * a.h1 * a.w1 * a.cw1 * 4 >= 0x80000000ull) return hipErrorInvalidValue;
   int dev = 0;
   if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
-  const int cus = device_cus();
-  const bool pool = epi == EPI_POOL;
-  const size_t waves = mfma_waves(mc.mt, epi);  // blocks a CU holds by registers
-  MfmaTile T{};
-  mfma_tile(a.N, a.H, a.W, cw, pool, 256, 1, &T);
-  size_t lds = mfma_lds(mc, cw, &T);
-  int G = 4;
-  if (epi != EPI_HEAD && (size_t)T.ntiles * T.ncg < 2 * (size_t)cus) {
-    // 32 pixels a wave where 64 leave CUs without a block
-    MfmaTile T2{};
-    mfma_tile(a.N, a.H, a.W, cw, pool, 128, 1, &T2);
-    const size_t l2 = mfma_lds(mc, cw, &T2);
-    if (l2 <= 160 * 1024) { T = T2; lds = l2; G = 2; }
-  } else {
-    // two or four tiles staged together where that costs no round of blocks
-    // (a tile's staging costs about one and a half times its sums)
-    double best = 0.0;
-    MfmaTile T2{};
-    for (int sub = 1; sub <= 4; sub *= 2) {
-      mfma_tile(a.N, a.H, a.W, cw, pool, 256, sub, &T2);
-      const size_t l2 = mfma_lds(mc, cw, &T2);
-      if (T2.sub != sub || (sub > 1 && l2 > 53 * 1024)) break;
-      const size_t slots = std::max<size_t>(1, std::min<size_t>(waves, 160 * 1024 / l2)) * cus;
-      const double t = (double)(((size_t)T2.ntiles * T2.ncg + slots - 1) / slots) * (sub + 1.5);
-      if (sub == 1 || t < best) { best = t; T = T2; lds = l2; }
-    }
-  }
+  const MfmaPlan p = mfma_plan(mc, cw, a.N, a.H, a.W, epi, device_cus());
+  const MfmaTile& T = p.T;
   if ((size_t)a.N * T.dhp.d >= 0x7FFFFFFFull) return hipErrorInvalidValue;
-  const MfmaFn fn = T.resident ? mfma_fn<true>(mc.mt, G, epi) : mfma_fn<false>(mc.mt, G, epi);
+  const MfmaFn fn = T.resident ? mfma_fn<true>(mc.mt, p.G, epi) : mfma_fn<false>(mc.mt, p.G, epi);
   if (!fn) return hipErrorInvalidValue;
   // more than 64 KB of LDS: allowed once per variant and device (bit d of
   // the variant's mask for device d)
   static std::atomic<uint64_t> attr[2][3][2][4];
-  std::atomic<uint64_t>& at = attr[T.resident][mc.mt >> 1][G >> 2][epi];
+  std::atomic<uint64_t>& at = attr[T.resident][mc.mt >> 1][p.G >> 2][epi];
   const uint64_t bit = 1ull << (dev & 63);
   if (!(at.load(std::memory_order_acquire) & bit)) {
     if (hipError_t e = hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -782,16 +860,10 @@ hipError_t launch_bconv_mfma(const BconvArgs& a, const MfmaConv& mc, int epi, hi
       return e;
     at.fetch_or(bit, std::memory_order_acq_rel);
   }
-  // as many blocks as fit on the chip at once (LDS, registers), the tiles
-  // spread evenly over them
-  const size_t per_cu = std::max<size_t>(1, std::min<size_t>(waves, (160 * 1024) / lds));
-  const uint32_t t8 = (T.ntiles + 7) / 8;
-  const uint32_t most = std::max<uint32_t>(1, (uint32_t)(per_cu * cus / 8 / T.ncg));
-  const uint32_t rounds = (t8 + most - 1) / most, nts = (t8 + rounds - 1) / rounds;
   const uint32_t b0 = (uint32_t)(npix * a.cw0 * 4);
   // (a v3 tensor's pad pixel lies just past its last one)
   const uint32_t b1 = a.in1 ? (uint32_t)((size_t)a.N * a.h1 * a.w1 * a.cw1 * 4) : 0u;
-  hipLaunchKernelGGL(fn, dim3(8 * (unsigned)T.ncg * nts), dim3(256), lds, s, MfmaParams{a, mc, T, b0, b1});
+  hipLaunchKernelGGL(fn, dim3(8 * (unsigned)T.ncg * p.nts), dim3(256), p.lds, s, MfmaParams{a, mc, T, b0, b1});
   return hipGetLastError();
 }
 

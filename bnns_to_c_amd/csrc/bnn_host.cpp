@@ -357,7 +357,7 @@ FoldHost canon_fold(const Act& a, int coutp) {
 }
 
 // Which binary convs run on the matrix cores (same results as the popcount
-// kernel either way; use_mfma).  BNN_BCONV_MFMA=0 keeps them all on the
+// kernel either way; mfma_conv_pays).  BNN_BCONV_MFMA=0 keeps them all on the
 // popcount kernel, =2 takes the matrix cores wherever a tile fits (both read
 // when a model or layer is created).
 int mfma_conv_mode() {
@@ -428,50 +428,13 @@ int cert_mode() {
   return 1;
 }
 
-// Fold and pool layers of full 64-channel groups from 64 or more input
-// channels with rows a power of two at least 16 wide.
-bool wide_layer(const DevBconv& L, int epi, int W) {
-  return L.cout % 64 == 0 && (epi == EPI_FOLD || epi == EPI_POOL) && W >= 16 && (W & (W - 1)) == 0 &&
-         L.cw0 + L.cw1 >= 2;
-}
-// The matrix-core conv by default where it measured faster than the popcount
-// kernel, which starts a launch about 2 us sooner but counts a word at a time
-// (macs: the whole batch's bit-MACs, also for a part of it, since the parts
-// run side by side).  Times in us, matrix cores against popcount:
-//  * fold: from 2e9 every layer wins or ties (256 -> 256 at 1.9e9 11.0 : 16.2,
-//    96 -> 32 at 2.2e9 8.3 : 8.8; below, 24 -> 48 at 8.3e8 8.0 : 7.0, 144 -> 48
-//    at 1.6e9 9.3 : 8.4), and so do deep layers on few pixels, where a
-//    popcount wave walks all words of a pixel (256 -> 256 at 2.8e8 9.4 : 10.7,
-//    512 -> 512 at 9e6 11.6 : 14.0, but 192 -> 384 at 1.9e8 10.4 : 7.6);
-//  * pool: from 96 channels at any size (96 -> 40 at 2.4e7 7.2 : 7.6, 248 ->
-//    192 at 4.5e7 8.5 : 14.6), else from 2.5e9 (24 -> 24 at 3.7e9 18.2 : 23.1,
-//    16 -> 16 at 2.4e9 17.9 : 16.8);
-//  * head: 32 -> 32 at 4.8e9 14.0 : 16.9; 24 -> 24 at 3.7e9 31.8 : 24.4;
-//  * P: its stores bind, and rows of other lengths than whole groups of 16
-//    leave lanes and lines partly filled, so shallow layers take the matrix
-//    cores only with such rows (64 -> 64, 64 x 64, 75 : 89; 16 -> 128 there
-//    143 : 95; 64 -> 64, 45 x 51, 52 : 41), those from 96 channels also where
-//    many rounds of blocks even the last one out (152 -> 40, 3.4e5 pixels, 43 :
-//    62; 152 -> 64, 1.2e5 pixels, 36 : 28), deep ones always (232 -> 24 at
-//    1.6e9 10.2 : 15.4, 456 -> 168 at 1.2e9 16.3 : 10.3).
-// Wide layers (wide_layer) have always run there.
-bool mfma_pays(const DevBconv& L, int epi, int N, int H, int W) {
-  if (L.mfma == 2 || wide_layer(L, epi, W)) return true;
-  const double px = (double)N * H * W, macs = 9.0 * px * L.cin * L.cout;
-  switch (epi) {
-    case EPI_FOLD: return macs >= 2e9 || (L.cw1 == 0 && L.cin >= 256 && (macs >= 2.5e8 || L.cin >= 512));
-    case EPI_POOL: return macs >= 2.5e9 || L.cin >= 96;
-    case EPI_HEAD: return macs >= 4e9 && L.cin >= 32;
-  }
-  if (L.cin >= 224) return macs >= 1.5e9;
-  if (L.cin >= 176) return macs >= 4e9;
-  if (W % 16 == 0 && L.cin >= 48 && macs >= 8e9) return true;
-  return L.cin >= 96 && macs >= 4e9 && px * ((L.cout + 63) / 64) >= 3e5;
-}
 bool use_mfma(const DevBconv& L, int epi, int N, int H, int W) {
-  // (the tile is worked out only where it could run: 0.4 us of the host)
-  return L.mc.w && mfma_pays(L, epi, N, H, W) && mfma_conv_fits(L.mc, L.cw0 + L.cw1, N, H, W, epi);
+  if (!L.mc.w) return false;
+  const int cw = L.cw0 + L.cw1;
+  return L.mfma == 2 ? mfma_conv_fits(L.mc, cw, N, H, W, epi)
+                     : mfma_conv_pays(L.mc, L.cin, L.cout, cw, L.pair, epi, N, H, W);
 }
+
 struct Workspace {
   int N = 0, H = 0, W = 0;
   uint8_t* base = nullptr;
@@ -1100,19 +1063,6 @@ struct ProfRec {
 };
 std::vector<ProfRec> g_prof;
 
-// work-item shape: pool epilogue needs 2x2 blocks, the head one pixel; the
-// channel group shrinks until the launch has ~4 waves per SIMD
-void pick_shape(int epi, int N, int H, int W, int cout, int* mt, int* cog) {
-  *mt = (epi == EPI_POOL) ? 2 : 1;
-  if (epi == EPI_HEAD) { *cog = cout <= 16 ? 16 : 32; return; }
-  const long tiles = (long)N * ((H + *mt - 1) / *mt) * ((W + *mt - 1) / *mt);
-  int c = *mt == 2 ? 16 : 32;
-  while (c > 8 && c / 2 >= cout) c /= 2;  // no group wider than the layer
-  auto waves = [&](int g) { return ((tiles + 63) / 64) * (long)((cout + g - 1) / g); };
-  while (c > 8 && waves(c) < 4096) c /= 2;
-  *cog = c;
-}
-
 struct Dumps {
   bool on = false;
   float* conv1 = nullptr;
@@ -1230,7 +1180,7 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
       a.P = dmp->P[pi++];
       if (epi == EPI_POOL) a.P2 = dmp->P2[lvl];
     }
-    const bool mm = use_mfma(L, epi, N, a.H, a.W);  // (the whole batch, as pick_shape below)
+    const bool mm = use_mfma(L, epi, N, a.H, a.W);  // (the whole batch, as bconv_shape below)
     if (mm) {
       if (dump) {
         // the debug forward's P: the same sums with the integer epilogue
@@ -1242,7 +1192,7 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
       int mt, cog;
       // the shape the whole batch would take: the parts run side by side,
       // so each part's kernel needs only its share of the waves
-      pick_shape(epi, N, a.H, a.W, L.cout, &mt, &cog);
+      bconv_shape(epi, N, a.H, a.W, L.cout, &mt, &cog);
       HIP_TRY(launch_bconv(a, epi, mt, cog, dump, st));
     }
     const char* ot = epi == EPI_POOL   ? (mm ? "bconv_pool_mfma" : "bconv_pool")
@@ -2348,7 +2298,7 @@ int bnn_layer_P_device(const BnnConvLayer* L, const uint32_t* d_act, int N, int 
     return BNN_OK;
   }
   int mt, cog;
-  pick_shape(EPI_P, N, H, W, a.cout, &mt, &cog);
+  bconv_shape(EPI_P, N, H, W, a.cout, &mt, &cog);
   HIP_TRY(launch_bconv(a, EPI_P, mt, cog, false, (hipStream_t)stream));
   return BNN_OK;
 }
@@ -2366,7 +2316,7 @@ int bnn_layer_fold_pool_device(const BnnConvLayer* L, const uint32_t* d_act, int
     return BNN_OK;
   }
   int mt, cog;
-  pick_shape(EPI_POOL, N, H, W, a.cout, &mt, &cog);
+  bconv_shape(EPI_POOL, N, H, W, a.cout, &mt, &cog);
   HIP_TRY(launch_bconv(a, EPI_POOL, mt, cog, false, (hipStream_t)stream));
   return BNN_OK;
 }

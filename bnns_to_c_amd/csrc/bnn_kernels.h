@@ -420,6 +420,19 @@ hipError_t launch_conv3_chain(const float* x, const int8_t* wsign, const float* 
 hipError_t launch_bconv(const BconvArgs& a, int epi, int mt, int cog, bool dump,
                         hipStream_t s);
 
+// work-item shape: pool epilogue needs 2x2 blocks, the head one pixel; the
+// channel group shrinks until the launch has ~4 waves per SIMD
+inline void bconv_shape(int epi, int N, int H, int W, int cout, int* mt, int* cog) {
+  *mt = (epi == EPI_POOL) ? 2 : 1;
+  if (epi == EPI_HEAD) { *cog = cout <= 16 ? 16 : 32; return; }
+  const long tiles = (long)N * ((H + *mt - 1) / *mt) * ((W + *mt - 1) / *mt);
+  int c = *mt == 2 ? 16 : 32;
+  while (c > 8 && c / 2 >= cout) c /= 2;  // no group wider than the layer
+  auto waves = [&](int g) { return ((tiles + 63) / 64) * (long)((cout + g - 1) / g); };
+  while (c > 8 && waves(c) < 4096) c /= 2;
+  *cog = c;
+}
+
 // Binary conv on the matrix cores (FP4 operands, FP32 sums; the kernel's file
 // says how).  With activation bits alpha in {0,1} (0 for taps outside the
 // image) and weights w in {-1,+1}, D = sum over valid taps of w*alpha and
@@ -533,12 +546,16 @@ inline void mfma_rule(int32_t lo, uint32_t wid, int K, float* c, float* r, bool*
   *c = n ? 0.5f * (float)(a + b) : 0.0f;
   *r = n ? 0.5f * (float)(b - a) + 0.5f : -1.0f;
 }
+// compute units of the current device (cached per device)
+int device_cus();
 // Whether launch_bconv_mfma takes a layer of cw input words a pixel (every
 // shape whose tile, operand and tables fit a CU's LDS; the head in one wave's
 // channels; the rules the epilogue needs).
-// compute units of the current device (cached per device)
-int device_cus();
 bool mfma_conv_fits(const MfmaConv& mc, int cw, int N, int H, int W, int epi);
+// Whether the layer fits and this is its faster kernel (the kernel's file says
+// by which times).  N is the whole batch's, also for a part of it: the parts
+// run side by side.
+bool mfma_conv_pays(const MfmaConv& mc, int cin, int cout, int cw, bool pair, int epi, int N, int H, int W);
 hipError_t launch_bconv_mfma(const BconvArgs& a, const MfmaConv& m, int epi, hipStream_t s);
 hipError_t launch_real(const RealArgs& a, hipStream_t s);
 

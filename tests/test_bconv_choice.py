@@ -1,0 +1,54 @@
+"""Which kernel a binary conv takes by default (mfma_conv_pays,
+bnns_to_c_amd/csrc/bnn_bconv_mfma.hip): layers that measured at least a tenth
+faster on one of the two, on either side of the choice.  CPU only: the choice
+is host code."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+LIB = os.path.join(ROOT, "bnns_to_c_amd", "lib")
+
+# (epilogue, cin, cout, skip channels of a concat, N, H, W, popcount us, matrix-core us)
+LAYERS = [
+    ("pool", 16, 16, 0, 1618, 70, 25, 31.1, 45.1),
+    ("pool", 16, 8, 0, 35609, 9, 17, 39.5, 101.7),
+    ("pool", 32, 8, 0, 6154, 15, 19, 17.1, 39.2),
+    ("pool", 16, 16, 0, 3444, 13, 48, 23.9, 39.7),
+    ("pool", 16, 72, 0, 3013, 26, 8, 33.0, 37.2),
+    ("pool", 40, 192, 0, 192, 35, 4, 16.1, 10.1),
+    ("pool", 128, 128, 0, 1024, 32, 32, 288.0, 82.0),
+    ("pool", 152, 16, 0, 7466, 29, 6, 66.9, 47.4),
+    ("fold", 64, 64, 0, 1, 128, 128, 5.0, 7.1),
+    ("fold", 96, 192, 0, 1, 32, 32, 5.2, 8.1),
+    ("fold", 192, 64, 64, 3, 32, 32, 7.0, 10.1),
+    ("fold", 48, 16, 16, 61, 113, 73, 12.7, 16.9),
+    ("fold", 64, 64, 0, 1, 145, 32, 5.2, 7.0),
+    ("fold", 512, 512, 0, 1, 32, 32, 33.8, 12.4),
+    ("fold", 256, 256, 0, 148, 4, 4, 16.4, 10.5),
+    ("fold", 1152, 384, 384, 1, 13, 20, 38.6, 21.4),
+    ("fold", 768, 256, 256, 1, 17, 36, 26.4, 16.4),
+    ("head", 32, 32, 0, 64, 256, 256, 97.6, 69.1),
+    ("head", 24, 24, 0, 152, 113, 51, 28.2, 34.0),
+    ("P", 64, 64, 0, 256, 64, 64, 89.0, 75.0),
+    ("P", 72, 168, 0, 2381, 17, 5, 67.1, 91.3),
+]
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc (for the HIP headers) not found")
+def test_layers_take_their_faster_kernel(tmp_path):
+    assert os.path.exists(os.path.join(LIB, "libbnn_hip.so")), "the library is not built"
+    exe = tmp_path / "bcc"
+    subprocess.run([HIPCC, "-O1", "-std=c++17", "-I", os.path.join(ROOT, "bnns_to_c_amd", "csrc"), "-I",
+                    os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "bconv_choice_check.cpp"), "-o", str(exe),
+                    "-L", LIB, "-lbnn_hip", "-Wl,-rpath," + LIB], check=True, capture_output=True, timeout=300)
+    text = "".join("%s %d %d %d %d %d %d\n" % layer[:7] for layer in LAYERS)
+    r = subprocess.run([str(exe)], input=text, capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stderr
+    took = [int(v) for v in r.stdout.split()]
+    want = [int(layer[8] < layer[7]) for layer in LAYERS]
+    wrong = [layer for layer, t, w in zip(LAYERS, took, want) if t != w]
+    assert len(took) == len(LAYERS) and not wrong, wrong
