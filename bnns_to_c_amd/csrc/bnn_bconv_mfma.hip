@@ -183,12 +183,12 @@ __global__ __launch_bounds__(256, mfma_waves(MT, EPI)) void k_bconv_mfma(const M
     offn = okr && (unsigned)(x + 1) < (unsigned)W ? (pix + 1u) * 4u : kFar;
     off1 = kFar;
     if (k->a.cw1) {
-      // nearest 2x upsample placed at (oh, ow); what it does not cover reads at padoff
+      // nearest 2x upsample placed at (oh, ow); what it does not cover reads 0
       const int uy = y - k->a.oh, ux = x - k->a.ow;
       off1 = (unsigned)uy < (unsigned)k->a.uh && (unsigned)ux < (unsigned)k->a.uw
                  ? (((uint32_t)n * (uint32_t)k->a.h1 + (uint32_t)(uy >> 1)) * (uint32_t)k->a.w1 +
                     (uint32_t)(ux >> 1)) * ((uint32_t)k->a.cw1 * 4u)
-                 : k->a.padoff;
+                 : kFar;
       off1 = ok ? off1 : kFar;
     }
   };
@@ -836,6 +836,9 @@ hipError_t launch_bconv_mfma(const BconvArgs& a, const MfmaConv& mc, int epi, hi
   const int cw = a.cw0 + a.cw1;
   if (!mfma_conv_fits(mc, cw, a.N, a.H, a.W, epi) || a.cout > mc.coutp) return hipErrorInvalidValue;
   if (mc.slots != mfma_nslots(a.cw0, a.cw1, a.pair)) return hipErrorInvalidValue;
+  // v1 concats only: what the upsample leaves uncovered reads 0 bits (a v3
+  // tensor's pad pixel lies past the range in1 is read in)
+  if (a.in1 && a.padoff != kFar) return hipErrorInvalidValue;
   if (epi == EPI_P && !a.P) return hipErrorInvalidValue;
   if (epi == EPI_POOL && !a.out2) return hipErrorInvalidValue;
   if (epi == EPI_FOLD && !a.out) return hipErrorInvalidValue;
@@ -861,7 +864,6 @@ hipError_t launch_bconv_mfma(const BconvArgs& a, const MfmaConv& mc, int epi, hi
     at.fetch_or(bit, std::memory_order_acq_rel);
   }
   const uint32_t b0 = (uint32_t)(npix * a.cw0 * 4);
-  // (a v3 tensor's pad pixel lies just past its last one)
   const uint32_t b1 = a.in1 ? (uint32_t)((size_t)a.N * a.h1 * a.w1 * a.cw1 * 4) : 0u;
   hipLaunchKernelGGL(fn, dim3(8 * (unsigned)T.ncg * p.nts), dim3(256), p.lds, s, MfmaParams{a, mc, T, b0, b1});
   return hipGetLastError();

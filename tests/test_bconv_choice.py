@@ -38,17 +38,28 @@ LAYERS = [
 ]
 
 
+def _build(tmp_path, source):
+    assert os.path.exists(os.path.join(LIB, "libbnn_hip.so")), "the library is not built"
+    exe = tmp_path / "check"
+    subprocess.run([HIPCC, "-O1", "-std=c++17", "-I", os.path.join(ROOT, "bnns_to_c_amd", "csrc"), "-I",
+                    os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", source), "-o", str(exe),
+                    "-L", LIB, "-lbnn_hip", "-Wl,-rpath," + LIB], check=True, capture_output=True, timeout=300)
+    return str(exe)
+
+
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc (for the HIP headers) not found")
 def test_layers_take_their_faster_kernel(tmp_path):
-    assert os.path.exists(os.path.join(LIB, "libbnn_hip.so")), "the library is not built"
-    exe = tmp_path / "bcc"
-    subprocess.run([HIPCC, "-O1", "-std=c++17", "-I", os.path.join(ROOT, "bnns_to_c_amd", "csrc"), "-I",
-                    os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "bconv_choice_check.cpp"), "-o", str(exe),
-                    "-L", LIB, "-lbnn_hip", "-Wl,-rpath," + LIB], check=True, capture_output=True, timeout=300)
     text = "".join("%s %d %d %d %d %d %d\n" % layer[:7] for layer in LAYERS)
-    r = subprocess.run([str(exe)], input=text, capture_output=True, text=True, timeout=60)
+    r = subprocess.run([_build(tmp_path, "bconv_choice_check.cpp")], input=text, capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr
     took = [int(v) for v in r.stdout.split()]
     want = [int(layer[8] < layer[7]) for layer in LAYERS]
     wrong = [layer for layer, t, w in zip(LAYERS, took, want) if t != w]
     assert len(took) == len(LAYERS) and not wrong, wrong
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc (for the HIP headers) not found")
+def test_pad_pixel_concat_is_refused(tmp_path):
+    """1: hipErrorInvalidValue."""
+    r = subprocess.run([_build(tmp_path, "bconv_refusal_check.cpp")], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.split() == ["1"], r.stdout + r.stderr
