@@ -56,6 +56,17 @@ int set_err(int code, const char* fmt, ...) {
 
 bool prof_enabled() { return g_prof_on; }
 
+static bool capturing(hipStream_t q) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(q, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+bool side_stream(hipStream_t own, hipStream_t caller) {
+  return own != caller && !capturing(caller) && !capturing(own);
+}
+
 std::vector<uint32_t> repack_bin(const uint64_t* kbits, int cin, int cout, int taps, int cs) {
   const int nw = (cin * taps + 63) / 64;
   const int cw0 = words(cs ? cs : cin), cw1 = cs ? words(cin - cs) : 0;
@@ -490,7 +501,8 @@ struct BnnDevice {
   hipStream_t copy = nullptr;
   hipEvent_t ev_copied[2] = {}, ev_free[2] = {}, ev_done[2] = {};
   // the parts of a large batch before the last run their binary layers on
-  // these streams, each from the event after its first conv
+  // `stream` or, where that one is not free to (side_stream), on these, each
+  // from the event after its first conv
   hipStream_t side[kSplitMax - 1] = {};
   hipEvent_t ev_conv[kSplitMax - 1] = {}, ev_join[kSplitMax - 1] = {};
   // this device's copy of `scratch` (bnn_forward_device_noalloc), null if
@@ -1386,7 +1398,6 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
   if (parts == 1) return part();
   if (!D->ev_conv[0]) {
     // all or nothing: a failure leaves no half-made set behind
-    hipStream_t side[kSplitMax - 1] = {};
     hipEvent_t conv[kSplitMax - 1] = {}, join[kSplitMax - 1] = {};
     // (the conv event orders two streams of this GPU only: the consumer
     // kernels see the conv's output through its own device-scope release,
@@ -1395,22 +1406,27 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
     // caller may read the side streams' logits from the host)
     bool ok = true;
     for (int k = 0; ok && k < kSplitMax - 1; ++k)
-      ok = hipStreamCreateWithFlags(&side[k], hipStreamNonBlocking) == hipSuccess &&
-           hipEventCreateWithFlags(&conv[k], hipEventDisableTiming | hipEventDisableSystemFence) == hipSuccess &&
+      ok = hipEventCreateWithFlags(&conv[k], hipEventDisableTiming | hipEventDisableSystemFence) == hipSuccess &&
            hipEventCreateWithFlags(&join[k], hipEventDisableTiming) == hipSuccess;
     if (!ok) {
       for (int k = 0; k < kSplitMax - 1; ++k) {
         if (conv[k]) (void)hipEventDestroy(conv[k]);
         if (join[k]) (void)hipEventDestroy(join[k]);
-        if (side[k]) (void)hipStreamDestroy(side[k]);
       }
-      return set_err(BNN_EHIP, "cannot create the streams of a split batch");
+      return set_err(BNN_EHIP, "cannot create the events of a split batch");
     }
     for (int k = 0; k < kSplitMax - 1; ++k) {
-      D->side[k] = side[k];
       D->ev_conv[k] = conv[k];
       D->ev_join[k] = join[k];
     }
+  }
+  hipStream_t side[kSplitMax - 1];
+  for (int k = 0; k + 1 < parts; ++k) {
+    side[k] = k == 0 && side_stream(D->stream, s) ? D->stream : D->side[k];
+    if (side[k]) continue;
+    if (hipStreamCreateWithFlags(&D->side[k], hipStreamNonBlocking) != hipSuccess)
+      return set_err(BNN_EHIP, "cannot create the streams of a split batch");
+    side[k] = D->side[k];
   }
   const int rows = N / unit;
   // Where two parts meet: at half the batch, or, when the certified first
@@ -1442,13 +1458,13 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
     stage = 1;
     if ((rc = part())) return rc;
     HIP_TRY(hipEventRecord(D->ev_conv[k], s));
-    HIP_TRY(hipStreamWaitEvent(D->side[k], D->ev_conv[k], 0));
-    st = D->side[k];
+    HIP_TRY(hipStreamWaitEvent(side[k], D->ev_conv[k], 0));
+    st = side[k];
     stage = 2;
     if ((rc = part())) return rc;
   }
   for (int k = 0; k + 1 < parts; ++k) {
-    HIP_TRY(hipEventRecord(D->ev_join[k], D->side[k]));
+    HIP_TRY(hipEventRecord(D->ev_join[k], side[k]));
     HIP_TRY(hipStreamWaitEvent(s, D->ev_join[k], 0));
   }
   return BNN_OK;
@@ -2253,10 +2269,6 @@ BnnConvLayer* bnn_layer_create(const uint64_t* packed_w, int Cin, int Cout, cons
   BnnDevice* D = &Lr->dev;
   auto fail = [&]() -> BnnConvLayer* { release(D); delete Lr; return nullptr; };
   if (hipGetDevice(&D->device) != hipSuccess) { set_err(BNN_EHIP, "no HIP device"); return fail(); }
-  if (hipStreamCreateWithFlags(&D->stream, hipStreamNonBlocking) != hipSuccess) {
-    set_err(BNN_EHIP, "hipStreamCreate failed");
-    return fail();
-  }
   Conv c{};
   c.tag = TAG_BIN; c.Cin = Cin; c.Cout = Cout; c.kh = c.kw = 3; c.pad = c.stride = 1;
   c.nwords = (Cin * 9 + 63) / 64;

@@ -698,28 +698,30 @@ int enqueue_forward(const ModelR* m, BnnReactDevice* D, RWorkspace& w, const flo
   const int unit = sc ? sc->pcols : 1;
   const bool split = !dump && !evs && N >= 256 && N / unit >= 2;
   if (!split) return part();
-  if (!D->side) {
+  if (!D->ev_fork) {
     // all or nothing: a failure leaves no half-made set behind
-    hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
-    if (hipStreamCreateWithFlags(&side, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&fork, hipEventDisableTiming) != hipSuccess ||
+    if (hipEventCreateWithFlags(&fork, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&join, hipEventDisableTiming) != hipSuccess) {
-      if (join) (void)hipEventDestroy(join);
       if (fork) (void)hipEventDestroy(fork);
-      if (side) (void)hipStreamDestroy(side);
-      return set_err(BNN_EHIP, "cannot create the stream of a split batch");
+      return set_err(BNN_EHIP, "cannot create the events of a split batch");
     }
-    D->side = side; D->ev_fork = fork; D->ev_join = join;
+    D->ev_fork = fork; D->ev_join = join;
+  }
+  hipStream_t side = side_stream(D->stream, s) ? D->stream : D->side;
+  if (!side) {
+    if (hipStreamCreateWithFlags(&D->side, hipStreamNonBlocking) != hipSuccess)
+      return set_err(BNN_EHIP, "cannot create the stream of a split batch");
+    side = D->side;
   }
   HIP_TRY(hipEventRecord(D->ev_fork, s));
-  HIP_TRY(hipStreamWaitEvent(D->side, D->ev_fork, 0));
+  HIP_TRY(hipStreamWaitEvent(side, D->ev_fork, 0));
   const int half = (N / unit) / 2 * unit;
   nb = 0; cnt = half; st = s;
   if ((rc = part())) return rc;
-  nb = half; cnt = N - half; st = D->side;
+  nb = half; cnt = N - half; st = side;
   if ((rc = part())) return rc;
-  HIP_TRY(hipEventRecord(D->ev_join, D->side));
+  HIP_TRY(hipEventRecord(D->ev_join, side));
   HIP_TRY(hipStreamWaitEvent(s, D->ev_join, 0));
   return BNN_OK;
 }
