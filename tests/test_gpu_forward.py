@@ -247,14 +247,16 @@ def test_cli_matches_reference_cli(tmp_path, golden):
     assert r.returncode == 1 and "cannot open" in r.stderr
 
 
+@pytest.mark.parametrize("base", [16, 24])
 @pytest.mark.parametrize("N", [256, 300, 513, 768, 769, 1031])
-def test_batch_size_independent(tmp_path, N):
+def test_batch_size_independent(tmp_path, N, base):
     """Any batch size, including ones that fill the last block partially,
-    gives the same bits for every patch as batches of 64: halves in row
-    parts (256, 300), one full round of the first conv and the rest in row
-    quarters or halves (513, 768), halves in whole rows (769, 1031)."""
+    gives the same bits for every patch as batches of 64.  Base 24 runs its
+    layers apart as two parts on two streams: halves in row parts (256, 300),
+    one full round of the first conv and the rest in row parts (513, 768),
+    halves in whole rows (769, 1031)."""
     import torch
-    b = synth.make_blob(seed=11)
+    b = synth.make_blob(seed=11, base=base)
     eng, _ = _engine(tmp_path, b)
     x = synth.make_input(12, N)
     small = np.concatenate([eng.forward_batch(x[i:i + 64]) for i in range(0, N, 64)])
@@ -314,12 +316,13 @@ def test_cfg4_full_batch(tmp_path, orc, monkeypatch):
     eng.close()
 
 
-def test_default_stream_is_ordered(tmp_path):
+@pytest.mark.parametrize("base", [16, 24])
+def test_default_stream_is_ordered(tmp_path, base):
     """stream = NULL is the HIP default stream: the host copy the caller
     enqueues there next (it waits for that stream only) sees the finished
-    logits of a split batch."""
+    logits, also of a split batch (base 24)."""
     import torch
-    eng, _ = _engine(tmp_path, synth.make_blob(seed=9))
+    eng, _ = _engine(tmp_path, synth.make_blob(seed=9, base=base))
     N = 512
     x = synth.make_input(10, N)
     want = eng.forward_batch(x)
@@ -332,14 +335,15 @@ def test_default_stream_is_ordered(tmp_path):
     eng.close()
 
 
-def test_split_forward_graph_capture(tmp_path):
-    """bnn_forward_device of a split batch (600 patches: a full round of the
-    certified conv, then 88 patches in row quarters, the first part's binary
-    layers on the model's side stream) captured in a HIP graph after one
+@pytest.mark.parametrize("base", [16, 24])
+def test_split_forward_graph_capture(tmp_path, base):
+    """bnn_forward_device of 600 patches captured in a HIP graph after one
     eager call, replayed on new inputs with eager work between the replays:
-    every replay bit-identical to the eager forward of the same input."""
+    every replay bit-identical to the eager forward of the same input.  Base
+    24 is a split batch (a full round of the certified conv, then 88 patches
+    in row parts, the first part's binary layers on a side stream)."""
     import torch
-    eng, _ = _engine(tmp_path, synth.make_blob(seed=12))
+    eng, _ = _engine(tmp_path, synth.make_blob(seed=12, base=base))
     N, H, W = 600, 32, 32
     gen = torch.Generator(device="cuda").manual_seed(13)
     x = torch.randn((N, 120, H, W), device="cuda", generator=gen)

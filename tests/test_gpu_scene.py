@@ -72,11 +72,13 @@ def test_scene_errors(tmp_path):
     eng.close()
 
 
-def test_scene_split_at_patch_rows(tmp_path, orc):
-    """a scene of 306 patches (18 patch rows, edge patches ragged) runs as two
-    parts of whole patch rows on two streams: the map equals the checker's"""
+@pytest.mark.parametrize("base", [16, 24])
+def test_scene_split_at_patch_rows(tmp_path, orc, base):
+    """a scene of 306 patches (18 patch rows, edge patches ragged), at base 24
+    as two parts of whole patch rows on two streams: the map equals the
+    checker's"""
     import torch
-    b = synth.make_blob(seed=5)
+    b = synth.make_blob(seed=5, base=base)
     eng = _engine(tmp_path, b)
     H, W, P = 549, 520, 32
     cube = _cube(6, H, W)
@@ -94,8 +96,7 @@ def test_scene_split_at_patch_rows(tmp_path, orc):
 def test_scene_cfg3_geometry(tmp_path, orc):
     """Benchmark config 3 at its exact geometry: a 956 x 684 x 120 cube
     (N(0,1) plus a per-band offset) cut into 30 x 22 = 660 patches of 32 x 32,
-    the last patch row and column zero past the scene, run as two parts of
-    whole patch rows.  Device and host-pointer maps against the checker's
+    the last patch row and column zero past the scene.  Device and host-pointer maps against the checker's
     per-patch forward, stitched."""
     import torch
     b = synth.make_blob(seed=0, base=16)
