@@ -1304,9 +1304,9 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
   static const char* enc_c2[4] = {"enc1.c2", "enc2.c2", "enc3.c2", "enc4.c2"};
   static const char* dec_c1[4] = {"dec4.c1", "dec3.c1", "dec2.c1", "dec1.c1"};
   static const char* dec_c2[4] = {"dec4.c2", "dec3.c2", "dec2.c2", "dec1.c2"};
-  // every binary layer of a 32x32 patch as one kernel; with per-kernel events
-  // (one kernel has no time per layer) or debug dumps the layers run apart
-  const bool use_tail = D->tail && H == 32 && W == 32 && !evs && !dump;
+  // every binary layer of a 32x32 patch as one kernel; with debug dumps the
+  // layers run apart
+  const bool use_tail = D->tail && H == 32 && W == 32 && !dump;
   auto tail = [&]() -> int {
     const int np = tail_np(cnt);
     TailArgs a = D->ta[np - 1];
@@ -1316,7 +1316,12 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
     a.logits = sc ? d_logits : d_logits + (size_t)nb * D->ncls * H * W;
     if (sc) { a.sH = sc->sH; a.sW = sc->sW; a.pcols = sc->pcols; a.prow0 = sc->prow0 + nb / sc->pcols; }
     HIP_TRY(launch_tail(a, np, st));
-    return BNN_OK;
+    double work = 0;
+    for (int i = 0; i < 4; ++i)
+      for (const DevBconv* L : {&D->e1[i], &D->e2[i], &D->d1[3 - i], &D->d2[3 - i]})
+        work += (double)N * L->cout * hs[i] * wsz[i] * L->cin * 9;  // (v1 has no e1[0]: 0)
+    for (const DevBconv* L : {&D->b1, &D->b2}) work += (double)N * L->cout * hs[4] * wsz[4] * L->cin * 9;
+    return mark(D->stem ? "enc1.c1-dec1" : "enc1.c2-dec1", "bconv_tail", work, 1.0);
   };
   int stage = 3;  // what part() enqueues: 1 the first conv, 2 the binary layers
   auto part = [&]() -> int {

@@ -47,15 +47,29 @@ def _build(tmp_path, source):
     return str(exe)
 
 
-@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc (for the HIP headers) not found")
-def test_layers_take_their_faster_kernel(tmp_path):
-    text = "".join("%s %d %d %d %d %d %d\n" % layer[:7] for layer in LAYERS)
+def _choice(tmp_path, layers):
+    """[(taken by default, fits)] of (epilogue, cin, cout, skip, N, H, W)."""
+    text = "".join("%s %d %d %d %d %d %d\n" % layer for layer in layers)
     r = subprocess.run([_build(tmp_path, "bconv_choice_check.cpp")], input=text, capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr
-    took = [int(v) for v in r.stdout.split()]
-    want = [int(layer[8] < layer[7]) for layer in LAYERS]
-    wrong = [layer for layer, t, w in zip(LAYERS, took, want) if t != w]
-    assert len(took) == len(LAYERS) and not wrong, wrong
+    out = [tuple(map(int, line.split())) for line in r.stdout.splitlines()]
+    assert len(out) == len(layers)
+    return out
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc (for the HIP headers) not found")
+def test_layers_take_their_faster_kernel(tmp_path):
+    took = _choice(tmp_path, [layer[:7] for layer in LAYERS])
+    wrong = [layer for layer, t in zip(LAYERS, took) if t[0] != int(layer[8] < layer[7])]
+    assert not wrong, wrong
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc (for the HIP headers) not found")
+def test_gpu_shapes_fit(tmp_path):
+    """The layers that the GPU tests force onto the matrix cores run there."""
+    from test_gpu_mfma import SHAPES
+    layers = [(epi, cin, cout, 0, N, H, W) for N, H, W, cin, cout in SHAPES for epi in ("P", "pool")]
+    assert all(fits for _, fits in _choice(tmp_path, layers))
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc (for the HIP headers) not found")

@@ -413,10 +413,11 @@ def test_fused_middle_rule_and_logits(tmp_path, monkeypatch, base, H, W, N, mode
     """enc3.c1 .. dec3.c2 run as one kernel when level 2 is 8 x 8 and the
     widths fit (base <= 16); with enc2.c1, enc2.c2, dec2.c1 and dec2.c2
     around them when level 1 is 16 x 16 and a part of the batch has at
-    least 256 patches.  BNN_MIDX=0 keeps the level-1 layers as per-layer
+    least 256 patches; 32x32 patches so with BNN_TAIL=0 only.  BNN_MIDX=0 keeps the level-1 layers as per-layer
     kernels and BNN_MID=0 every layer, with the same logits bit for bit."""
     b = synth.make_blob(seed=40 + base, base=base)
     x = synth.make_input(41, N, 120, H, W)
+    monkeypatch.setenv("BNN_TAIL", "0")
     monkeypatch.delenv("BNN_MID", raising=False)
     monkeypatch.delenv("BNN_MIDX", raising=False)
     eng, _ = _engine(tmp_path, b)

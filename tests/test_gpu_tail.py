@@ -24,6 +24,23 @@ def _pair(tmp_path, monkeypatch, b):
     return one, apart
 
 
+def _ops(eng, x):
+    """label -> profiler op name of one forward."""
+    E.prof_reset()
+    E.prof_enable(True)
+    try:
+        eng.forward_batch(x)
+    finally:
+        E.prof_enable(False)
+    return {lab: op for lab, op, _ms, _w in E.prof_records()}
+
+
+def _takes(one, apart, x):
+    """The first model runs its layers as one kernel, the second apart."""
+    assert "bconv_tail" in _ops(one, x).values()
+    assert "enc1.c2" in _ops(apart, x)
+
+
 def _bits(a):
     return np.ascontiguousarray(a).view(np.uint32)
 
@@ -35,6 +52,7 @@ def test_tail_equals_layers(tmp_path, monkeypatch, orc, base, N, cov):
     b = synth.make_blob(seed=90 + base + N, base=base, coverage=cov)
     one, apart = _pair(tmp_path, monkeypatch, b)
     x = synth.make_input(91 + N, N, 120, 32, 32)
+    _takes(one, apart, x)
     got = one.forward_batch(x)
     assert np.array_equal(_bits(got), _bits(apart.forward_batch(x)))
     model = orc.parse(B.to_bytes(b))
@@ -49,6 +67,7 @@ def test_tail_stem(tmp_path, monkeypatch, base, stem, N):
     b = synth.make_blob_v2(seed=92 + N, base=base, stem=stem, coverage=True)
     one, apart = _pair(tmp_path, monkeypatch, b)
     x = synth.make_input(93 + N, N, 120, 32, 32)
+    _takes(one, apart, x)
     assert np.array_equal(_bits(one.forward_batch(x)), _bits(apart.forward_batch(x)))
     one.close()
     apart.close()
@@ -59,7 +78,18 @@ def test_tail_scene(tmp_path, monkeypatch, H, W, classes):
     """Edge patches past the scene, other class counts."""
     b = synth.make_blob(seed=94, base=16, n_classes=classes, coverage=True)
     one, apart = _pair(tmp_path, monkeypatch, b)
+    _takes(one, apart, synth.make_input(98, 2, 120, 32, 32))
     cube = np.random.default_rng(95).standard_normal((120, H, W), dtype=np.float32)
     assert np.array_equal(_bits(one.forward_patched(cube, 32)), _bits(apart.forward_patched(cube, 32)))
+    one.close()
+    apart.close()
+
+
+@pytest.mark.parametrize("base,H,W", [(20, 32, 32), (16, 33, 32), (16, 32, 31), (16, 64, 64)])
+def test_tail_not_taken(tmp_path, monkeypatch, base, H, W):
+    """A model just too wide, and patches of other sizes, run their layers apart."""
+    one, apart = _pair(tmp_path, monkeypatch, synth.make_blob(seed=96, base=base))
+    x = synth.make_input(97, 2, 120, H, W)
+    assert "enc1.c2" in _ops(one, x)
     one.close()
     apart.close()
