@@ -38,11 +38,17 @@ before each other configuration.  Prints ONE JSON line on stdout:
                 peak
   first_conv_exact  the order-exact first conv (a model loaded with
                 BNN_CERT=0): its time and FP32 rate against the matrix peak
-  bconv         the 17 binary convs: binary-op/s (2 per bit-MAC, border taps
-                counted) against the VALU-popcount roofline
+  bconv         the 17 binary convs of the timed forward, one kernel with the
+                head (FP4 matrix cores): binary-op/s (2 per bit-MAC, border
+                taps counted) against the FP4 roofline (and, for comparison,
+                the VALU-popcount one); popcount: the same layers on the
+                XNOR-popcount kernels (a model loaded with BNN_BCONV_MFMA=0)
+                against the VALU-popcount roofline
   cfg1          benchmark config 1: the isolated binary conv 64->64 at
-                64x64, batch 256, int32 P out: binary-op/s against the
-                VALU-popcount roofline and the HBM rate of its bytes
+                64x64, batch 256, int32 P out: the HBM rate of its bytes,
+                which bind, and binary-op/s against the FP4 roofline; the
+                popcount kernel (BNN_BCONV_MFMA=0) against the VALU-popcount
+                roofline
   fused_pool    the isolated fused bconv+fold+maxpool kernel at 128->128,
                 32x32, batch 1024 (the benchmark's fused-kernel config):
                 the kernel the default rule takes (the matrix cores, FP4)
@@ -380,6 +386,33 @@ def cert_adversarial(torch, np, engine, blob, synth, td, sp, N, H, W):
     return res
 
 
+def bconv_row(lab, op, ms, work):
+    """A profiled kernel of binary layers against the peak of the unit it runs on."""
+    fp4 = op.endswith("_mfma") or op == "bconv_tail"
+    rate = 2 * work / (ms / 1e3)
+    return {"label": lab, "op": op, "ms": round(ms, 5), "tbinops": round(rate / 1e12, 2),
+            "frac": round(rate / (2 * PEAK_FP4_MACS if fp4 else valu_binop_peak()), 4),
+            "frac_of": "FP4 matrix peak" if fp4 else "VALU popcount peak"}
+
+
+def with_env(name, value, make):
+    """make() with an environment variable that a model or layer reads when it is made."""
+    old = os.environ.get(name)
+    os.environ[name] = value
+    try:
+        return make()
+    finally:
+        if old is None:
+            os.environ.pop(name, None)
+        else:
+            os.environ[name] = old
+
+
+def popcount_layer(engine, *args):
+    """A conv layer on the bit-packed popcount kernel."""
+    return with_env("BNN_BCONV_MFMA", "0", lambda: engine.ConvLayer(*args))
+
+
 def bench_cfg4(sp, stream, td, reps4=5):
     """Benchmark config 4: large tiles, 256 x 256 x 120, batch 64, base 32
     (wide layers, 512 channels at the bottleneck): the forward's time per
@@ -518,9 +551,31 @@ def main() -> int:
         c1_bitmacs = N1 * C1 * S1 * S1 * C1 * 9
         c1_rate = 2 * c1_bitmacs / (c1_ms / 1e3)
         c1_bytes = N1 * S1 * S1 * (C1 // 8) + P1.numel() * 4  # packed bits in, int32 P out
-        log(f"cfg1 bconv 64->64 64x64 b{N1}, int32 P out: {c1_ms * 1e3:.1f} us, frac {c1_rate / valu_binop_peak():.3f} "
-            f"of VALU popcount peak, {c1_bytes / (c1_ms / 1e3) / 1e9:.0f} GB/s of algorithmic HBM bytes")
+        # (this shape runs on the matrix cores unless BNN_BCONV_MFMA=0)
+        c1_mfma = os.environ.get("BNN_BCONV_MFMA") != "0"
+        c1_peak = 2 * PEAK_FP4_MACS if c1_mfma else valu_binop_peak()
+        log(f"cfg1 bconv 64->64 64x64 b{N1}, int32 P out: {c1_ms * 1e3:.1f} us, "
+            f"{c1_bytes / (c1_ms / 1e3) / 1e9:.0f} GB/s of algorithmic HBM bytes, frac {c1_rate / c1_peak:.3f} of the "
+            f"{'FP4 matrix' if c1_mfma else 'VALU popcount'} peak")
         L1.close()
+        c1_pc = None
+        if c1_mfma:
+            L1 = popcount_layer(engine, blob.pack_kidx(synth.make_signs(21, C1, C1)), C1, C1)
+            settle(lambda: L1.P_device(act1.data_ptr(), N1, S1, S1, P1.data_ptr(), sp), torch)
+            torch.cuda.synchronize()
+            e0.record(stream)
+            for _ in range(20):
+                L1.P_device(act1.data_ptr(), N1, S1, S1, P1.data_ptr(), sp)
+            e1.record(stream)
+            torch.cuda.synchronize()
+            pc_ms = e0.elapsed_time(e1) / 20
+            pc_rate = 2 * c1_bitmacs / (pc_ms / 1e3)
+            c1_pc = {"kernel": "k_bconv (VALU popcount, BNN_BCONV_MFMA=0)", "us": round(pc_ms * 1e3, 2),
+                     "binary_op_s": round(pc_rate, 1), "frac": round(pc_rate / valu_binop_peak(), 4),
+                     "frac_of": "VALU popcount peak"}
+            log(f"  the same on the popcount kernel: {pc_ms * 1e3:.1f} us, frac {pc_rate / valu_binop_peak():.3f} "
+                f"of the VALU popcount peak")
+            L1.close()
         del act1, P1
 
         # fused bconv + fold + 2x2 max-pool, 128->128 at 32x32, batch 1024
@@ -558,18 +613,10 @@ def main() -> int:
         L.close()
         pool_pc = None
         if pool_mfma:
-            # the same layer on the bit-packed popcount kernel (the mode is
-            # read when a layer is made), against the VALU-popcount peak
-            old = os.environ.get("BNN_BCONV_MFMA")
-            os.environ["BNN_BCONV_MFMA"] = "0"
-            try:
-                Lp = engine.ConvLayer(blob.pack_kidx(w), C, C, synth.make_thresholds(32, C, 288),
-                                      synth.make_thresholds(33, C, 288))
-            finally:
-                if old is None:
-                    os.environ.pop("BNN_BCONV_MFMA", None)
-                else:
-                    os.environ["BNN_BCONV_MFMA"] = old
+            # the same layer on the bit-packed popcount kernel, against the
+            # VALU-popcount peak
+            Lp = popcount_layer(engine, blob.pack_kidx(w), C, C, synth.make_thresholds(32, C, 288),
+                                synth.make_thresholds(33, C, 288))
             settle(lambda: Lp.fold_pool_device(act.data_ptr(), N, H, W, skip.data_ptr(), down.data_ptr(), sp), torch)
             torch.cuda.synchronize()
             e0.record(stream)
@@ -781,8 +828,8 @@ def main() -> int:
         a = agg.setdefault(lab, [op, [], 0, work])
         a[1].append(ms)
         a[2] += 1
-    # which first-conv kernel ran: the certified one unless BNN_CERT=0 (its
-    # shape condition, 4 <= cin <= 128 and W in multiples of 4, holds here)
+    # which first-conv kernel ran: the certified one, the faster at this
+    # shape, unless BNN_CERT=0
     cert = os.environ.get("BNN_CERT") != "0"
     real_bytes = N * 120 * H * W * 4 + N * H * W * 4  # input floats once, output words once
     kernels = []
@@ -800,9 +847,7 @@ def main() -> int:
                 kernels.append({"label": lab, "op": op, "ms": round(mean, 5), "bound": "mfma",
                                 "tflops": round(rate / 1e12, 3), "frac": round(rate / PEAK_FP32_FLOPS, 4)})
         else:
-            rate = 2 * work / (mean / 1e3)
-            kernels.append({"label": lab, "op": op, "ms": round(mean, 5), "tbinops": round(rate / 1e12, 2),
-                            "frac": round(rate / valu_binop_peak(), 4)})
+            kernels.append(bconv_row(lab, op, mean, work))
     for k in kernels:
         log(f"  {k['label']:10s} {k['op']:10s} {k['ms']*1e3:9.1f} us  frac {k['frac']:.3f}")
     real = next(k for k in kernels if k["op"] == "conv_real")
@@ -842,11 +887,7 @@ def main() -> int:
     if cert and not args.headline_only:
         # the order-exact first conv on the same batch, from a model loaded
         # with BNN_CERT=0 (the variable is read when a model is loaded)
-        os.environ["BNN_CERT"] = "0"
-        try:
-            xeng = engine.Engine(blob_path)
-        finally:
-            os.environ.pop("BNN_CERT", None)
+        xeng = with_env("BNN_CERT", "0", lambda: engine.Engine(blob_path))
         settle(lambda: xeng.forward_device(x.data_ptr(), N, H, W, y.data_ptr(), sp), torch)
         engine.prof_reset()
         engine.prof_enable(True)
@@ -865,6 +906,34 @@ def main() -> int:
     bin_ms = sum(k["ms"] for k in kernels if k["op"] != "conv_real")
     bin_work = sum(agg[k["label"]][3] for k in kernels if k["op"] != "conv_real")
     bin_rate = 2 * bin_work / (bin_ms / 1e3)
+    bin_fp4 = all(k["frac_of"] == "FP4 matrix peak" for k in kernels if k["op"] != "conv_real")
+    bin_peak = 2 * PEAK_FP4_MACS if bin_fp4 else valu_binop_peak()
+
+    popc = None
+    if not args.headline_only and any(k["op"] == "bconv_tail" for k in kernels):
+        # the same layers on the popcount kernels, from a model loaded with
+        # BNN_BCONV_MFMA=0
+        aeng = with_env("BNN_BCONV_MFMA", "0", lambda: engine.Engine(blob_path))
+        settle(lambda: aeng.forward_device(x.data_ptr(), N, H, W, y.data_ptr(), sp), torch)
+        engine.prof_reset()
+        engine.prof_enable(True)
+        for _ in range(10):
+            aeng.forward_device(x.data_ptr(), N, H, W, y.data_ptr(), sp)
+        torch.cuda.synchronize()
+        engine.prof_enable(False)
+        aagg = {}
+        for lab, op, ms, work in engine.prof_records():
+            if op != "conv_real":
+                aagg.setdefault(lab, [op, [], work])[1].append(ms)
+        aeng.close()
+        rows = [bconv_row(lab, op, float(np.median(v)), work) for lab, (op, v, work) in aagg.items()]
+        a_ms = sum(k["ms"] for k in rows)
+        a_rate = 2 * sum(v[2] for v in aagg.values()) / (a_ms / 1e3)
+        popc = {"config": "the same layers on the popcount kernels (BNN_BCONV_MFMA=0, one stream, timed by events)",
+                 "ms": round(a_ms, 5), "binary_op_s": round(a_rate, 1), "peak": valu_binop_peak(),
+                 "frac": round(a_rate / valu_binop_peak(), 4), "frac_of": "VALU popcount peak", "kernels": rows}
+        for k in rows:
+            log(f"  popcount {k['label']:10s} {k['op']:10s} {k['ms']*1e3:9.1f} us  frac {k['frac']:.3f} of {k['frac_of']}")
 
     if not args.headline_only:
         # the same batch from and to host memory (pinned buffers): the copies in
@@ -939,9 +1008,12 @@ def main() -> int:
                    "batch": N, "H": H, "W": W, "n_bands": 120, "n_classes": 3, "base_channels": 16},
         "roofline": roofline,
         "bconv": {"layers": 17, "kernels": sum(1 for k in kernels if k["op"] != "conv_real"),
-                  "binary_op_s": round(bin_rate, 1), "peak": valu_binop_peak(),
-                  "frac": round(bin_rate / valu_binop_peak(), 4), "ms": round(bin_ms, 5),
-                  "unit": "binary-op/s (2 per bit-MAC, border taps counted)"},
+                  "binary_op_s": round(bin_rate, 1), "peak": bin_peak,
+                  "frac": round(bin_rate / bin_peak, 4),
+                  "frac_of": "FP4 matrix peak" if bin_fp4 else "VALU popcount peak", "ms": round(bin_ms, 5),
+                  "unit": "binary-op/s (2 per bit-MAC, border taps counted)",
+                  "of_valu_popcount_peak": round(bin_rate / valu_binop_peak(), 4),
+                  **({"popcount": popc} if popc else {})},
         "kernels": kernels,
         "cpu_baseline": cpu,
     }
@@ -954,9 +1026,12 @@ def main() -> int:
             "first_conv_exact": exact,
             "cfg1": {"config": "isolated bconv 64->64, 64x64, batch 256, int32 P out (benchmark config 1)",
                      "us": round(c1_ms * 1e3, 2), "binary_op_s": round(c1_rate, 1),
-                     "frac": round(c1_rate / valu_binop_peak(), 4),
+                     "kernel": "k_bconv_mfma (FP4 matrix cores)" if c1_mfma else "k_bconv (VALU popcount)",
+                     "frac": round(c1_rate / c1_peak, 4),
+                     "frac_of": "FP4 matrix peak" if c1_mfma else "VALU popcount peak",
                      "hbm_GB_s": round(c1_bytes / (c1_ms / 1e3) / 1e9, 1),
-                     "hbm_frac": round(c1_bytes / (c1_ms / 1e3) / PEAK_HBM, 4)},
+                     "hbm_frac": round(c1_bytes / (c1_ms / 1e3) / PEAK_HBM, 4),
+                     **({"popcount": c1_pc} if c1_pc else {})},
             "fused_pool": {"config": "bconv 128->128 + fold + 2x2 maxpool + fold, 32x32, batch 1024",
                            "us": round(pool_ms * 1e3, 2), "binary_op_s": round(pool_rate, 1),
                            "kernel": "k_bconv_mfma (FP4 matrix cores)" if pool_mfma else "k_bconv (VALU popcount)",
