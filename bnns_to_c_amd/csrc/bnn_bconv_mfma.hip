@@ -761,7 +761,8 @@ static MfmaPlan mfma_plan(const MfmaConv& mc, int cw, int N, int H, int W, int e
 // the better of the two 20.5, the popcount kernel alone 27.5, this one 22.7.
 //  * popcount: a wave counts its words (9 a tap word, 5 a pair) over cog
 //    channels x 1 or 4 pixels, the waves over the 1,024 SIMDs; from 60 words
-//    on, and with the weights' bytes, its weight loads show;
+//    on, and with the weights' bytes, its weight loads show (half as much
+//    where fewer than half the CUs have a wave);
 //  * here: K steps and rounds of tiles, by the blocks that share a CU: staging
 //    by pixels and planes, sums by operands, the epilogue by outputs.
 // Pairs (us, popcount : here): folds 64 -> 64, one 128x128 image, 5.0 : 7.1,
@@ -779,7 +780,8 @@ static MfmaPlan mfma_plan(const MfmaConv& mc, int cw, int N, int H, int W, int e
 //    even the last one out (152 -> 40, 3.4e5 pixels, 62 : 43; 152 -> 64, 1.2e5
 //    pixels, 28 : 36), from 224 channels at 1.5e9 bit-MACs (232 -> 24 at 1.6e9
 //    15.4 : 10.2; 456 -> 168 at 1.2e9 10.3 : 16.3).
-bool mfma_conv_pays(const MfmaConv& mc, int cin, int cout, int cw, bool pair, int epi, int N, int H, int W) {
+bool mfma_conv_pays(const MfmaConv& mc, int cin, int cout, int cw0, int cw1, bool pair, int epi, int N, int H, int W, int cus) {
+  const int cw = cw0 + cw1;
   const double px = (double)N * H * W, macs = 9.0 * px * cin * cout;
   if (epi == EPI_HEAD || epi == EPI_P) {
     const bool pays = epi == EPI_HEAD ? macs >= 4e9 && cin >= 32
@@ -790,7 +792,10 @@ bool mfma_conv_pays(const MfmaConv& mc, int cin, int cout, int cw, bool pair, in
     return pays && mfma_conv_fits(mc, cw, N, H, W, epi);
   }
   const bool pool = epi == EPI_POOL;
-  const int cus = device_cus();
+  // (deep folds on few pixels, where a popcount wave walks all words of a
+  // pixel and its time outgrows the estimate: 256 -> 512, 155 patches 1x5,
+  // 17.0 : 11.2, 384 -> 384, 48 of 2x3, 14.0 : 11.5)
+  if (!pool && cw1 == 0 && ((cin >= 256 && macs >= 2.5e8) || cin >= 512)) return mfma_conv_fits(mc, cw, N, H, W, epi);
   int mt, cog;
   bconv_shape(epi, N, H, W, cout, &mt, &cog);
   const long waves = ((long)N * ((H + mt - 1) / mt) * ((W + mt - 1) / mt) + 63) / 64 * ((cout + cog - 1) / cog);
@@ -798,16 +803,20 @@ bool mfma_conv_pays(const MfmaConv& mc, int cin, int cout, int cw, bool pair, in
   const double turns = ws < 2 ? std::ceil(ws) : ws, out = turns * cog * mt * mt;
   const double deep = turns * std::max(0.0, words - 60), kw = words * cout / 1024;
   const double pop = pool ? 4.91 + out * (0.0035 * words + 0.0188) + 0.27 * kw + 0.048 * deep
-                          : 4.33 + out * (0.0036 * words + 0.0085) + 0.088 * kw + 0.021 * deep;
+                          : 4.33 + out * (0.0036 * words + 0.0085) +
+                                (0.088 * kw + 0.021 * deep) * (2 * waves < cus ? 0.5 : 1.0);
+  const double planes = (cw + 3) / 4, loads = cw < 4 ? cw : 0;
   const double start = pool ? 5.87 + 0.093 * mc.steps : 5.19 + 0.071 * mc.steps;
-  if (pop <= start || !mfma_conv_fits(mc, cw, N, H, W, epi)) return false;
+  const double operand = pool ? 0.0077 * mc.steps + 0.0348 : 0.0100 * mc.steps + 0.0286, round = (pool ? 0.33 : 0.28) * planes;
+  // (the tile is worked out only where one round of one block a CU might do:
+  // 0.2 us of the host)
+  if (start + round + operand * mc.mt * 2 + 0.4 >= pop || !mfma_conv_fits(mc, cw, N, H, W, epi)) return false;
   const MfmaPlan p = mfma_plan(mc, cw, N, H, W, epi, cus);
-  const double blocks = 8.0 * p.T.ncg * p.nts, planes = (cw + 3) / 4, loads = cw < 4 ? cw : 0;
+  const double blocks = 8.0 * p.T.ncg * p.nts;
   const double share = blocks <= (double)p.per_cu * cus ? std::min((double)p.per_cu, std::ceil(blocks / cus)) : blocks / cus;
-  const double stage = p.rounds * share * p.T.ns / 256, sums = p.rounds * share * p.T.sub * mc.mt * p.G;
-  const double here = pool ? start + stage * (0.287 * planes + 0.0218 * loads) + sums * (0.0077 * mc.steps + 0.0348) + 0.33 * p.rounds * planes
-                           : start + stage * 0.378 * planes + sums * (0.0100 * mc.steps + 0.0286) + 0.28 * p.rounds * planes;
-  return here < pop;
+  const double stage = share * p.T.ns / 256 * (pool ? 0.287 * planes + 0.0218 * loads : 0.378 * planes);
+  const double here = start + p.rounds * (round + stage + operand * share * p.T.sub * mc.mt * p.G);
+  return here + 0.4 < pop;  // (near ties on the popcount kernel)
 }
 
 namespace {

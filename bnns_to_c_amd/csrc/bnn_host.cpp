@@ -395,6 +395,7 @@ struct DevBconv {
   FoldDev f1{}, f2{};
   MfmaConv mc{};  // matrix-core tables (mc.w null: the popcount kernel only)
   int mfma = 0;   // mfma_conv_mode() at creation
+  int cus = 0;    // compute units of its device
   int pair = 0;   // cin <= 16, no concat: wt holds tap pairs, 5 words per channel
   uint32_t* mw = nullptr;  // the fused middle's table [words][channel group][9][64] (mid layers only)
 };
@@ -441,9 +442,8 @@ int cert_mode() {
 
 bool use_mfma(const DevBconv& L, int epi, int N, int H, int W) {
   if (!L.mc.w) return false;
-  const int cw = L.cw0 + L.cw1;
-  return L.mfma == 2 ? mfma_conv_fits(L.mc, cw, N, H, W, epi)
-                     : mfma_conv_pays(L.mc, L.cin, L.cout, cw, L.pair, epi, N, H, W);
+  return L.mfma == 2 ? mfma_conv_fits(L.mc, L.cw0 + L.cw1, N, H, W, epi)
+                     : mfma_conv_pays(L.mc, L.cin, L.cout, L.cw0, L.cw1, L.pair, epi, N, H, W, L.cus);
 }
 
 struct Workspace {
@@ -620,6 +620,7 @@ int upload_bconv(BnnDevice* D, DevBconv* L, const Conv& c, int cs, const Act* a1
   std::vector<uint32_t> wt = repack_bin(c.packed, c.Cin, c.Cout, 9, cs);
   L->pair = (cs ? cs : c.Cin) <= 16;
   L->mfma = mfma_conv_mode();
+  L->cus = device_cus();
   int rc;
   if (L->mfma && (rc = upload_mfma(D, L, c, cs, a1, a2, wt))) return rc;
   L->words = wt;

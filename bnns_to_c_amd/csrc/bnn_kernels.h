@@ -552,10 +552,11 @@ int device_cus();
 // shape whose tile, operand and tables fit a CU's LDS; the head in one wave's
 // channels; the rules the epilogue needs).
 bool mfma_conv_fits(const MfmaConv& mc, int cw, int N, int H, int W, int epi);
-// Whether the layer fits and this is its faster kernel (the kernel's file says
-// by which times).  N is the whole batch's, also for a part of it: the parts
-// run side by side.
-bool mfma_conv_pays(const MfmaConv& mc, int cin, int cout, int cw, bool pair, int epi, int N, int H, int W);
+// Whether the layer fits and this is its faster kernel on a device of cus
+// compute units (the kernel's file says by which times).  N is the whole
+// batch's, also for a part of it: the parts run side by side.
+bool mfma_conv_pays(const MfmaConv& mc, int cin, int cout, int cw0, int cw1, bool pair, int epi, int N, int H, int W,
+                    int cus);
 hipError_t launch_bconv_mfma(const BconvArgs& a, const MfmaConv& m, int epi, hipStream_t s);
 hipError_t launch_real(const RealArgs& a, hipStream_t s);
 

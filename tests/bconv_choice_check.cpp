@@ -1,7 +1,7 @@
 // Prints, for each line "epi cin cout skip N H W" on stdin (epi: fold, pool,
 // head or P; skip: the channels of a concat's first segment, 0 without), 1 if
 // the binary conv would run on the matrix cores by default, 0 if on the
-// popcount kernel (mfma_conv_pays; 256 compute units where there is no GPU),
+// popcount kernel (mfma_conv_pays, 256 compute units),
 // and 1 if the matrix-core kernel takes the layer at all (mfma_conv_fits).
 #include <cstdio>
 #include <cstring>
@@ -26,7 +26,7 @@ int main() {
     mc.mt = mfma_mt(cout);
     mc.slots = mfma_nslots(cw0, cw1, pair);
     mc.steps = (mc.slots + 3) / 4;
-    printf("%d %d\n", mfma_conv_pays(mc, cin, cout, cw0 + cw1, pair, epi, N, H, W) ? 1 : 0,
+    printf("%d %d\n", mfma_conv_pays(mc, cin, cout, cw0, cw1, pair, epi, N, H, W, 256) ? 1 : 0,
            mfma_conv_fits(mc, cw0 + cw1, N, H, W, epi) ? 1 : 0);
   }
   return 0;

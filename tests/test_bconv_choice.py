@@ -29,6 +29,9 @@ LAYERS = [
     ("fold", 64, 64, 0, 1, 145, 32, 5.2, 7.0),
     ("fold", 512, 512, 0, 1, 32, 32, 33.8, 12.4),
     ("fold", 256, 256, 0, 148, 4, 4, 16.4, 10.5),
+    ("fold", 384, 384, 0, 48, 2, 3, 14.0, 11.5),
+    ("fold", 256, 512, 0, 155, 1, 5, 17.0, 11.2),
+    ("fold", 768, 256, 256, 13, 2, 3, 14.6, 16.6),
     ("fold", 1152, 384, 384, 1, 13, 20, 38.6, 21.4),
     ("fold", 768, 256, 256, 1, 17, 36, 26.4, 16.4),
     ("head", 32, 32, 0, 64, 256, 256, 97.6, 69.1),
