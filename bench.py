@@ -8,8 +8,9 @@ base 16, x ~ N(0,1)) with the input already resident in HBM; K steps are
 timed back to back between device synchronisations and one pair of
 timing-only HIP events (no cache fence of their own); a second pass with an
 event between consecutive steps gives the spread of single steps.  The
-GPU's clocks ramp under sustained load over about 25 ms (per-step time
-falls from ~0.58 to ~0.50 ms over the first ~40 forwards, then holds), so
+GPU's clocks ramp under sustained load over about 25 ms (measured on the
+order-exact forward: ~0.58 to ~0.50 ms a step over the first ~40, then it
+holds), so
 every measurement first runs its workload untimed, back to back
 with its warmup and timed runs: --settle forwards (default 120, reported as
 settle_steps) before the headline's W warmup and K timed steps, about 40 ms
@@ -771,9 +772,8 @@ def main() -> int:
         eng.forward_device(x.data_ptr(), N, H, W, y.data_ptr(), sp)
 
     # Settle: the GPU's clocks ramp under sustained load (measured on the
-    # box: per-step time falls from ~0.58 to ~0.50 ms over the first ~40
-    # forwards, about 25 ms, then holds; after half a second idle it ramps
-    # again).  args.settle untimed forwards go first, queued back to back
+    # order-exact forward: a step falls from ~0.58 to ~0.50 ms over the first
+    # ~40, about 25 ms, then holds; after half a second idle it ramps again).  args.settle untimed forwards go first, queued back to back
     # with the W warmup steps and the timed ones, so the timed steps run at
     # the steady clock; the count is reported as "settle_steps".
     for _ in range(args.settle):

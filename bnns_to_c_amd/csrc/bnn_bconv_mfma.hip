@@ -28,7 +28,8 @@ namespace {
 // -S - c (S: the weight sum over the taps inside the image, one of 16 border
 // classes, c: the centre of the channel's rule) and ends at P - c, since
 // P = 2*sum(w*alpha) - S.  Every term and sum is an integer or a half below
-// 2^24, so the FP32 sums are exact in any order.
+// 2^24, so the FP32 sums are exact in any order (a layer whose tile and slot
+// table fit a CU's LDS has fewer than 70,000 input channels, 18 to a sum).
 //
 // Work split.  A wave makes MT*16 channels x G*16 pixels, a block of four
 // waves the same channels of 64*G pixels: a tile of TR rows x TW columns of a

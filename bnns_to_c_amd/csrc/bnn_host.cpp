@@ -1439,9 +1439,9 @@ int enqueue_forward(const Model* m, BnnDevice* D, Workspace& w, const float* d_i
   // conv runs and the batch is at most one and a half of its rounds (the
   // patches whose blocks it holds at once), after one whole round, so that
   // the second part's conv, at most half a round, splits its patches' rows
-  // over two or four blocks and takes a fraction of a round's time
-  // (launch_real_cert; config 3's 660 patches as 506 + 154 instead of two
-  // half-full rounds of 330)
+  // over as many blocks as fill the device and takes a fraction of a round's
+  // time (launch_real_cert; 660 patches of 32x32, 30 rows of 22, as 506 + 154
+  // instead of two half-full rounds of 330)
   long cut = rows / 2;
   RealArgs whole{};
   whole.x = d_in;

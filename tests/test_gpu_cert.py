@@ -156,7 +156,7 @@ def test_cert_dense_infinities(tmp_path, orc, base, H, W):
                                          (40, 32, 64, 32), (3, 17, 36, 32)])
 def test_cert_row_parts(tmp_path, orc, N, H, W, base):
     """A launch of fewer patches than a round of the GPU holds splits each
-    patch's rows over two or four blocks, each starting one input row above
+    patch's rows over several blocks, each starting one input row above
     its first output row: 100 patches of 33 rows in parts of 9, 9, 9 and 6;
     200 of 32 in halves; 250 of 20 in halves; tiled rows of 44 and 64 (both
     16-channel groups in one block at base 32), 17 rows in parts of 9 and 8.
