@@ -143,8 +143,9 @@ int bnn_forward_debug(const Model *m, const float *input, int N, int H, int W,
  * the previous call (or the load): the outputs it decided from its bounded
  * approximation plus the ones it recomputed in the reference's order
  * (*outputs), and the recomputed ones (*undecided).  Waits for all work on
- * the model's GPU, then resets both counts.  Both are 0 for a model whose
- * first conv runs in the reference's order (BNN_CERT=0, general signs). */
+ * the model's GPU, then resets both counts.  Both are 0 where the
+ * first conv ran in the reference's order (BNN_CERT=0, general signs, or a
+ * launch whose size and bands make that the faster kernel). */
 int bnn_cert_stats(const Model *m, unsigned long long *undecided, unsigned long long *outputs);
 
 /* Per-op GPU timing of the device forward (hipEvents around every kernel). */
